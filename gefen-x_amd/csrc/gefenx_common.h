@@ -38,48 +38,70 @@ static_assert(sizeof(QTable) % 16 == 0, "QTable must stay 16-byte aligned in siz
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 // Factored stats tiling: a workgroup covers kFactTileCols columns (64 lanes x
-// two 8-column chunks) of `tile_rows` consecutive rows.  Tiles hold about
-// N/32 elements, between 64K (16K-element tiles spend a third of the pass on
-// per-workgroup set-up and flushes) and 1M.  The multi-tensor launch puts
-// every parameter's tiles in one grid, largest tiles first, so fewer, larger
-// tiles cost no occupancy until the last round of workgroups, one of the
-// smallest tiles, runs part-empty.  Measured (stats kernel on the Llama-3-8B
-// set, tiles ordered by size): caps of 256K / 512K / 768K / 1M / 1.5M / 2M
-// 4.29-4.31 / 4.08 / 4.01-4.04 / 3.96-3.99 / 4.05-4.07 / 3.95-3.96 ms (1.5M
-// and 2M leave 4096-row tensors a short last row tile; 1M splits the common
-// shapes evenly).  The tiling is per tensor, so a tensor's float64 partials
-// do not depend on the other tensors of its launch.
+// two 8-column chunks) of `tile_rows` consecutive rows.  A tile's size has two
+// bounds.  Per tensor: about N/32 elements, between 64K and 1M (in a launch of
+// billions of elements larger tiles spend less of the pass on set-up and
+// flushes: on the Llama-3-8B set caps of 256K / 512K / 1M / 2M measured
+// 4.30 / 4.08 / 3.97 / 3.96 ms).  Per launch: launch_elems / kFactLaunchWgs,
+// so that a launch of any size fills the 256 CUs' four workgroups each (the
+// LDS of a workgroup allows four); with N/32 alone a single tensor is 32
+// workgroups and a decoder layer 298, one wave per SIMD and most of the chip
+// idle.  Not below kFactTileSmallElems, where a tile's set-up and its column
+// partials cost more than the waves it adds.  Measured (stats kernel, us;
+// N/32 alone -> launch_elems / 512, / 1024, / 2048 with 16K): one decoder
+// layer (218M bf16) 282 -> 154, 129, 136; 4096x4096 fp32 140 -> 28, 30, 35;
+// 43M fp16 elements in odd sizes 470 -> 57, 46, 47; 7.5M bf16 in 8 matrices
+// 258 -> 76, 75, 75.
+// Tiles start at multiples of 32 rows, so the rows whose squares meet in one
+// fp32 column partial are the same in every launch; the launch decides the
+// order of the float64 additions of those partials only.
 constexpr int64_t kFactTileCols = 1024;
 constexpr int64_t kFactTileMinElems = 1 << 16;
 constexpr int64_t kFactTileMaxElems = 1 << 20;
+constexpr int64_t kFactTileSmallElems = 1 << 14;
+constexpr int64_t kFactLaunchWgs = 1024;
 
-// Transposed-view stats (strides (1, ld)) use the same column tiles but row
-// tiles of whole 64-row bands, at most kTvStatsMaxRows rows.
+// As launch_elems: the largest tiles whatever the launch.
+constexpr int64_t kCoarseTiles = (int64_t)1 << 62;
+
+// Transposed-view stats (strides (1, ld)): tiles of up to four 64-row bands,
+// one for each wave of the workgroup, and a multiple of 64 columns, half as
+// many elements as the contiguous tiles (a wave walks its columns one 64 x 64
+// tile at a time, with nothing else in flight: on 51M elements of a decoder
+// layer 1024-column tiles 59 us, the share of 1/1024 of the launch 42 us, of
+// 1/2048 37 us).
 constexpr int64_t kTvStatsMaxRows = 256;
 
 struct FactTiles {
     int64_t ct, rt, tile_rows;
-    int64_t rt_tv, tv_rows;  // row tiles of the transposed-view stats kernel
-    static FactTiles make(int64_t rows, int64_t cols) {
+    int64_t ct_tv, tv_cols, rt_tv, tv_rows;  // tiles of the transposed-view stats kernel
+    // launch_elems: elements of all tensors of the launch (>= rows * cols)
+    static FactTiles make(int64_t rows, int64_t cols, int64_t launch_elems) {
         FactTiles t;
         t.ct = (cols + kFactTileCols - 1) / kFactTileCols;
         if (t.ct < 1) t.ct = 1;
         const int64_t tc = cols < kFactTileCols ? (cols < 1 ? 1 : cols) : kFactTileCols;
         int64_t elems = rows * cols / 32;
         elems = elems < kFactTileMinElems ? kFactTileMinElems : (elems > kFactTileMaxElems ? kFactTileMaxElems : elems);
+        int64_t share = launch_elems / kFactLaunchWgs;
+        if (share < kFactTileSmallElems) share = kFactTileSmallElems;
+        if (elems > share) elems = share;
         int64_t tr = (elems + tc - 1) / tc;
-        tr = (tr + 7) & ~int64_t(7);  // whole two-row steps for each of the 4 waves
+        tr = (tr + 31) & ~int64_t(31);  // whole 8-row fp32 column groups of each of the 4 waves
         if (tr > rows) tr = rows;
         if (tr < 1) tr = 1;
         t.tile_rows = tr;
         t.rt = (rows + tr - 1) / tr;
         if (t.rt < 1) t.rt = 1;
-        int64_t tv = (tr + 63) & ~int64_t(63);
-        if (tv > kTvStatsMaxRows) tv = kTvStatsMaxRows;
+        int64_t tv = kTvStatsMaxRows;
         if (tv > rows) tv = rows < 1 ? 1 : rows;
         t.tv_rows = tv;
         t.rt_tv = (rows + tv - 1) / tv;
         if (t.rt_tv < 1) t.rt_tv = 1;
+        int64_t vc = (share / (2 * kTvStatsMaxRows) + 63) & ~int64_t(63);
+        t.tv_cols = vc < 64 ? 64 : vc > kFactTileCols ? kFactTileCols : vc;
+        t.ct_tv = (cols + t.tv_cols - 1) / t.tv_cols;
+        if (t.ct_tv < 1) t.ct_tv = 1;
         return t;
     }
 };
@@ -97,18 +119,20 @@ inline int64_t mag_shards(int64_t nb) { return nb <= kMagShardMaxBlocks ? kMagSh
 constexpr int64_t kFinRowsPerWg = 256;
 
 struct FactoredWs {
-    // double row_part[ct][rows], double col_part[max(rt, rt_tv)][cols] (per-tile partial
-    // sums, fully rewritten every step), uint32 magbits[shards][nb] (zero
+    // double row_part[max(ct, ct_tv)][rows], double col_part[max(rt, rt_tv)][cols] (per-tile
+    // partial sums, fully rewritten every step; launch_elems = rows * cols sizes them for the
+    // smallest tiles, so one workspace serves the tensor in every launch), uint32 magbits[shards][nb] (zero
     // between steps), float mag_old[nb], float minv[nb],
     // double vrow_sum[ceil(rows/256)] (partials of sum(v_row)), float vcs[cols] (sqrt(v_col)),
     // {uint32 finalize counter (zero between steps), float mean(v_row)}
     size_t off_rowp, off_colp, off_magbits, off_magold, off_minv, off_vsum, off_vcs, off_fin, total;
-    static FactoredWs make(int64_t rows, int64_t cols, int64_t nb) {
+    static FactoredWs make(int64_t rows, int64_t cols, int64_t nb, int64_t launch_elems) {
         FactoredWs w;
-        const FactTiles t = FactTiles::make(rows, cols);
+        const FactTiles t = FactTiles::make(rows, cols, launch_elems);
         size_t o = 0;
-        w.off_rowp = o;    o += align256(sizeof(double) * (size_t)(t.ct * rows));
-        const int64_t rt = t.rt > t.rt_tv ? t.rt : t.rt_tv;  // either stats layout fits
+        const int64_t ct = t.ct > t.ct_tv ? t.ct : t.ct_tv;  // either stats layout fits
+        w.off_rowp = o;    o += align256(sizeof(double) * (size_t)(ct * rows));
+        const int64_t rt = t.rt > t.rt_tv ? t.rt : t.rt_tv;
         w.off_colp = o;    o += align256(sizeof(double) * (size_t)(rt * cols));
         w.off_magbits = o; o += align256(sizeof(uint32_t) * (size_t)(nb * mag_shards(nb)));
         w.off_magold = o;  o += align256(sizeof(float) * (size_t)nb);

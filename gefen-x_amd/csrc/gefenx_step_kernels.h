@@ -482,9 +482,8 @@ struct TvStatsLds {
     double bsum[MODE == 1 ? kTvLdsBlocks : 1];
 };
 
-// Stats of a transposed view.  Workgroup (ctile, rtile) covers the same
-// kFactTileCols columns as the contiguous factored kernel (so row_part keeps
-// its layout) and tile_rows (<= 256) rows; wave w takes the 64-row band w and
+// Stats of a transposed view.  Workgroup (ctile, rtile) covers tile_cols
+// (<= kFactTileCols) columns and tile_rows (<= 256) rows; wave w takes the 64-row band w and
 // walks the workgroup's columns in 64 x 64 tiles, so the 4 waves read 512-byte
 // runs of the same storage rows at about the same time (measured 6% faster
 // than 4 waves on 4 column ranges) and a wave reads the two halves of each
@@ -522,8 +521,8 @@ __device__ __forceinline__ void stats_tv(const TensorWork& wr, int64_t wg, TvSta
     uint32_t* mb = wr.magbits + (wg % wr.shards) * nb;
     double* bsq = MODE == 1 ? wr.blk_sq + (wg % wr.shards) * nb : nullptr;
     const int64_t ctile = wg % wr.ct, rtile = wg / wr.ct;
-    const int64_t c_begin = ctile * kFactTileCols;
-    const int64_t c_end = std::min<int64_t>(c_begin + kFactTileCols, C);
+    const int64_t c_begin = ctile * wr.tile_cols;
+    const int64_t c_end = std::min<int64_t>(c_begin + wr.tile_cols, C);
     const int64_t r_begin = rtile * wr.tile_rows;
     const int64_t r_end = std::min<int64_t>(r_begin + wr.tile_rows, R);
     // blocks of the workgroup's region: few of them (large periods) reduce

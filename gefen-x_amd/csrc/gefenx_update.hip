@@ -287,6 +287,8 @@ struct WorkInput {
     const int64_t* seed_dev;
     void* workspace;
     size_t ws_bytes;
+    int64_t launch_elems;  // elements of all tensors of the launch (sizes the stats tiles)
+    int64_t ws_elems;      // the launch size the factored workspace is laid out for (its smallest tiles)
 };
 
 // The divisor of the reference's decomposed step (bc2, or sqrt(bc2) on the
@@ -328,10 +330,10 @@ static int build_work(const WorkInput& in, TensorWork& w) {
     const bool tv_g = in.gs0 == 1 && in.gs1 >= in.R && (in.gs1 * es) % 16 == 0 && aligned(in.grad, 16);
     const bool tv_p = in.ps0 == 1 && in.ps1 >= in.R && (in.ps1 * es) % 16 == 0 && aligned(in.p, 16);
     if (in.mode == 0) {
-        const FactoredWs L = FactoredWs::make(in.R, in.C, nb);
+        const FactoredWs L = FactoredWs::make(in.R, in.C, nb, in.ws_elems);
         if (in.ws_bytes < L.total)
             return set_error(GEFENX_EINVAL, "factored update: workspace %zu bytes < required %zu", in.ws_bytes, L.total);
-        const FactTiles t = FactTiles::make(in.R, in.C);
+        const FactTiles t = FactTiles::make(in.R, in.C, in.launch_elems);
         w.row_part = reinterpret_cast<double*>(ws + L.off_rowp);
         w.col_part = reinterpret_cast<double*>(ws + L.off_colp);
         w.magbits = reinterpret_cast<uint32_t*>(ws + L.off_magbits);
@@ -351,9 +353,9 @@ static int build_work(const WorkInput& in, TensorWork& w) {
                        aligned(in.grad, 16) && aligned(in.p, 16) && aligned(in.idx, 8) && aligned(in.v1, 16);
         if (!w.fast_stats && tv_shape && tv_g) {
             w.fast_stats = 2;
-            w.rt = t.rt_tv;
-            w.tile_rows = t.tv_rows;
-            w.stats_wgs = t.ct * t.rt_tv;
+            w.ct = t.ct_tv; w.rt = t.rt_tv;
+            w.tile_rows = t.tv_rows; w.tile_cols = t.tv_cols;
+            w.stats_wgs = t.ct_tv * t.rt_tv;
         }
         // column sums over many row tiles (embeddings: ~250-300) split into
         // up to 8 runs (of <= 32 partials up to 256 row tiles), so no thread
@@ -398,9 +400,9 @@ static int build_work(const WorkInput& in, TensorWork& w) {
             const bool g_contig = in.gs1 == 1 && in.gs0 == in.C;
             const bool p_contig = in.ps1 == 1 && in.ps0 == in.C;
             if (tv_shape && tv_g) {
-                const FactTiles t = FactTiles::make(in.R, in.C);
-                w.ct = t.ct; w.rt = t.rt_tv; w.tile_rows = t.tv_rows;
-                w.stats_wgs = t.ct * t.rt_tv;
+                const FactTiles t = FactTiles::make(in.R, in.C, in.launch_elems);
+                w.ct = t.ct_tv; w.rt = t.rt_tv; w.tile_rows = t.tv_rows; w.tile_cols = t.tv_cols;
+                w.stats_wgs = t.ct_tv * t.rt_tv;
                 w.fast_stats = 2;
                 w.det_rec = nullptr;  // the view tiles accumulate into the shards
             } else if (!g_contig) {
@@ -971,6 +973,7 @@ int gefenx_factored_update(
     if (rc || empty) return rc;
     if (!workspace) return set_error(GEFENX_EINVAL, "gefenx_factored_update: null workspace");
     in.workspace = workspace; in.ws_bytes = workspace_bytes;
+    in.launch_elems = in.ws_elems = in.R * in.C;
     TensorWork w;
     rc = build_work(in, w);
     if (rc) return rc;
@@ -994,7 +997,7 @@ int gefenx_factored_update_noalloc(
                             inv_bias_correction_1, weight_decay_factor, stochastic_round, rng_seed, step_scalars,
                             seed_dev, in, empty);
     if (rc || empty) return rc;
-    const FactoredWs L = FactoredWs::make(rows, cols, rows * cols / period);
+    const FactoredWs L = FactoredWs::make(rows, cols, rows * cols / period, kCoarseTiles);
     if (L.total > (size_t)GEFENX_NOALLOC_SCRATCH_BYTES)
         return set_error(GEFENX_EINVAL, "%s: a [%lld, %lld] parameter with period %lld needs %zu bytes of scratch; "
                          "the static scratch holds %zu (use gefenx_factored_update with a workspace)", fn,
@@ -1005,6 +1008,7 @@ int gefenx_factored_update_noalloc(
     if (rc) return rc;
     in.workspace = ptr;
     in.ws_bytes = GEFENX_NOALLOC_SCRATCH_BYTES;
+    in.launch_elems = in.ws_elems = kCoarseTiles;
     TensorWork w;
     rc = build_work(in, w);
     if (rc) return rc;
@@ -1052,6 +1056,7 @@ int gefenx_block_update(
     in.sr = stochastic_round ? 1 : 0; in.seed = (uint64_t)rng_seed;
     in.step_scalars = step_scalars; in.seed_dev = seed_dev;
     in.workspace = workspace; in.ws_bytes = workspace_bytes;
+    in.launch_elems = in.ws_elems = in.R * in.C;
     TensorWork w;
     rc = build_work(in, w);
     if (rc) return rc;
@@ -1078,6 +1083,7 @@ int gefenx_momentum_apply(
     in.lerp_w = (float)(1.0 - beta1); in.beta2 = 0.0f; in.alpha2 = 0.0f; in.eps = 0.0f;
     in.sc = StepScalars{(float)lr, 1.0f, 1.0f, 1.0f};
     in.workspace = workspace; in.ws_bytes = workspace_bytes;
+    in.launch_elems = in.ws_elems = in.R * in.C;
     TensorWork w;
     rc = build_work(in, w);
     if (rc) return rc;
@@ -1087,7 +1093,8 @@ int gefenx_momentum_apply(
 }
 
 static int desc_to_work(const gefenx_tensor_desc& d, int i, const void* const* qtables, int sr,
-                        int64_t seed, const float* step_scalars, const int64_t* seed_dev, TensorWork& w) {
+                        int64_t seed, const float* step_scalars, const int64_t* seed_dev, int64_t launch_elems,
+                        TensorWork& w) {
     int rc = check_dtype(d.dtype, "gefenx_multi_tensor_step");
     if (rc) return rc;
     const int64_t N = d.rows * d.cols;
@@ -1115,6 +1122,7 @@ static int desc_to_work(const gefenx_tensor_desc& d, int i, const void* const* q
     in.sr = sr ? 1 : 0; in.seed = (uint64_t)seed;
     in.step_scalars = step_scalars; in.seed_dev = seed_dev;
     in.workspace = d.workspace;
+    in.launch_elems = launch_elems; in.ws_elems = N;
     in.ws_bytes = d.factored ? gefenx_workspace_bytes(GEFENX_WS_FACTORED, d.rows, d.cols, N / d.period)
                              : gefenx_workspace_bytes(GEFENX_WS_BLOCK, d.rows, d.cols, N / d.period);
     return build_work(in, w);
@@ -1126,11 +1134,13 @@ static int build_layout(const gefenx_tensor_desc* descs, int n, const void* cons
         return set_error(GEFENX_EINVAL, "gefenx_multi_tensor_step: bad descriptor array");
     std::vector<TensorWork> works;
     works.reserve((size_t)n);
+    int64_t total = 0;
+    for (int i = 0; i < n; ++i) total += descs[i].rows * descs[i].cols;
     for (int i = 0; i < n; ++i) {
         if (descs[i].rows * descs[i].cols == 0) continue;  // empty tensors are a no-op
         TensorWork w;
         int rc = desc_to_work(descs[i], i, qtables, sr, seed, step_scalars ? step_scalars[i] : nullptr,
-                              seed_dev, w);
+                              seed_dev, total, w);
         if (rc) return rc;
         works.push_back(w);
     }

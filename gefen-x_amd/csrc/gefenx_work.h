@@ -54,7 +54,7 @@ struct TensorWork {
     int64_t R, C, N, P, nb;
     double invC, invP;
     int64_t ps0, ps1, gs0, gs1;
-    int64_t ct, rt, tile_rows, shards;
+    int64_t ct, rt, tile_rows, tile_cols, shards;  // tile_cols: transposed-view stats
     int64_t stats_wgs, nr, nc, nbw, fin_wgs, apply_wgs;
     int64_t det_elems;   // block stats: elements per workgroup
     int64_t dR, dC, dB, dP;  // apply: chunk advance for a stride of apply_wgs*256*8 elements
