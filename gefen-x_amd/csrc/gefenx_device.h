@@ -198,6 +198,24 @@ __device__ __forceinline__ void load_raw8_elems(const typename Elem<DT>::T* __re
 __device__ __forceinline__ void sq_add(float& a, float g) { a = __builtin_fmaf(g, g, a); }
 __device__ __forceinline__ void sq_add(double& a, float g) { a += (double)(g * g); }
 
+// The same 8 elements through vector loads at any element alignment (global
+// memory takes them; an access that crosses a cache line costs that line too).
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
+template <int DT>
+__device__ __forceinline__ void load_raw8_any(const typename Elem<DT>::T* __restrict__ base, Raw8<DT>& r) {
+    if constexpr (DT == F32) {
+        const GX_GLOBAL f32x4_a4* q = gbl(reinterpret_cast<const f32x4_a4*>(base));
+        const f32x4 a = __builtin_nontemporal_load(q);
+        const f32x4 b = __builtin_nontemporal_load(q + 1);
+        r.f[0] = a.x; r.f[1] = a.y; r.f[2] = a.z; r.f[3] = a.w;
+        r.f[4] = b.x; r.f[5] = b.y; r.f[6] = b.z; r.f[7] = b.w;
+    } else {
+        const u32x4 v = __builtin_nontemporal_load(gbl(reinterpret_cast<const u32x4_a2*>(base)));
+        r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
+    }
+}
+
 struct RawIdx8 { uint32_t lo, hi; };
 
 __device__ __forceinline__ RawIdx8 load_raw_idx8(const uint8_t* __restrict__ base) {

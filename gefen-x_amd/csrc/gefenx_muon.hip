@@ -628,10 +628,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const f32x16 (&
             }
             if (D == nullptr) continue;
             uint16_t* dp = D + gr * g.ldd + gc;
-            if (full && (reinterpret_cast<uintptr_t>(dp) & 15) == 0) {
+            if (full) {
                 const u32x4 dv = {(uint32_t)hv[0] | ((uint32_t)hv[1] << 16), (uint32_t)hv[2] | ((uint32_t)hv[3] << 16),
                                   (uint32_t)hv[4] | ((uint32_t)hv[5] << 16), (uint32_t)hv[6] | ((uint32_t)hv[7] << 16)};
-                *gbl(reinterpret_cast<u32x4*>(dp)) = dv;
+                *gbl(reinterpret_cast<u32x4_a2*>(dp)) = dv;  // rows of any alignment
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
@@ -650,10 +650,10 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const f32x16 (&
 #pragma unroll
                 for (int e = 0; e < 8; ++e) hv[e] = f2bf(sOut[(r8 + e) * kOutPitch + cc]);
                 uint16_t* tp = Dt + gc * g.lddt + gr;
-                if (gr + 8 <= g.M && (reinterpret_cast<uintptr_t>(tp) & 15) == 0) {
+                if (gr + 8 <= g.M) {
                     const u32x4 tv = {(uint32_t)hv[0] | ((uint32_t)hv[1] << 16), (uint32_t)hv[2] | ((uint32_t)hv[3] << 16),
                                       (uint32_t)hv[4] | ((uint32_t)hv[5] << 16), (uint32_t)hv[6] | ((uint32_t)hv[7] << 16)};
-                    *gbl(reinterpret_cast<u32x4*>(tp)) = tv;
+                    *gbl(reinterpret_cast<u32x4_a2*>(tp)) = tv;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
@@ -1322,31 +1322,31 @@ static int gemm_nt(const GemmArgs& g, int64_t batch, hipStream_t s) {
 // ==================================================================
 // Partial sums of squares (float64) of bf16(in), one per workgroup: the
 // Frobenius norm of X = in.bfloat16() read straight from the input.
-// grid (kParts, batch).  VEC: N % 8 == 0 and the input 16-byte aligned.
-template <int DT, bool VEC>
+// grid (kParts, batch).  ALIGNED: N % 8 == 0 and the input 16-byte aligned,
+// so every matrix is; otherwise the same 8-element loads at any alignment
+// and the last N % 8 elements one by one.
+template <int DT, bool ALIGNED>
 __global__ void __launch_bounds__(kT) k_ns_sumsq(const void* in, int64_t N, double* part) {
     using T = typename Elem<DT>::T;
     __shared__ double s_w[kT / 64];
     const int64_t bz = blockIdx.y;
     const T* x = static_cast<const T*>(in) + bz * N;
     double acc = 0.0;
-    if constexpr (VEC) {
-        const int64_t n8 = N / 8;
+    const int64_t n8 = N / 8;
 #pragma unroll 2
-        for (int64_t c = (int64_t)blockIdx.x * kT + threadIdx.x; c < n8; c += (int64_t)gridDim.x * kT) {
-            Raw8<DT> r;
-            load_raw8<DT>(x + c * 8, r);
+    for (int64_t c = (int64_t)blockIdx.x * kT + threadIdx.x; c < n8; c += (int64_t)gridDim.x * kT) {
+        Raw8<DT> r;
+        if constexpr (ALIGNED) load_raw8<DT>(x + c * 8, r);
+        else load_raw8_any<DT>(x + c * 8, r);
 #pragma unroll
-            for (int k = 0; k < 8; ++k) {
-                const float v = bf16f(f2bf(raw_elem<DT>(r, k)));
-                acc += (double)(v * v);
-            }
-        }
-    } else {
-        for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < N; e += (int64_t)gridDim.x * kT) {
-            const float v = bf16f(f2bf(to_f32<DT>(*gbl(x + e))));
+        for (int k = 0; k < 8; ++k) {
+            const float v = bf16f(f2bf(raw_elem<DT>(r, k)));
             acc += (double)(v * v);
         }
+    }
+    if (!ALIGNED && blockIdx.x == 0 && n8 * 8 + threadIdx.x < N) {
+        const float v = bf16f(f2bf(to_f32<DT>(*gbl(x + n8 * 8 + threadIdx.x))));
+        acc += (double)(v * v);
     }
     acc = wave_sum_d(acc);
     if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = acc;
@@ -1358,57 +1358,71 @@ __global__ void __launch_bounds__(kT) k_ns_sumsq(const void* in, int64_t N, doub
     }
 }
 
-// den = max(bf16(||X||), eps) per matrix (Tensor.norm of bf16 returns bf16).
-__global__ void k_ns_norm(const double* part, int nparts, int64_t batch, float eps, float* den) {
-    const int64_t bz = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (bz >= batch) return;
-    double t = 0.0;
-    for (int i = 0; i < nparts; ++i) t += part[bz * nparts + i];
-    const float nb = bf16f(f2bf((float)sqrt(t)));
-    den[bz] = nb < eps ? bf16f(f2bf(eps)) : nb;
-}
-
-// X (m x n) and Xt (n x m) from the input [R x C] of any grad dtype:
-// bf16(bf16(in) / den), tall inputs (R > C) transposed (m = min(R, C),
-// n = max(R, C)).  A workgroup moves one 64 x 64 tile: rows of 8 elements
-// from the input to the same-layout output (16-byte stores), and through LDS
-// (pitch 66 bf16, so the column reads below spread over the banks) to the
-// transposed output, whose rows leave as 8-row 16-byte vectors, 8 lanes per
-// 128-byte row segment.  grid (ceil(C/64), ceil(R/64), batch).  VEC: C % 8
-// == 0 and the input, X and Xt 16-byte aligned (then every 8-element row
-// piece is in bounds or entirely out).
+// X and Xt from the input [R x C] of any grad dtype: bf16(bf16(in) / den),
+// den = max(bf16(||X||), eps) (Tensor.norm of bf16 returns bf16), tall inputs
+// (R > C) transposed.  X is [mp x np], Xt [np x mp], m = min(R, C) and
+// n = max(R, C) rounded up to multiples of 64, the padding zero: every
+// Newton-Schulz product of any shape then has a K of whole 64-wide steps and
+// 16-byte rows, and zero rows and columns stay zero through the iteration.
+// (Unpadded, a K that is no multiple of 64 took the register-staged kernel:
+// the products of 1000 x 3000, batch 2, took 65.7 and 39.0 us against 36.2 and
+// 31.6 padded, those of 1111 x 777 and 2305 x 769 103-117 against 18-21, whose
+// rows were not even 16-byte aligned.)
+// A workgroup moves one 64 x 64 tile: rows of 8 elements from the input to
+// the same-layout output (16-byte stores), and through LDS (pitch 66 bf16, so
+// the column reads below spread over the banks) to the transposed output,
+// whose rows leave as 8-row 16-byte vectors, 8 lanes per 128-byte row
+// segment.  grid (Cp/64, Rp/64, batch), Rp and Cp the padded sides.  ALIGNED:
+// C % 8 == 0 and the input 16-byte aligned (every 8-element row piece is in
+// bounds or entirely out); otherwise the pieces load at any alignment and a
+// row's last one element by element.  Each workgroup adds up the matrix's
+// partial sums of squares itself, while its tile loads (a kernel of its own
+// for the norm took 21 us, most of it one thread's serial loads).
 constexpr int kTilePitch = 66;
+constexpr int64_t kNsPad = 64;
+constexpr int kNsParts = kT;  // partial sums of squares per matrix: one per thread of the load
 
-template <int DT, bool VEC>
-__global__ void __launch_bounds__(kT) k_ns_load(const void* in, int64_t R, int64_t Cc, uint16_t* X, uint16_t* Xt,
-                                                const float* den_p) {
+template <int DT, bool ALIGNED>
+__global__ void __launch_bounds__(kT) k_ns_load(const void* in, int64_t R, int64_t Cc, int64_t Rp, int64_t Cp,
+                                                uint16_t* X, uint16_t* Xt, const double* part, float eps) {
     using T = typename Elem<DT>::T;
     __shared__ uint16_t tile[64 * kTilePitch];
+    __shared__ double s_w[kT / 64];
     const int64_t bz = blockIdx.z;
-    const int64_t N = R * Cc;
-    const T* src = static_cast<const T*>(in) + bz * N;
+    const T* src = static_cast<const T*>(in) + bz * R * Cc;
     const bool tall = R > Cc;
-    uint16_t* same = (tall ? Xt : X) + bz * N;   // [R x C]
-    uint16_t* trans = (tall ? X : Xt) + bz * N;  // [C x R]
-    const float den = den_p[bz];
-    const float yden = block_recip(den);  // RN(1/den), or 0 when den or 1/den is not normal
+    uint16_t* same = (tall ? Xt : X) + bz * Rp * Cp;   // [Rp x Cp]
+    uint16_t* trans = (tall ? X : Xt) + bz * Rp * Cp;  // [Cp x Rp]
     const int64_t r0 = (int64_t)blockIdx.y * 64, c0 = (int64_t)blockIdx.x * 64;
     // both chunks' loads before any store (the output may alias the input as
     // far as the compiler knows, so a load after a store could not move up)
+    double sq = *gbl(part + bz * kNsParts + threadIdx.x);
     Raw8<DT> raws[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         const int v = threadIdx.x + k * kT;
         const int64_t r = r0 + (v >> 3), c = c0 + (v & 7) * 8;
-        if (VEC && r < R && c < Cc) load_raw8<DT>(src + r * Cc + c, raws[k]);
+        if (r < R && c + 8 <= Cc) {
+            if constexpr (ALIGNED) load_raw8<DT>(src + r * Cc + c, raws[k]);
+            else load_raw8_any<DT>(src + r * Cc + c, raws[k]);
+        }
     }
+    sq = wave_sum_d(sq);
+    if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = sq;
+    __syncthreads();
+    sq = 0.0;
+#pragma unroll
+    for (int w = 0; w < kT / 64; ++w) sq += s_w[w];
+    const float nrm = bf16f(f2bf((float)sqrt(sq)));
+    const float den = nrm < eps ? bf16f(f2bf(eps)) : nrm;
+    const float yden = block_recip(den);  // RN(1/den), or 0 when den or 1/den is not normal
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
         const int v = threadIdx.x + k * kT;
         const int row = v >> 3, c8 = (v & 7) * 8;
         const int64_t r = r0 + row, c = c0 + c8;
         uint32_t h[8];
-        if (VEC && r < R && c < Cc) {
+        if (r < R && c + 8 <= Cc) {
             const Raw8<DT>& raw = raws[k];
             // x / den through the reciprocal with one Markstein correction
             // (correctly rounded while x, the first quotient and 1/den stay
@@ -1429,18 +1443,14 @@ __global__ void __launch_bounds__(kT) k_ns_load(const void* in, int64_t R, int64
             }
 #pragma unroll
             for (int e = 0; e < 8; ++e) h[e] = f2bf(qs[e]);
-            const u32x4 pk = {h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
-            *gbl(reinterpret_cast<u32x4*>(same + r * Cc + c)) = pk;
-        } else {
+        } else {  // a row's last piece, or padding
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                h[e] = 0u;
-                if (r < R && c + e < Cc) {
-                    h[e] = f2bf(bf16f(f2bf(to_f32<DT>(*gbl(src + r * Cc + c + e)))) / den);
-                    *gbl(same + r * Cc + c + e) = (uint16_t)h[e];
-                }
-            }
+            for (int e = 0; e < 8; ++e)
+                h[e] = !ALIGNED && r < R && c + e < Cc
+                           ? f2bf(bf16f(f2bf(to_f32<DT>(*gbl(src + r * Cc + c + e)))) / den) : 0u;
         }
+        const u32x4 pk = {h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+        *gbl(reinterpret_cast<u32x4*>(same + r * Cp + c)) = pk;
         uint32_t* trow = reinterpret_cast<uint32_t*>(tile + row * kTilePitch + c8);
 #pragma unroll
         for (int q = 0; q < 4; ++q) trow[q] = h[2 * q] | (h[2 * q + 1] << 16);
@@ -1450,35 +1460,28 @@ __global__ void __launch_bounds__(kT) k_ns_load(const void* in, int64_t R, int64
     for (int k = 0; k < 2; ++k) {
         const int v = threadIdx.x + k * kT;
         const int cc = v >> 3, r8 = (v & 7) * 8;  // output row (input column), first output column
-        const int64_t c = c0 + cc, r = r0 + r8;
-        if (c >= Cc) continue;
         uint32_t h[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) h[e] = tile[(r8 + e) * kTilePitch + cc];
-        uint16_t* tp = trans + c * R + r;
-        if (VEC && r + 8 <= R && (R & 7) == 0) {
-            const u32x4 pk = {h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
-            *gbl(reinterpret_cast<u32x4*>(tp)) = pk;
-        } else {
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                if (r + e < R) *gbl(tp + e) = (uint16_t)h[e];
-        }
+        const u32x4 pk = {h[0] | (h[1] << 16), h[2] | (h[3] << 16), h[4] | (h[5] << 16), h[6] | (h[7] << 16)};
+        *gbl(reinterpret_cast<u32x4*>(trans + (c0 + cc) * Rp + r0 + r8)) = pk;
     }
 }
 
-// out [R x C] (bf16) from the normalised X / Xt (a schedule of no steps).
-__global__ void __launch_bounds__(kT) k_ns_store(const uint16_t* src, int64_t N, int64_t sX, uint16_t* out, int64_t s_out) {
-    const int64_t bz = blockIdx.y;
-    for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < N; e += (int64_t)gridDim.x * kT)
-        *gbl(out + bz * s_out + e) = *gbl(src + bz * sX + e);
+// out [R x C] (bf16) from the normalised matrix [Rp x Cp] (a schedule of no steps).
+__global__ void __launch_bounds__(kT) k_ns_store(const uint16_t* src, int64_t R, int64_t Cc, int64_t Rp, int64_t Cp,
+                                                 double invC, uint16_t* out) {
+    const int64_t bz = blockIdx.y, N = R * Cc;
+    for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < N; e += (int64_t)gridDim.x * kT) {
+        const int64_t r = div_floor(e, Cc, invC);
+        *gbl(out + bz * N + e) = *gbl(src + bz * Rp * Cp + r * Cp + (e - r * Cc));
+    }
 }
 
 struct NsWs {
-    size_t off_x, off_xt0, off_xt1, off_g, off_b, off_part, off_den, total;
-    static constexpr int kParts = 256;
+    size_t off_x, off_xt0, off_xt1, off_g, off_b, off_part, total;
     static NsWs make(int64_t batch, int64_t R, int64_t C) {
-        const int64_t m = std::min(R, C), n = std::max(R, C);
+        const int64_t m = cdiv(std::min(R, C), kNsPad) * kNsPad, n = cdiv(std::max(R, C), kNsPad) * kNsPad;
         NsWs w;
         size_t o = 0;
         const size_t mn = align256(sizeof(uint16_t) * (size_t)(batch * m * n));
@@ -1488,8 +1491,7 @@ struct NsWs {
         w.off_xt1 = o; o += mn;
         w.off_g = o; o += mm;
         w.off_b = o; o += mm;
-        w.off_part = o; o += align256(sizeof(double) * (size_t)(batch * kParts));
-        w.off_den = o; o += align256(sizeof(float) * (size_t)batch);
+        w.off_part = o; o += align256(sizeof(double) * (size_t)(batch * kNsParts));
         w.total = o;
         return w;
     }
@@ -2118,19 +2120,20 @@ int gefenx_newton_schulz(const void* in, int in_dtype, void* out, int64_t batch,
     uint16_t* G = reinterpret_cast<uint16_t*>(ws + L.off_g);
     uint16_t* Bm = reinterpret_cast<uint16_t*>(ws + L.off_b);
     double* part = reinterpret_cast<double*>(ws + L.off_part);
-    float* den = reinterpret_cast<float*>(ws + L.off_den);
     uint16_t* o16 = static_cast<uint16_t*>(out);
     const int64_t m = std::min(rows, cols), n = std::max(rows, cols);
+    const int64_t Rp = cdiv(rows, kNsPad) * kNsPad, Cp = cdiv(cols, kNsPad) * kNsPad;
+    const int64_t mp = std::min(Rp, Cp), np = std::max(Rp, Cp), sX = mp * np;
     const int64_t N = m * n;
     const bool tall = rows > cols;
-    const dim3 gt((unsigned)cdiv(cols, 64), (unsigned)cdiv(rows, 64), (unsigned)batch);
-    if (cdiv(rows, 64) > 65535 || batch > 65535)
+    const dim3 gt((unsigned)(Cp / 64), (unsigned)(Rp / 64), (unsigned)batch);
+    if (Rp / 64 > 65535 || batch > 65535)
         return set_error(GEFENX_EINVAL, "gefenx_newton_schulz: %lld rows x batch %lld exceed the launch grid",
                          (long long)rows, (long long)batch);
     // X = bf16(in) / max(bf16(||bf16(in)||), eps): the norm straight from the
     // input, the division fused into the load that lays out X and X^T
     const bool vin = N % 8 == 0 && al16(in);
-    const dim3 gp(NsWs::kParts, (unsigned)batch);
+    const dim3 gp(kNsParts, (unsigned)batch);
 #define GX_NS_SUMSQ(DTV)                                                                                   \
     if (vin) hipLaunchKernelGGL((k_ns_sumsq<DTV, true>), gp, dim3(kT), 0, s, in, N, part);                \
     else hipLaunchKernelGGL((k_ns_sumsq<DTV, false>), gp, dim3(kT), 0, s, in, N, part);
@@ -2140,12 +2143,11 @@ int gefenx_newton_schulz(const void* in, int in_dtype, void* out, int64_t batch,
         default: GX_NS_SUMSQ(BF16) break;
     }
 #undef GX_NS_SUMSQ
-    hipLaunchKernelGGL(k_ns_norm, dim3((unsigned)cdiv(batch, 64)), dim3(64), 0, s, part, NsWs::kParts, batch,
-                       (float)eps, den);
     const bool vload = cols % 8 == 0 && al16(in);
+    const float epsf = (float)eps;
 #define GX_NS_LOAD(DTV)                                                                                    \
-    if (vload) hipLaunchKernelGGL((k_ns_load<DTV, true>), gt, dim3(kT), 0, s, in, rows, cols, X, Xt[0], den); \
-    else hipLaunchKernelGGL((k_ns_load<DTV, false>), gt, dim3(kT), 0, s, in, rows, cols, X, Xt[0], den);
+    if (vload) hipLaunchKernelGGL((k_ns_load<DTV, true>), gt, dim3(kT), 0, s, in, rows, cols, Rp, Cp, X, Xt[0], part, epsf); \
+    else hipLaunchKernelGGL((k_ns_load<DTV, false>), gt, dim3(kT), 0, s, in, rows, cols, Rp, Cp, X, Xt[0], part, epsf);
     switch (in_dtype) {
         case F32: GX_NS_LOAD(F32) break;
         case F16: GX_NS_LOAD(F16) break;
@@ -2156,7 +2158,7 @@ int gefenx_newton_schulz(const void* in, int in_dtype, void* out, int64_t batch,
     if (rc) return rc;
     if (steps == 0) {
         const dim3 g2(grid_for(N, 4096), (unsigned)batch);
-        hipLaunchKernelGGL(k_ns_store, g2, dim3(kT), 0, s, tall ? Xt[0] : X, N, N, o16, N);
+        hipLaunchKernelGGL(k_ns_store, g2, dim3(kT), 0, s, tall ? Xt[0] : X, rows, cols, Rp, Cp, 1.0 / (double)cols, o16);
         return launch_check("newton-schulz epilogue");
     }
     int cur = 0;
@@ -2168,17 +2170,22 @@ int gefenx_newton_schulz(const void* in, int in_dtype, void* out, int64_t batch,
         const bool last = it + 1 == steps;
         int ph = prof_begin(GEFENX_K_NS_GEMM, 0.0, flops_iter, s);
         // G = X X^T (symmetric: lower tiles, mirrored)
-        GemmArgs g1{X, n, N, X, n, N, nullptr, 0, 0, G, m, m * m, G, m, m * m, m, m, n, 1.0f, 0.0f, 0, 1};
+        GemmArgs g1{X, np, sX, X, np, sX, nullptr, 0, 0, G, mp, mp * mp, G, mp, mp * mp, mp, mp, np, 1.0f, 0.0f, 0, 1};
         rc = gemm_nt(g1, batch, s);
         // B = b G + c G G^T (symmetric: lower tiles, mirrored)
-        GemmArgs gg{G, m, m * m, G, m, m * m, G, m, m * m, Bm, m, m * m, Bm, m, m * m, m, m, m, c, b, 0, 1};
+        GemmArgs gg{G, mp, mp * mp, G, mp, mp * mp, G, mp, mp * mp, Bm, mp, mp * mp, Bm, mp, mp * mp, mp, mp, mp, c, b,
+                    0, 1};
         if (!rc) rc = gemm_nt(gg, batch, s);
         // X = a X + B X  (B operand X^T), X^T of the result into the other
-        // buffer; the last iteration writes the result straight to out in the
-        // input's orientation (X when wide, X^T when tall) and nothing else
-        uint16_t* D = last ? (tall ? nullptr : o16) : X;
-        uint16_t* Dt = last ? (tall ? o16 : nullptr) : Xt[cur ^ 1];
-        GemmArgs gx{Bm, m, m * m, Xt[cur], m, N, X, n, N, D, n, N, Dt, m, N, m, n, m, 1.0f, a, 0};
+        // buffer; the last iteration writes the result, without the padding,
+        // straight to out in the input's orientation (X when wide, X^T when
+        // tall) and nothing else
+        GemmArgs gx{Bm, mp, mp * mp, Xt[cur], mp, sX, X, np, sX, X, np, sX, Xt[cur ^ 1], mp, sX, mp, np, mp, 1.0f, a, 0};
+        if (last) {
+            gx.M = m; gx.N = n;
+            gx.D = tall ? nullptr : o16; gx.ldd = n; gx.sD = N;
+            gx.Dt = tall ? o16 : nullptr; gx.lddt = m; gx.sDt = N;
+        }
         if (!rc) rc = gemm_nt(gx, batch, s);
         prof_end(ph, s);
         if (rc) return rc;
