@@ -232,6 +232,13 @@ __device__ __forceinline__ RawIdx8 load_raw_idx8_cached(const uint8_t* __restric
     return RawIdx8{v.x, v.y};
 }
 
+// The same at any alignment.
+typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
+__device__ __forceinline__ RawIdx8 load_raw_idx8_any(const uint8_t* __restrict__ base) {
+    const u32x2 v = __builtin_nontemporal_load(gbl(reinterpret_cast<const u32x2_a1*>(base)));
+    return RawIdx8{v.x, v.y};
+}
+
 __device__ __forceinline__ RawIdx8 load_raw_idx8_elems(const uint8_t* __restrict__ base) {
     RawIdx8 r{0u, 0u};
 #pragma unroll
@@ -436,6 +443,58 @@ __device__ __forceinline__ uint32_t wave_max_u63(uint32_t v) {
     o = dpp32<0x142, 0xa>(v); v = o > v ? o : v;
     o = dpp32<0x143, 0xc>(v); v = o > v ? o : v;
     return v;
+}
+
+// Lane-order run starts (bit l: lane l begins a new key) and the segmented
+// suffix sum / max: each lane ends with the sum (max) of its run from itself
+// to the run's last lane, so a run's first lane holds the run's total.
+__device__ __forceinline__ uint64_t run_heads(int64_t key) {
+    const int lane = threadIdx.x & 63;
+    const uint32_t lo = (uint32_t)__shfl_up((int)(uint32_t)key, 1, 64);
+    const uint32_t hi = (uint32_t)__shfl_up((int)(uint32_t)((uint64_t)key >> 32), 1, 64);
+    const int64_t prev = (int64_t)(((uint64_t)hi << 32) | lo);
+    return (uint64_t)__ballot(lane == 0 || prev != key);
+}
+
+__device__ __forceinline__ double seg_suffix_sum(double v, uint64_t heads) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t after = lane < 63 ? heads >> (lane + 1) : 0ull;  // run starts past this lane
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const double o = __shfl_down(v, d, 64);
+        const bool ok = lane + d < 64 && (after & ((1ull << d) - 1ull)) == 0ull;
+        v = ok ? v + o : v;
+    }
+    return v;
+}
+
+__device__ __forceinline__ uint32_t seg_suffix_max(uint32_t m, uint64_t heads) {
+    const int lane = threadIdx.x & 63;
+    const uint64_t after = lane < 63 ? heads >> (lane + 1) : 0ull;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const uint32_t o = (uint32_t)__shfl_down((int)m, d, 64);
+        const bool ok = lane + d < 64 && (after & ((1ull << d) - 1ull)) == 0ull;
+        m = (ok && o > m) ? o : m;
+    }
+    return m;
+}
+
+// Folds each lane's block max (key: its block, -1 for none; m: ordered bits)
+// into mb: lanes of one block, consecutive in a wave, meet in registers, so a
+// block takes one atomic for each wave that holds some of it.
+__device__ __forceinline__ void wave_block_max(uint32_t* mb, int64_t key, uint32_t m) {
+    const int32_t lo = __builtin_amdgcn_readfirstlane((int)(uint32_t)key);
+    const int32_t hi = __builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)key >> 32));
+    const int64_t k0 = (int64_t)(((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+    if (__all(key == k0)) {
+        const uint32_t r = wave_max_u63(m);
+        if ((threadIdx.x & 63) == 63 && key >= 0 && r != 0u) gatomic_max(mb + key, r);
+    } else {
+        const uint64_t heads = run_heads(key);
+        const uint32_t r = seg_suffix_max(m, heads);
+        if (((heads >> (threadIdx.x & 63)) & 1ull) != 0ull && key >= 0 && r != 0u) gatomic_max(mb + key, r);
+    }
 }
 
 // Stage the quantisation table parts a kernel needs into LDS.  thr is padded

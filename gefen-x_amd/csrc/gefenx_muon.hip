@@ -90,13 +90,21 @@ __device__ __forceinline__ float mom_u(float cr, float m_old, float g, float w) 
     return round_dt<DT>(l);
 }
 
+constexpr int kPiece = 8;
+
 // Offset of logical element e of a [R, C] view with strides (gs0, gs1).
 __device__ __forceinline__ int64_t view_offset(int64_t e, int64_t C, double invC, int64_t s0, int64_t s1) {
     const int64_t r = div_floor(e, C, invC);
     return r * s0 + (e - r * C) * s1;
 }
 
-// Any layout: grid-stride over the matrix's elements.
+// Any layout and block length: grid-stride over 8-element pieces in logical
+// order, vector loads at any alignment for a contiguous grad.  The lanes of a
+// wave hold consecutive pieces, so a block takes one atomic per wave that
+// holds some of it, and one more for a piece in which it ends.  (With one
+// element per thread and an atomic each time the grid stride left its block,
+// 2305 x 769 fp32 with rows as blocks took 171 us and 1111 x 777 82; now 6.5
+// and 5.8.)
 template <int DT>
 __global__ void __launch_bounds__(kT) k_mom_max(MomArgs a, MomBatch bt) {
     using T = typename Elem<DT>::T;
@@ -107,25 +115,53 @@ __global__ void __launch_bounds__(kT) k_mom_max(MomArgs a, MomBatch bt) {
     const T* g = static_cast<const T*>(it.g);
     const bool dense = it.gs1 == 1 && it.gs0 == a.C;
     uint32_t* mb = it.magbits + ((int64_t)blockIdx.x % it.shards) * it.nb;
-    const int64_t stride = (int64_t)gridDim.x * kT;
-    int64_t cur = -1;
-    uint32_t cbits = 0u;
-    float mo = 0.0f;
-    for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < a.N; e += stride) {
-        const int64_t b = div_floor(e, it.P, it.invP);
-        if (b != cur) {
-            if (cur >= 0 && cbits) gatomic_max(mb + cur, cbits);
-            cur = b;
-            cbits = 0u;
-            mo = *gbl(it.mag + b);
+    const int64_t np = cdiv(a.N, kPiece);
+    for (int64_t p0 = (int64_t)blockIdx.x * kT; p0 < np; p0 += (int64_t)gridDim.x * kT) {
+        const int64_t e0 = (p0 + threadIdx.x) * kPiece;
+        int64_t b = -1;
+        uint32_t m = 0u;
+        if (e0 < a.N) {
+            const int nval = (int)std::min<int64_t>(kPiece, a.N - e0);
+            Raw8<DT> gr;
+            RawIdx8 ir;
+            float gv[kPiece];
+            uint32_t iv[kPiece];
+            if (dense && nval == kPiece) {
+                load_raw8_any<DT>(g + e0, gr);
+                ir = load_raw_idx8_any(it.idx + e0);
+#pragma unroll
+                for (int k = 0; k < kPiece; ++k) {
+                    gv[k] = raw_elem<DT>(gr, k);
+                    iv[k] = raw_idx(ir, k);
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < kPiece; ++k) {
+                    const int64_t e = k < nval ? e0 + k : e0;
+                    gv[k] = to_f32<DT>(*gbl(g + (dense ? e : view_offset(e, a.C, a.invC, it.gs0, it.gs1))));
+                    iv[k] = *gbl(it.idx + e);
+                }
+            }
+            b = div_floor(e0, it.P, it.invP);
+            int64_t pin = e0 - b * it.P;
+            float mo = *gbl(it.mag + b);
+#pragma unroll
+            for (int k = 0; k < kPiece; ++k) {
+                if (k >= nval) break;
+                const float u = mom_u<DT>(s_cbr[iv[k]], mo, gv[k], a.w);
+                const uint32_t ub = __float_as_uint(u) & 0x7fffffffu;  // ordered: NaN > inf > finite
+                m = ub > m ? ub : m;
+                if (++pin == it.P && k + 1 < nval) {
+                    if (m) gatomic_max(mb + b, m);
+                    ++b;
+                    pin = 0;
+                    m = 0u;
+                    mo = *gbl(it.mag + b);
+                }
+            }
         }
-        const int64_t ge = dense ? e : view_offset(e, a.C, a.invC, it.gs0, it.gs1);
-        const float gv = to_f32<DT>(*gbl(g + ge));
-        const float u = mom_u<DT>(s_cbr[*gbl(it.idx + e)], mo, gv, a.w);
-        const uint32_t ub = __float_as_uint(u) & 0x7fffffffu;  // ordered: NaN > inf > finite
-        cbits = ub > cbits ? ub : cbits;
+        wave_block_max(mb, b, m);
     }
-    if (cur >= 0 && cbits) gatomic_max(mb + cur, cbits);
 }
 
 __global__ void __launch_bounds__(kT) k_mom_finalize(MomBatch bt) {
@@ -1711,9 +1747,15 @@ __global__ void __launch_bounds__(kT) k_muon_apply(MuonApplyArgs a, ApplyBatch b
 }
 
 // Cautious agreement counts of n matrices (grid (parts, n)): the update u'
-// as the apply forms it (NorMuon row scale included) against the raw grad;
-// one atomic per wave into the matrix's 64-bit counter (a count is exact in
-// any order).  C % 8 == 0: chunks of 8 along a row, else element by element.
+// as the apply forms it (NorMuon row scale included) against the raw grad.
+// C % 8 == 0: chunks of 8 along a row; a contiguous grad with any C: 8-element
+// pieces at any alignment; else element by element.  A workgroup's count goes
+// out as one atomic, and at most kCautWgs workgroups share a matrix's counter:
+// a count is exact in any order, but atomics on one address take ~12 ns each
+// (one per wave of up to 2048 workgroups: 2305 x 769 103 us, 1000 x 3000 batch
+// 2 144; now 9.6 and 15.1).
+constexpr int64_t kCautWgs = 1024;
+
 struct CautItem {
     const void* g;
     int64_t gs0, gs1;
@@ -1750,6 +1792,41 @@ __global__ void __launch_bounds__(kT) k_cautious_count(const uint16_t* U, const 
                 cnt += cautious_agree<DT>(x, gv[e]) ? 1u : 0u;
             }
         }
+    } else if (it.gs1 == 1 && it.gs0 == C) {
+        using T = typename Elem<DT>::T;
+        const T* g = static_cast<const T*>(it.g);
+        for (int64_t e0 = ((int64_t)blockIdx.x * kT + threadIdx.x) * kPiece; e0 < N;
+             e0 += (int64_t)gridDim.x * kT * kPiece) {
+            const int nval = (int)std::min<int64_t>(kPiece, N - e0);
+            u32x4 uv;
+            Raw8<DT> gr;
+            if (nval == kPiece) {
+                uv = __builtin_nontemporal_load(gbl(reinterpret_cast<const u32x4_a2*>(u + e0)));
+                load_raw8_any<DT>(g + e0, gr);
+            }
+            int64_t r = div_floor(e0, C, invC);
+            int64_t c = e0 - r * C;
+            float sc = s ? bf16f(*gbl(s + r)) : 1.0f;
+#pragma unroll
+            for (int e = 0; e < kPiece; ++e) {
+                if (e >= nval) break;
+                float x, gv;
+                if (nval == kPiece) {
+                    x = bf16f((uint16_t)(uv[e >> 1] >> (16 * (e & 1))));
+                    gv = raw_elem<DT>(gr, e);
+                } else {
+                    x = bf16f(*gbl(u + e0 + e));
+                    gv = to_f32<DT>(*gbl(g + e0 + e));
+                }
+                if (s) x = bf16f(f2bf(x * sc));
+                cnt += cautious_agree<DT>(x, gv) ? 1u : 0u;
+                if (++c == C && e + 1 < nval) {
+                    c = 0;
+                    ++r;
+                    if (s) sc = bf16f(*gbl(s + r));
+                }
+            }
+        }
     } else {
         using T = typename Elem<DT>::T;
         for (int64_t e = (int64_t)blockIdx.x * kT + threadIdx.x; e < N; e += (int64_t)gridDim.x * kT) {
@@ -1762,9 +1839,14 @@ __global__ void __launch_bounds__(kT) k_cautious_count(const uint16_t* U, const 
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) cnt += (uint32_t)__shfl_xor((int)cnt, off, 64);
-    if ((threadIdx.x & 63) == 0 && cnt != 0u)
-        (void)__hip_atomic_fetch_add(gbl(it.count), (unsigned long long)cnt, __ATOMIC_RELAXED,
-                                     __HIP_MEMORY_SCOPE_AGENT);
+    __shared__ uint32_t s_cnt[kT / 64];
+    if ((threadIdx.x & 63) == 0) s_cnt[threadIdx.x >> 6] = cnt;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long t = 0ull;
+        for (int w = 0; w < kT / 64; ++w) t += s_cnt[w];
+        if (t != 0ull) (void)__hip_atomic_fetch_add(gbl(it.count), t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 static unsigned grid_for(int64_t n, int64_t cap = 8192) {
@@ -1808,11 +1890,12 @@ static void mom_launch(const MomArgs& a, const MomBatch& bt, int n, int dtype, b
 #undef GX_EMIT_FAST
         return;
     }
-    const dim3 g(grid_for(a.N, 16384), (unsigned)n);
+    const dim3 g(grid_for(a.N, 16384), (unsigned)n);  // emit: one element per thread
+    const dim3 gm(grid_for(cdiv(a.N, (int64_t)kPiece), 4096), (unsigned)n);
     switch (dtype) {
-        case F32: hipLaunchKernelGGL(k_mom_max<F32>, g, dim3(kT), 0, s, a, bt); break;
-        case F16: hipLaunchKernelGGL(k_mom_max<F16>, g, dim3(kT), 0, s, a, bt); break;
-        default: hipLaunchKernelGGL(k_mom_max<BF16>, g, dim3(kT), 0, s, a, bt); break;
+        case F32: hipLaunchKernelGGL(k_mom_max<F32>, gm, dim3(kT), 0, s, a, bt); break;
+        case F16: hipLaunchKernelGGL(k_mom_max<F16>, gm, dim3(kT), 0, s, a, bt); break;
+        default: hipLaunchKernelGGL(k_mom_max<BF16>, gm, dim3(kT), 0, s, a, bt); break;
     }
     hipLaunchKernelGGL(k_mom_finalize, gfin, dim3(kT), 0, s, bt);
 #define GX_EMIT(SRV)                                                                                       \
@@ -2043,7 +2126,7 @@ static int cautious_count_batch(const char* fn, const gefenx_muon_item* items, i
         // counters cleared by a kernel (no memset node under graph capture)
         hipLaunchKernelGGL(k_cautious_zero, dim3(1), dim3(kMaxBatch), 0, s, bt, m);
         if (N == 0) continue;
-        const dim3 g(grid_for(cols % 8 == 0 ? N / 8 : N, 2048), (unsigned)m);
+        const dim3 g(grid_for(cdiv(N, 4 * (int64_t)kPiece), kCautWgs), (unsigned)m);  // about four pieces per thread
         const uint16_t* Ui = U + (size_t)i0 * (size_t)N;
         const uint16_t* Si = S ? S + (size_t)i0 * (size_t)rows : nullptr;
         const double invC = 1.0 / (double)cols;

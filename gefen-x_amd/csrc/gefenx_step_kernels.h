@@ -736,41 +736,6 @@ __device__ __forceinline__ void stats_tv_wg(const TensorWork& w, int64_t wg) {
 static_assert(kThreads == kCodebookMax, "one codebook entry per thread");
 static_assert(2 * kDetIters * kWaves == 64, "the workgroup's run partials fill one wave");
 
-// Lane-order run starts (bit l: lane l begins a new key) and the segmented
-// suffix sum / max: each lane ends with the sum (max) of its run from itself
-// to the run's last lane, so a run's first lane holds the run's total.
-__device__ __forceinline__ uint64_t run_heads(int64_t key) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t lo = (uint32_t)__shfl_up((int)(uint32_t)key, 1, 64);
-    const uint32_t hi = (uint32_t)__shfl_up((int)(uint32_t)((uint64_t)key >> 32), 1, 64);
-    const int64_t prev = (int64_t)(((uint64_t)hi << 32) | lo);
-    return (uint64_t)__ballot(lane == 0 || prev != key);
-}
-
-__device__ __forceinline__ double seg_suffix_sum(double v, uint64_t heads) {
-    const int lane = threadIdx.x & 63;
-    const uint64_t after = lane < 63 ? heads >> (lane + 1) : 0ull;  // run starts past this lane
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const double o = __shfl_down(v, d, 64);
-        const bool ok = lane + d < 64 && (after & ((1ull << d) - 1ull)) == 0ull;
-        v = ok ? v + o : v;
-    }
-    return v;
-}
-
-__device__ __forceinline__ uint32_t seg_suffix_max(uint32_t m, uint64_t heads) {
-    const int lane = threadIdx.x & 63;
-    const uint64_t after = lane < 63 ? heads >> (lane + 1) : 0ull;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_down((int)m, d, 64);
-        const bool ok = lane + d < 64 && (after & ((1ull << d) - 1ull)) == 0ull;
-        m = (ok && o > m) ? o : m;
-    }
-    return m;
-}
-
 // Flush a wave's running block max (wave-uniform key and value): one atomic
 // into the workgroup's shard.
 __device__ __forceinline__ void flush_det_max(uint32_t* mb, int64_t key, int64_t nb, uint32_t m) {
