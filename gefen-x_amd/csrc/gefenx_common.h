@@ -61,6 +61,15 @@ constexpr int64_t kFactTileMaxElems = 1 << 20;
 constexpr int64_t kFactTileSmallElems = 1 << 14;
 constexpr int64_t kFactLaunchWgs = 1024;
 
+// Contiguous matrices of 8 to 256 columns: a wave takes several rows at a
+// time (stats_narrow), a power of two of lanes for each.  Lanes per row for `cols`:
+constexpr int64_t kNarrowMaxCols = 256;
+inline int narrow_lanes(int64_t cols) {
+    int l = 1;
+    while (8 * l < cols) l *= 2;
+    return l;
+}
+
 // As launch_elems: the largest tiles whatever the launch.
 constexpr int64_t kCoarseTiles = (int64_t)1 << 62;
 
@@ -87,7 +96,9 @@ struct FactTiles {
         if (share < kFactTileSmallElems) share = kFactTileSmallElems;
         if (elems > share) elems = share;
         int64_t tr = (elems + tc - 1) / tc;
-        tr = (tr + 31) & ~int64_t(31);  // whole 8-row fp32 column groups of each of the 4 waves
+        // whole 8-row fp32 column groups of each of the 4 waves (narrow: of each lane)
+        const int64_t gran = cols >= 8 && cols <= kNarrowMaxCols ? 32 * (64 / narrow_lanes(cols)) : 32;
+        tr = (tr + gran - 1) / gran * gran;
         if (tr > rows) tr = rows;
         if (tr < 1) tr = 1;
         t.tile_rows = tr;

@@ -250,6 +250,29 @@ __device__ __forceinline__ RawIdx8 load_raw_idx8_elems(const uint8_t* __restrict
     return r;
 }
 
+// Elements s .. 7 of a chunk moved down to 0 .. 7 - s (s in 0..7, per lane;
+// zeros follow).
+template <int DT>
+__device__ __forceinline__ void shift_down(Raw8<DT>& g, RawIdx8& i, int s) {
+    if constexpr (DT == F32) {
+#pragma unroll
+        for (int d = 4; d > 0; d >>= 1)
+#pragma unroll
+            for (int k = 0; k < 8; ++k) g.f[k] = (s & d) ? (k + d < 8 ? g.f[k + d] : 0.0f) : g.f[k];
+    } else {
+#pragma unroll
+        for (int d = 2; d > 0; d >>= 1)  // whole words
+#pragma unroll
+            for (int k = 0; k < 4; ++k) g.w[k] = (s & (2 * d)) ? (k + d < 4 ? g.w[k + d] : 0u) : g.w[k];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            g.w[k] = (s & 1) ? (g.w[k] >> 16) | (k + 1 < 4 ? g.w[k + 1] << 16 : 0u) : g.w[k];
+    }
+    const uint64_t v = (((uint64_t)i.hi << 32) | i.lo) >> (8 * s);
+    i.lo = (uint32_t)v;
+    i.hi = (uint32_t)(v >> 32);
+}
+
 __device__ __forceinline__ uint32_t raw_idx(const RawIdx8& r, int k) {
     return ((k < 4 ? r.lo : r.hi) >> (8 * (k & 3))) & 0xffu;
 }

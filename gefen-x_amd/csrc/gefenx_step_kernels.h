@@ -39,7 +39,14 @@ __device__ __forceinline__ void wavemax_flush63(uint32_t* __restrict__ mb, WaveM
 // of the row sum (one value per row per column tile).  Column sums: fp32 in
 // registers over 8 rows, then float64; the 4 waves combine in LDS at the end.
 // Both go out as float64 partials (no float atomics, deterministic).
-// FAST: contiguous, 16-byte aligned grad, C % 8 == 0, P % 8 == 0.
+// FAST: contiguous grad and C >= 8, any alignment, any C and P (the vector
+// loads take any address; a row's last chunk, when C % 8 != 0, loads the row's
+// last 8 elements and shifts its own down).  Blocks that end inside a wave's
+// row segment combine over the lanes first (wave_block_max): one atomic per
+// block and wave where each lane used to send its own.  Measured, us: 43M fp16
+// elements of which two matrices are odd-sized 46 + 48 (the odd ones through
+// element loads in a launch of their own) -> 49; 7.5M bf16 elements with
+// 256-element blocks 75 -> 40.
 // ====================================================================
 struct FactStatsLds {
     float cbr[kCodebookMax];
@@ -87,8 +94,8 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
         cc[h] = tc0 + h * (kFactTileCols / 2) + (int64_t)lane * kChunk;
         nv[h] = (int)std::max<int64_t>(0, std::min<int64_t>(kChunk, C - cc[h]));
         // FAST loads every chunk unconditionally: a chunk past C (nv == 0,
-        // skipped by the math) reads the row's last chunk instead
-        ccl[h] = nv[h] > 0 ? cc[h] : C - kChunk;
+        // skipped by the math) or cut by it reads the row's last 8 elements
+        ccl[h] = nv[h] == kChunk ? cc[h] : C - kChunk;
     }
     const int64_t r_begin = rtile * tile_rows;
     const int64_t r_end = std::min<int64_t>(r_begin + tile_rows, R);
@@ -132,6 +139,7 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
         hall[h] = tc0 + (h + 1) * (kFactTileCols / 2) <= C;
         hany[h] = tc0 + h * (kFactTileCols / 2) < C;
     }
+    const bool cut = (C & 7) != 0;  // a chunk cut by C may sit in a half that is not full
 
     // One batch = the wave's next two rows (r0, r0 + 4): raw grads and
     // indices, plus (FAST) the old magnitude of each row segment's first
@@ -151,13 +159,13 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
             const int64_t r = rr0 + (int64_t)u * kWaves;
             if constexpr (FAST) {
                 // rows past the tile re-read the tile's last row; the math
-                // stops before them (C % 8 == 0, so nv is 0 or 8)
+                // stops before them
                 const int64_t rl = r < r_end ? r : r_end - 1;
 #pragma unroll
                 for (int h = 0; h < H; ++h) {
                     const int64_t el = rl * C + ccl[h];
-                    load_raw8<DT>(g + el, b.graw[u][h]);
-                    b.iraw[u][h] = load_raw_idx8(idxp + el);
+                    load_raw8_any<DT>(g + el, b.graw[u][h]);
+                    b.iraw[u][h] = load_raw_idx8_any(idxp + el);
                 }
                 b.mo[u] = sload(mag_old + (pblk < nb ? pblk : nb - 1));  // uniform: scalar load
                 ppin += dP4;
@@ -177,11 +185,18 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
             }
         }
     };
-    auto reduce_batch = [&](int64_t rr0, const Batch& b) {
+    auto reduce_batch = [&](int64_t rr0, Batch& b) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const int64_t r = rr0 + (int64_t)u * kWaves;
             if (r >= r_end) break;
+            if constexpr (FAST) {
+                if (cut) {
+#pragma unroll
+                    for (int h = 0; h < H; ++h)
+                        if (hany[h] && !hall[h]) shift_down<DT>(b.graw[u][h], b.iraw[u][h], (kChunk - nv[h]) & 7);
+                }
+            }
             Acc rs[H];
             const bool uniform = (pin + span - 1) < P;
             if (uniform) {
@@ -207,9 +222,9 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
 #pragma unroll
                         for (int k = 0; k < kChunk; ++k) {
                             float gv = raw_elem<DT>(b.graw[u][h], k);
-                            if constexpr (decltype(masked)::value) gv = nv[h] > 0 ? gv : 0.0f;
+                            if constexpr (decltype(masked)::value) gv = nv[h] > k ? gv : 0.0f;
                             const float uu = momentum_value<LF>(s_cbr[raw_idx(b.iraw[u][h], k)], mag_cur, gv, mc);
-                            if constexpr (decltype(masked)::value) mf = nv[h] > 0 ? __builtin_fmaxf(mf, fabsf(uu)) : mf;
+                            if constexpr (decltype(masked)::value) mf = nv[h] > k ? __builtin_fmaxf(mf, fabsf(uu)) : mf;
                             else mf = __builtin_fmaxf(mf, fabsf(uu));
                             sq_add(rs[h], gv);
                             sq_add(colf[h][k], gv);
@@ -235,6 +250,7 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
                             if (nv[h] == 0) continue;
 #pragma unroll
                             for (int k = 0; k < kChunk; ++k) {
+                                if (k >= nv[h]) continue;
                                 const float uu = momentum_value<LF>(s_cbr[raw_idx(b.iraw[u][h], k)], mag_cur,
                                                                     raw_elem<DT>(b.graw[u][h], k), mc);
                                 const uint32_t ub = __float_as_uint(uu) & 0x7fffffffu;
@@ -263,18 +279,25 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
                     wm.bits = m;
                 }
             } else {
-                // blocks end inside this row segment: per-lane runs, one atomic per run
+                // blocks end inside this row segment: per-lane blocks; a
+                // block that ends inside a chunk (P % 8 != 0) sends its part
+                // at once, each chunk's last block meets its neighbours'
                 wavemax_flush63(mb, wm);
                 wm.blk = -1;
+                int64_t bb[H], pp[H];
+                float mo[H];
+#pragma unroll
+                for (int h = 0; h < H; ++h) {
+                    const int64_t off = pin + (cc[h] - tc0);
+                    const int64_t db = div_floor(off, P, invP);
+                    bb[h] = nv[h] > 0 ? blk + db : -1;
+                    pp[h] = off - db * P;
+                    mo[h] = nv[h] > 0 ? *gbl(mag_old + bb[h]) : 0.0f;
+                }
 #pragma unroll
                 for (int h = 0; h < H; ++h) {
                     rs[h] = 0;
-                    if (nv[h] == 0) continue;
-                    const int64_t off = pin + (cc[h] - tc0);
-                    const int64_t db = div_floor(off, P, invP);
-                    int64_t bb = blk + db;
-                    int64_t pp = off - db * P;
-                    float mo = *gbl(mag_old + bb);
+                    if (!hany[h]) continue;
                     uint32_t m = 0u;
 #pragma unroll
                     for (int k = 0; k < kChunk; ++k) {
@@ -283,21 +306,21 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
                             uint32_t ix;
                             if constexpr (FAST) { gv = raw_elem<DT>(b.graw[u][h], k); ix = raw_idx(b.iraw[u][h], k); }
                             else { gv = b.gsc[u][h][k]; ix = b.isc[u][h][k]; }
-                            const float uu = momentum_value<LF>(s_cbr[ix], mo, gv, mc);
+                            const float uu = momentum_value<LF>(s_cbr[ix], mo[h], gv, mc);
                             const uint32_t ub = __float_as_uint(uu) & 0x7fffffffu;
                             m = ub > m ? ub : m;
                             sq_add(rs[h], gv);
                             sq_add(colf[h][k], gv);
-                            if (++pp == P) {
-                                if (m) gatomic_max(mb + bb, m);
+                            if (++pp[h] == P && k + 1 < nv[h]) {
+                                if (m) gatomic_max(mb + bb[h], m);
                                 m = 0u;
-                                pp = 0;
-                                ++bb;
-                                if (k + 1 < nv[h]) mo = *gbl(mag_old + bb);
+                                pp[h] = 0;
+                                ++bb[h];
+                                mo[h] = *gbl(mag_old + bb[h]);
                             }
                         }
                     }
-                    if (m) gatomic_max(mb + bb, m);
+                    wave_block_max(mb, bb[h], m);
                 }
             }
             double rsum = 0.0;
@@ -380,6 +403,113 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
         if (c < span) *gbl(col_part + rtile * C + tc0 + c) = sum;
     }
 }
+
+// ====================================================================
+// Factored stats of a contiguous matrix of 8 to kNarrowMaxCols columns, any
+// alignment and P.  L lanes (a power of two, 8 columns each) take a row, a wave
+// 64 / L rows at a time, four such steps in flight; the workgroup covers
+// tile_rows rows of all columns.  A row's lanes add up its sum of squares, a
+// lane keeps its columns' sums (fp32 over 8 rows, then float64), the lanes of
+// one column meet in LDS at the end in a fixed order.  stats_factored would
+// leave all but C / 16 of a wave's lanes idle and walk the rows one by one: a
+// set of 16-column and 16-row fp32 adapters 246 -> 16 us.
+// ====================================================================
+template <int DT, int LF>
+__device__ __forceinline__ void stats_narrow(const TensorWork& wr, int64_t wg, FactStatsLds& lds) {
+    using T = typename Elem<DT>::T;
+    using Acc = std::conditional_t<DT == F32, double, float>;
+    constexpr int Q = 4;  // steps in flight
+    float* s_cbr = lds.cbr;
+    if (threadIdx.x < kCodebookMax) s_cbr[threadIdx.x] = *gbl(wr.qt->cbr + threadIdx.x);
+    const T* g = static_cast<const T*>(wr.grad);
+    const uint8_t* idxp = wr.idx;
+    const float* mag_old = wr.mag;
+    const int64_t R = wr.R, C = wr.C, P = wr.P;
+    const double invP = wr.invP;
+    const MomentumCoef mc = wr.mc;
+    uint32_t* mb = wr.magbits + (wg % wr.shards) * wr.nb;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lgL = wr.lg_lanes, L = 1 << lgL, rpw = 64 >> lgL;
+    const int sub = lane >> lgL, c = (lane & (L - 1)) * kChunk;
+    const int nv = (int)std::max<int64_t>(0, std::min<int64_t>(kChunk, C - c));
+    const int64_t cl = nv == kChunk ? c : C - kChunk;  // a lane past C or cut by it reads the row's last 8
+    const int sh = (kChunk - nv) & 7;
+    const bool cut = (C & 7) != 0;
+    const int64_t r_begin = wg * wr.tile_rows;
+    const int64_t r_end = std::min<int64_t>(r_begin + wr.tile_rows, R);
+    __syncthreads();
+    Acc colf[kChunk];
+    double cold[kChunk];
+#pragma unroll
+    for (int k = 0; k < kChunk; ++k) { colf[k] = 0; cold[k] = 0.0; }
+    int nf = 0;
+    for (int64_t r0 = r_begin + wave * rpw; r0 < r_end; r0 += (int64_t)Q * kWaves * rpw) {
+        Raw8<DT> gr[Q];
+        RawIdx8 ir[Q];
+        int64_t bb[Q], pp[Q];
+        float mo[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int64_t r = r0 + (int64_t)q * kWaves * rpw + sub;
+            const int64_t rl = r < r_end ? r : r_end - 1;
+            load_raw8_any<DT>(g + rl * C + cl, gr[q]);
+            ir[q] = load_raw_idx8_any(idxp + rl * C + cl);
+            const int64_t e = rl * C + (nv > 0 ? c : 0);
+            bb[q] = div_floor(e, P, invP);
+            pp[q] = e - bb[q] * P;
+            mo[q] = *gbl(mag_old + bb[q]);
+        }
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            const int64_t r = r0 + (int64_t)q * kWaves * rpw + sub;
+            if (r - sub >= r_end) break;
+            if (cut) shift_down<DT>(gr[q], ir[q], sh);
+            const int n = r < r_end ? nv : 0;
+            Acc rs = 0;
+            uint32_t m = 0u;
+            int64_t key = n > 0 ? bb[q] : -1;
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {
+                if (k < n) {
+                    const float gv = raw_elem<DT>(gr[q], k);
+                    const float uu = momentum_value<LF>(s_cbr[raw_idx(ir[q], k)], mo[q], gv, mc);
+                    const uint32_t ub = __float_as_uint(uu) & 0x7fffffffu;
+                    m = ub > m ? ub : m;
+                    sq_add(rs, gv);
+                    sq_add(colf[k], gv);
+                    if (++pp[q] == P && k + 1 < n) {
+                        if (m) gatomic_max(mb + key, m);
+                        m = 0u;
+                        pp[q] = 0;
+                        ++key;
+                        mo[q] = *gbl(mag_old + key);
+                    }
+                }
+            }
+            wave_block_max(mb, key, m);
+            double rsum = (double)rs;
+            for (int o = 1; o < L; o <<= 1) rsum += __shfl_xor(rsum, o, 64);
+            if ((lane & (L - 1)) == 0 && r < r_end) *gbl(wr.row_part + r) = rsum;
+            if (++nf == 8) {
+                nf = 0;
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k) { cold[k] += (double)colf[k]; colf[k] = 0; }
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kChunk; ++k) lds.col[wave][k][0][lane] = cold[k] + (double)colf[k];
+    __syncthreads();
+    if (threadIdx.x < C) {  // C <= kNarrowMaxCols = the workgroup's threads
+        const int j = threadIdx.x / kChunk, k = threadIdx.x % kChunk;
+        double sum = 0.0;
+        for (int ww = 0; ww < kWaves; ++ww)
+            for (int s = 0; s < rpw; ++s) sum += lds.col[ww][k][0][s * L + j];
+        *gbl(wr.col_part + wg * C + threadIdx.x) = sum;
+    }
+}
+static_assert(kNarrowMaxCols <= kThreads, "stats_narrow: one thread per column at the end");
 
 // ====================================================================
 // Transposed views: g (and p) with strides (1, ld), ld >= R -- the layout of
@@ -1841,6 +1971,13 @@ __device__ __forceinline__ int64_t xcd_contiguous(int64_t b, int64_t G) {
 template <int DT, bool FAST>
 __device__ __forceinline__ void stats_factored_wg(const TensorWork& w, int64_t wg) {
     __shared__ FactStatsLds lds;
+    if constexpr (FAST) {
+        if (w.lg_lanes >= 0) {
+            if (w.mc.small) stats_narrow<DT, kLerpSmall>(w, wg, lds);
+            else stats_narrow<DT, kLerpLarge>(w, wg, lds);
+            return;
+        }
+    }
     if (w.mc.small) stats_factored<DT, FAST, kLerpSmall>(w, wg, lds);
     else stats_factored<DT, FAST, kLerpLarge>(w, wg, lds);
 }
@@ -1875,7 +2012,7 @@ __global__ void __launch_bounds__(kThreads) k_apply(TensorWork w) {
 // Factored stats of a launch group; the group's block-path tensors of the
 // same dtype (not transposed views) ride in the same launch.
 template <int DT, bool FAST>
-__global__ void __launch_bounds__(kThreads) k_mt_factored_stats(const TensorWork* __restrict__ ws,
+__global__ void __launch_bounds__(kThreads, FAST && DT != F32 ? 4 : 2) k_mt_factored_stats(const TensorWork* __restrict__ ws,
                                                                 SegTable tb) {
     const Seg sg = find_seg(tb, blockIdx.x);
     const TensorWork& w = ws[sg.t];

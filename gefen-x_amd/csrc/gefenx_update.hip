@@ -348,7 +348,12 @@ static int build_work(const WorkInput& in, TensorWork& w) {
         w.nbw = std::max<int64_t>(1, std::min<int64_t>(1024, ceil_div(nb, kFinBlocksPerWg)));
         const bool contig_g = (in.gs1 == 1 && in.gs0 == in.C);
         const bool contig_p = (in.ps1 == 1 && in.ps0 == in.C);
-        w.fast_stats = contig_g && (in.C % kChunk == 0) && aligned(in.grad, 16) && aligned(in.idx, 8);
+        w.fast_stats = contig_g && in.C >= kChunk;
+        w.lg_lanes = -1;
+        if (w.fast_stats && in.C <= kNarrowMaxCols) {
+            w.lg_lanes = 0;
+            while ((1 << w.lg_lanes) < narrow_lanes(in.C)) ++w.lg_lanes;
+        }
         w.fast_apply = contig_g && contig_p && (in.C % kChunk == 0) && (in.period % kChunk == 0) &&
                        aligned(in.grad, 16) && aligned(in.p, 16) && aligned(in.idx, 8) && aligned(in.v1, 16);
         if (!w.fast_stats && tv_shape && tv_g) {

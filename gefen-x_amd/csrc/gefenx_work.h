@@ -67,6 +67,7 @@ struct TensorWork {
     int32_t row_apply;   // factored contiguous apply over row segments (apply_rows)
     int32_t partial;     // block path with the caller's per-block stepsize (no vmean)
     int32_t fin_wide;    // block finalize: one workgroup per block (blocks span many stats records)
+    int32_t lg_lanes;    // factored contiguous stats of few columns: log2 lanes per row (stats_narrow), else -1
     int32_t csplit;      // factored finalize: threads per column (1, 2, 4 or 8), each over a run of row tiles
     float eps, beta2, alpha2;
     float bc2_div;       // reference-order divisor (factored bc2, block sqrt(bc2)) or 0

@@ -35,6 +35,23 @@ CASES = [
     ((256, 64), 64, BF16, "t", {}),
     ((264, 1096), 1096, BF16, "t", {}),
     ((1000, 200), 1600, F16, "t", {"factored": False}),
+    # contiguous stats of any width: chunks cut by the last column, blocks that
+    # end inside a chunk, storage that starts between vectors
+    ((70, 1025), 1025, BF16, "c", {}),
+    ((64, 1539), 3, F16, "c", {}),
+    ((65, 771), 771 * 5, F32, "c", {}),
+    ((40, 1031), 1031 * 4, BF16, "o", {}),
+    ((96, 1024), 24, BF16, "o", {}),
+    ((129, 520), 8, F32, "c", {}),
+    # narrow: 1 to 32 lanes per row, a cut chunk, several tiles
+    ((9, 8), 8, F32, "c", {}),
+    ((3000, 16), 48, BF16, "c", {}),
+    ((1025, 13), 65, F16, "c", {}),
+    ((515, 250), 250, BF16, "o", {}),
+    ((4099, 33), 4099, BF16, "c", {}),
+    ((300, 256), 300 * 256, F32, "c", {}),
+    # fewer than 8 columns: element loads
+    ((500, 7), 35, BF16, "c", {}),
 ]
 
 
