@@ -61,13 +61,15 @@ constexpr int64_t kFactTileMaxElems = 1 << 20;
 constexpr int64_t kFactTileSmallElems = 1 << 14;
 constexpr int64_t kFactLaunchWgs = 1024;
 
-// Contiguous matrices of 8 to 256 columns: a wave takes several rows at a
-// time (stats_narrow), a power of two of lanes for each.  Lanes per row for `cols`:
+// Contiguous matrices (C >= 8) of at most kNarrowMaxCols columns, or with
+// blocks shorter than kShortPeriod, take tiles of up to kLaneTileCols columns
+// (stats_lanes): with few columns a 1024-column tile leaves lanes idle, and
+// with short blocks nearly every 1024-column row segment holds block borders.
 constexpr int64_t kNarrowMaxCols = 256;
-inline int narrow_lanes(int64_t cols) {
-    int l = 1;
-    while (8 * l < cols) l *= 2;
-    return l;
+constexpr int64_t kShortPeriod = 1024;
+constexpr int64_t kLaneTileCols = 512;
+inline bool lane_tiles(int64_t cols, int64_t period) {
+    return cols >= 8 && (cols <= kNarrowMaxCols || (period < kShortPeriod && period < cols));
 }
 
 // As launch_elems: the largest tiles whatever the launch.
@@ -82,37 +84,45 @@ constexpr int64_t kCoarseTiles = (int64_t)1 << 62;
 constexpr int64_t kTvStatsMaxRows = 256;
 
 struct FactTiles {
-    int64_t ct, rt, tile_rows;
-    int64_t ct_tv, tv_cols, rt_tv, tv_rows;  // tiles of the transposed-view stats kernel
+    int64_t ct, rt, tile_rows;                            // 1024-column tiles
+    int64_t ct_l, rt_l, l_rows, l_cols, lg_lanes;         // lane tiles (lg_lanes: log2 lanes per row; -1: not taken)
+    int64_t ct_tv, rt_tv, tv_rows, tv_cols;               // transposed-view tiles
     // launch_elems: elements of all tensors of the launch (>= rows * cols)
-    static FactTiles make(int64_t rows, int64_t cols, int64_t launch_elems) {
+    static FactTiles make(int64_t rows, int64_t cols, int64_t period, int64_t launch_elems) {
         FactTiles t;
-        t.ct = (cols + kFactTileCols - 1) / kFactTileCols;
-        if (t.ct < 1) t.ct = 1;
-        const int64_t tc = cols < kFactTileCols ? (cols < 1 ? 1 : cols) : kFactTileCols;
+        const auto ceil_div = [](int64_t x, int64_t d) { return x > 0 ? (x + d - 1) / d : 1; };
         int64_t elems = rows * cols / 32;
         elems = elems < kFactTileMinElems ? kFactTileMinElems : (elems > kFactTileMaxElems ? kFactTileMaxElems : elems);
         int64_t share = launch_elems / kFactLaunchWgs;
         if (share < kFactTileSmallElems) share = kFactTileSmallElems;
         if (elems > share) elems = share;
-        int64_t tr = (elems + tc - 1) / tc;
-        // whole 8-row fp32 column groups of each of the 4 waves (narrow: of each lane)
-        const int64_t gran = cols >= 8 && cols <= kNarrowMaxCols ? 32 * (64 / narrow_lanes(cols)) : 32;
-        tr = (tr + gran - 1) / gran * gran;
-        if (tr > rows) tr = rows;
-        if (tr < 1) tr = 1;
-        t.tile_rows = tr;
-        t.rt = (rows + tr - 1) / tr;
-        if (t.rt < 1) t.rt = 1;
-        int64_t tv = kTvStatsMaxRows;
-        if (tv > rows) tv = rows < 1 ? 1 : rows;
-        t.tv_rows = tv;
-        t.rt_tv = (rows + tv - 1) / tv;
-        if (t.rt_tv < 1) t.rt_tv = 1;
-        int64_t vc = (share / (2 * kTvStatsMaxRows) + 63) & ~int64_t(63);
+        // rows of a tile of `width` columns: whole 8-row fp32 column groups of
+        // each wave (lane tiles: of each lane), `gran` rows together
+        const auto tile_rows = [&](int64_t width, int64_t gran) {
+            const int64_t w = cols < width ? (cols < 1 ? 1 : cols) : width;
+            int64_t r = ceil_div(ceil_div(elems, w), gran) * gran;
+            if (r > rows) r = rows;
+            return r < 1 ? 1 : r;
+        };
+        t.ct = ceil_div(cols, kFactTileCols);
+        t.tile_rows = tile_rows(kFactTileCols, 32);
+        t.rt = ceil_div(rows, t.tile_rows);
+        t.lg_lanes = -1;
+        t.ct_l = t.rt_l = 0;
+        t.l_rows = t.l_cols = 0;
+        if (lane_tiles(cols, period)) {
+            t.l_cols = (ceil_div(cols, ceil_div(cols, kLaneTileCols)) + 7) & ~int64_t(7);  // even column tiles
+            t.lg_lanes = 0;
+            while ((8 << t.lg_lanes) < t.l_cols) ++t.lg_lanes;
+            t.ct_l = ceil_div(cols, t.l_cols);
+            t.l_rows = tile_rows(t.l_cols, 32 * (64 >> t.lg_lanes));
+            t.rt_l = ceil_div(rows, t.l_rows);
+        }
+        t.tv_rows = rows < 1 ? 1 : (rows < kTvStatsMaxRows ? rows : kTvStatsMaxRows);
+        t.rt_tv = ceil_div(rows, t.tv_rows);
+        const int64_t vc = (share / (2 * kTvStatsMaxRows) + 63) & ~int64_t(63);
         t.tv_cols = vc < 64 ? 64 : vc > kFactTileCols ? kFactTileCols : vc;
-        t.ct_tv = (cols + t.tv_cols - 1) / t.tv_cols;
-        if (t.ct_tv < 1) t.ct_tv = 1;
+        t.ct_tv = ceil_div(cols, t.tv_cols);
         return t;
     }
 };
@@ -130,7 +140,7 @@ inline int64_t mag_shards(int64_t nb) { return nb <= kMagShardMaxBlocks ? kMagSh
 constexpr int64_t kFinRowsPerWg = 256;
 
 struct FactoredWs {
-    // double row_part[max(ct, ct_tv)][rows], double col_part[max(rt, rt_tv)][cols] (per-tile
+    // double row_part[max of the tilings' ct][rows], double col_part[max rt][cols] (per-tile
     // partial sums, fully rewritten every step; launch_elems = rows * cols sizes them for the
     // smallest tiles, so one workspace serves the tensor in every launch), uint32 magbits[shards][nb] (zero
     // between steps), float mag_old[nb], float minv[nb],
@@ -139,11 +149,12 @@ struct FactoredWs {
     size_t off_rowp, off_colp, off_magbits, off_magold, off_minv, off_vsum, off_vcs, off_fin, total;
     static FactoredWs make(int64_t rows, int64_t cols, int64_t nb, int64_t launch_elems) {
         FactoredWs w;
-        const FactTiles t = FactTiles::make(rows, cols, launch_elems);
+        const FactTiles t = FactTiles::make(rows, cols, nb > 0 ? rows * cols / nb : 1, launch_elems);
         size_t o = 0;
-        const int64_t ct = t.ct > t.ct_tv ? t.ct : t.ct_tv;  // either stats layout fits
+        // any of the three tilings fits
+        const auto max3 = [](int64_t x, int64_t y, int64_t z) { return x > y ? (x > z ? x : z) : (y > z ? y : z); };
+        const int64_t ct = max3(t.ct, t.ct_l, t.ct_tv), rt = max3(t.rt, t.rt_l, t.rt_tv);
         w.off_rowp = o;    o += align256(sizeof(double) * (size_t)(ct * rows));
-        const int64_t rt = t.rt > t.rt_tv ? t.rt : t.rt_tv;
         w.off_colp = o;    o += align256(sizeof(double) * (size_t)(rt * cols));
         w.off_magbits = o; o += align256(sizeof(uint32_t) * (size_t)(nb * mag_shards(nb)));
         w.off_magold = o;  o += align256(sizeof(float) * (size_t)nb);

@@ -472,11 +472,11 @@ __device__ __forceinline__ uint32_t wave_max_u63(uint32_t v) {
 // suffix sum / max: each lane ends with the sum (max) of its run from itself
 // to the run's last lane, so a run's first lane holds the run's total.
 __device__ __forceinline__ uint64_t run_heads(int64_t key) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t lo = (uint32_t)__shfl_up((int)(uint32_t)key, 1, 64);
-    const uint32_t hi = (uint32_t)__shfl_up((int)(uint32_t)((uint64_t)key >> 32), 1, 64);
+    // wave_shr:1 (lane l reads lane l - 1)
+    const uint32_t lo = dpp32<0x138, 0xf>((uint32_t)key);
+    const uint32_t hi = dpp32<0x138, 0xf>((uint32_t)((uint64_t)key >> 32));
     const int64_t prev = (int64_t)(((uint64_t)hi << 32) | lo);
-    return (uint64_t)__ballot(lane == 0 || prev != key);
+    return (uint64_t)__ballot((threadIdx.x & 63) == 0 || prev != key);
 }
 
 __device__ __forceinline__ double seg_suffix_sum(double v, uint64_t heads) {
@@ -491,14 +491,26 @@ __device__ __forceinline__ double seg_suffix_sum(double v, uint64_t heads) {
     return v;
 }
 
+// Inside a row of 16 lanes through DPP row shifts (no LDS traffic), then the
+// three row borders with scalars: a run that reaches past its row takes the
+// next row's first lane.
 __device__ __forceinline__ uint32_t seg_suffix_max(uint32_t m, uint64_t heads) {
     const int lane = threadIdx.x & 63;
     const uint64_t after = lane < 63 ? heads >> (lane + 1) : 0ull;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        const uint32_t o = (uint32_t)__shfl_down((int)m, d, 64);
-        const bool ok = lane + d < 64 && (after & ((1ull << d) - 1ull)) == 0ull;
+    const uint32_t in_row = 15u - (uint32_t)(lane & 15);  // lanes after this one in its row
+    auto step = [&](uint32_t o, uint32_t d) {
+        const bool ok = d <= in_row && ((uint32_t)after & ((1u << d) - 1u)) == 0u;
         m = (ok && o > m) ? o : m;
+    };
+    step(dpp32<0x101, 0xf>(m), 1);  // row_shl:d (lane l reads lane l + d)
+    step(dpp32<0x102, 0xf>(m), 2);
+    step(dpp32<0x104, 0xf>(m), 4);
+    step(dpp32<0x108, 0xf>(m), 8);
+#pragma unroll
+    for (int row = 3; row >= 1; --row) {  // last border first: a row's first lane then covers the rows after it
+        const uint32_t s = (uint32_t)__builtin_amdgcn_readlane((int)m, 16 * row);
+        const bool mine = (lane >> 4) == row - 1 && ((uint32_t)after & ((2u << in_row) - 1u)) == 0u;
+        m = (mine && s > m) ? s : m;
     }
     return m;
 }

@@ -405,17 +405,21 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
 }
 
 // ====================================================================
-// Factored stats of a contiguous matrix of 8 to kNarrowMaxCols columns, any
-// alignment and P.  L lanes (a power of two, 8 columns each) take a row, a wave
-// 64 / L rows at a time, four such steps in flight; the workgroup covers
-// tile_rows rows of all columns.  A row's lanes add up its sum of squares, a
-// lane keeps its columns' sums (fp32 over 8 rows, then float64), the lanes of
-// one column meet in LDS at the end in a fixed order.  stats_factored would
-// leave all but C / 16 of a wave's lanes idle and walk the rows one by one: a
-// set of 16-column and 16-row fp32 adapters 246 -> 16 us.
+// Factored stats with per-lane blocks, for contiguous matrices (C >= 8, any
+// alignment and P) of at most kNarrowMaxCols columns or of short blocks.  The
+// workgroup covers tile_rows rows of tile_cols <= 512 columns; L lanes (a
+// power of two, 8 columns each) take a row of the tile, a wave 64 / L rows at a
+// time, four such steps in flight, each lane's old magnitude loaded with its
+// chunk.  A row's lanes add up its sum of squares, a lane keeps its columns'
+// sums (fp32 over 8 rows, then float64), the lanes of one column meet in LDS
+// at the end in a fixed order.  stats_factored would leave all but C / 16 of a
+// wave's lanes idle on few columns and walk the rows one by one (a set of
+// 16-column and 16-row fp32 adapters 246 -> 16 us), and would wait for the
+// magnitudes of every row whose blocks end inside it (7.5M bf16 elements with
+// 256-element blocks 40 -> 21 us).
 // ====================================================================
 template <int DT, int LF>
-__device__ __forceinline__ void stats_narrow(const TensorWork& wr, int64_t wg, FactStatsLds& lds) {
+__device__ __forceinline__ void stats_lanes(const TensorWork& wr, int64_t wg, FactStatsLds& lds) {
     using T = typename Elem<DT>::T;
     using Acc = std::conditional_t<DT == F32, double, float>;
     constexpr int Q = 4;  // steps in flight
@@ -431,12 +435,16 @@ __device__ __forceinline__ void stats_narrow(const TensorWork& wr, int64_t wg, F
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lgL = wr.lg_lanes, L = 1 << lgL, rpw = 64 >> lgL;
-    const int sub = lane >> lgL, c = (lane & (L - 1)) * kChunk;
-    const int nv = (int)std::max<int64_t>(0, std::min<int64_t>(kChunk, C - c));
-    const int64_t cl = nv == kChunk ? c : C - kChunk;  // a lane past C or cut by it reads the row's last 8
+    const int64_t ct = wr.ct, ctile = wg % ct, rtile = wg / ct;
+    const int64_t tc0 = ctile * wr.tile_cols;
+    const int span = (int)std::min<int64_t>(wr.tile_cols, C - tc0);
+    const int sub = lane >> lgL;
+    const int64_t c = tc0 + (lane & (L - 1)) * kChunk;
+    const int nv = (int)std::max<int64_t>(0, std::min<int64_t>(kChunk, tc0 + span - c));
+    const int64_t cl = nv == kChunk ? c : tc0 + span - kChunk;  // a lane past the tile or cut by it: its last 8
     const int sh = (kChunk - nv) & 7;
-    const bool cut = (C & 7) != 0;
-    const int64_t r_begin = wg * wr.tile_rows;
+    const bool cut = (span & 7) != 0;
+    const int64_t r_begin = rtile * wr.tile_rows;
     const int64_t r_end = std::min<int64_t>(r_begin + wr.tile_rows, R);
     __syncthreads();
     Acc colf[kChunk];
@@ -455,7 +463,7 @@ __device__ __forceinline__ void stats_narrow(const TensorWork& wr, int64_t wg, F
             const int64_t rl = r < r_end ? r : r_end - 1;
             load_raw8_any<DT>(g + rl * C + cl, gr[q]);
             ir[q] = load_raw_idx8_any(idxp + rl * C + cl);
-            const int64_t e = rl * C + (nv > 0 ? c : 0);
+            const int64_t e = rl * C + (nv > 0 ? c : cl);
             bb[q] = div_floor(e, P, invP);
             pp[q] = e - bb[q] * P;
             mo[q] = *gbl(mag_old + bb[q]);
@@ -489,8 +497,13 @@ __device__ __forceinline__ void stats_narrow(const TensorWork& wr, int64_t wg, F
             }
             wave_block_max(mb, key, m);
             double rsum = (double)rs;
-            for (int o = 1; o < L; o <<= 1) rsum += __shfl_xor(rsum, o, 64);
-            if ((lane & (L - 1)) == 0 && r < r_end) *gbl(wr.row_part + r) = rsum;
+            if (lgL > 0) rsum += dpp64<0xB1, 0xf>(rsum);   // lane ^ 1
+            if (lgL > 1) rsum += dpp64<0x4E, 0xf>(rsum);   // lane ^ 2
+            if (lgL > 2) rsum += dpp64<0x141, 0xf>(rsum);  // the other half of 8
+            if (lgL > 3) rsum += dpp64<0x140, 0xf>(rsum);  // the other half of 16
+            if (lgL > 4) rsum += __shfl_xor(rsum, 16, 64);
+            if (lgL > 5) rsum += __shfl_xor(rsum, 32, 64);
+            if ((lane & (L - 1)) == 0 && r < r_end) *gbl(wr.row_part + ctile * R + r) = rsum;
             if (++nf == 8) {
                 nf = 0;
 #pragma unroll
@@ -501,15 +514,14 @@ __device__ __forceinline__ void stats_narrow(const TensorWork& wr, int64_t wg, F
 #pragma unroll
     for (int k = 0; k < kChunk; ++k) lds.col[wave][k][0][lane] = cold[k] + (double)colf[k];
     __syncthreads();
-    if (threadIdx.x < C) {  // C <= kNarrowMaxCols = the workgroup's threads
-        const int j = threadIdx.x / kChunk, k = threadIdx.x % kChunk;
+    for (int col = threadIdx.x; col < span; col += kThreads) {
+        const int j = col / kChunk, k = col % kChunk;
         double sum = 0.0;
         for (int ww = 0; ww < kWaves; ++ww)
             for (int s = 0; s < rpw; ++s) sum += lds.col[ww][k][0][s * L + j];
-        *gbl(wr.col_part + wg * C + threadIdx.x) = sum;
+        *gbl(wr.col_part + rtile * C + tc0 + col) = sum;
     }
 }
-static_assert(kNarrowMaxCols <= kThreads, "stats_narrow: one thread per column at the end");
 
 // ====================================================================
 // Transposed views: g (and p) with strides (1, ld), ld >= R -- the layout of
@@ -1973,8 +1985,8 @@ __device__ __forceinline__ void stats_factored_wg(const TensorWork& w, int64_t w
     __shared__ FactStatsLds lds;
     if constexpr (FAST) {
         if (w.lg_lanes >= 0) {
-            if (w.mc.small) stats_narrow<DT, kLerpSmall>(w, wg, lds);
-            else stats_narrow<DT, kLerpLarge>(w, wg, lds);
+            if (w.mc.small) stats_lanes<DT, kLerpSmall>(w, wg, lds);
+            else stats_lanes<DT, kLerpLarge>(w, wg, lds);
             return;
         }
     }

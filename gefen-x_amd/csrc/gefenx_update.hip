@@ -333,7 +333,7 @@ static int build_work(const WorkInput& in, TensorWork& w) {
         const FactoredWs L = FactoredWs::make(in.R, in.C, nb, in.ws_elems);
         if (in.ws_bytes < L.total)
             return set_error(GEFENX_EINVAL, "factored update: workspace %zu bytes < required %zu", in.ws_bytes, L.total);
-        const FactTiles t = FactTiles::make(in.R, in.C, in.launch_elems);
+        const FactTiles t = FactTiles::make(in.R, in.C, in.period, in.launch_elems);
         w.row_part = reinterpret_cast<double*>(ws + L.off_rowp);
         w.col_part = reinterpret_cast<double*>(ws + L.off_colp);
         w.magbits = reinterpret_cast<uint32_t*>(ws + L.off_magbits);
@@ -349,10 +349,10 @@ static int build_work(const WorkInput& in, TensorWork& w) {
         const bool contig_g = (in.gs1 == 1 && in.gs0 == in.C);
         const bool contig_p = (in.ps1 == 1 && in.ps0 == in.C);
         w.fast_stats = contig_g && in.C >= kChunk;
-        w.lg_lanes = -1;
-        if (w.fast_stats && in.C <= kNarrowMaxCols) {
-            w.lg_lanes = 0;
-            while ((1 << w.lg_lanes) < narrow_lanes(in.C)) ++w.lg_lanes;
+        w.lg_lanes = w.fast_stats ? (int32_t)t.lg_lanes : -1;
+        if (w.lg_lanes >= 0) {
+            w.ct = t.ct_l; w.rt = t.rt_l; w.tile_rows = t.l_rows; w.tile_cols = t.l_cols;
+            w.stats_wgs = t.ct_l * t.rt_l;
         }
         w.fast_apply = contig_g && contig_p && (in.C % kChunk == 0) && (in.period % kChunk == 0) &&
                        aligned(in.grad, 16) && aligned(in.p, 16) && aligned(in.idx, 8) && aligned(in.v1, 16);
@@ -405,7 +405,7 @@ static int build_work(const WorkInput& in, TensorWork& w) {
             const bool g_contig = in.gs1 == 1 && in.gs0 == in.C;
             const bool p_contig = in.ps1 == 1 && in.ps0 == in.C;
             if (tv_shape && tv_g) {
-                const FactTiles t = FactTiles::make(in.R, in.C, in.launch_elems);
+                const FactTiles t = FactTiles::make(in.R, in.C, in.period, in.launch_elems);
                 w.ct = t.ct_tv; w.rt = t.rt_tv; w.tile_rows = t.tv_rows; w.tile_cols = t.tv_cols;
                 w.stats_wgs = t.ct_tv * t.rt_tv;
                 w.fast_stats = 2;

@@ -54,7 +54,7 @@ struct TensorWork {
     int64_t R, C, N, P, nb;
     double invC, invP;
     int64_t ps0, ps1, gs0, gs1;
-    int64_t ct, rt, tile_rows, tile_cols, shards;  // tile_cols: transposed-view stats
+    int64_t ct, rt, tile_rows, tile_cols, shards;  // tile_cols: lane tiles and transposed views
     int64_t stats_wgs, nr, nc, nbw, fin_wgs, apply_wgs;
     int64_t det_elems;   // block stats: elements per workgroup
     int64_t dR, dC, dB, dP;  // apply: chunk advance for a stride of apply_wgs*256*8 elements
@@ -67,7 +67,7 @@ struct TensorWork {
     int32_t row_apply;   // factored contiguous apply over row segments (apply_rows)
     int32_t partial;     // block path with the caller's per-block stepsize (no vmean)
     int32_t fin_wide;    // block finalize: one workgroup per block (blocks span many stats records)
-    int32_t lg_lanes;    // factored contiguous stats of few columns: log2 lanes per row (stats_narrow), else -1
+    int32_t lg_lanes;    // factored contiguous stats on lane tiles: log2 lanes per row (stats_lanes), else -1
     int32_t csplit;      // factored finalize: threads per column (1, 2, 4 or 8), each over a run of row tiles
     float eps, beta2, alpha2;
     float bc2_div;       // reference-order divisor (factored bc2, block sqrt(bc2)) or 0

@@ -43,13 +43,19 @@ CASES = [
     ((40, 1031), 1031 * 4, BF16, "o", {}),
     ((96, 1024), 24, BF16, "o", {}),
     ((129, 520), 8, F32, "c", {}),
-    # narrow: 1 to 32 lanes per row, a cut chunk, several tiles
+    # lane tiles: 1 to 64 lanes per row, a cut chunk, several tiles, blocks of
+    # any length in a wave
     ((9, 8), 8, F32, "c", {}),
     ((3000, 16), 48, BF16, "c", {}),
     ((1025, 13), 65, F16, "c", {}),
     ((515, 250), 250, BF16, "o", {}),
     ((4099, 33), 4099, BF16, "c", {}),
     ((300, 256), 300 * 256, F32, "c", {}),
+    ((70, 1100), 100, BF16, "c", {}),
+    ((96, 1031), 96, F16, "c", {}),
+    ((64, 512), 8, BF16, "c", {}),
+    ((66, 2048), 1, F32, "c", {}),
+    ((48, 600), 72, BF16, "t", {}),
     # fewer than 8 columns: element loads
     ((500, 7), 35, BF16, "c", {}),
 ]
