@@ -216,6 +216,23 @@ __device__ __forceinline__ void load_raw8_any(const typename Elem<DT>::T* __rest
     }
 }
 
+template <int DT>
+__device__ __forceinline__ void store8_any(typename Elem<DT>::T* __restrict__ base, const float v[8]) {
+    if constexpr (DT == F32) {
+        GX_GLOBAL f32x4_a4* q = gbl(reinterpret_cast<f32x4_a4*>(base));
+        const f32x4 a = {v[0], v[1], v[2], v[3]}, b = {v[4], v[5], v[6], v[7]};
+        __builtin_nontemporal_store(a, q);
+        __builtin_nontemporal_store(b, q + 1);
+    } else {
+        uint32_t w[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            w[i] = (uint32_t)from_f32<DT>(v[2 * i]) | ((uint32_t)from_f32<DT>(v[2 * i + 1]) << 16);
+        const u32x4 a = {w[0], w[1], w[2], w[3]};
+        __builtin_nontemporal_store(a, gbl(reinterpret_cast<u32x4_a2*>(base)));
+    }
+}
+
 struct RawIdx8 { uint32_t lo, hi; };
 
 __device__ __forceinline__ RawIdx8 load_raw_idx8(const uint8_t* __restrict__ base) {
@@ -237,6 +254,13 @@ typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
 __device__ __forceinline__ RawIdx8 load_raw_idx8_any(const uint8_t* __restrict__ base) {
     const u32x2 v = __builtin_nontemporal_load(gbl(reinterpret_cast<const u32x2_a1*>(base)));
     return RawIdx8{v.x, v.y};
+}
+
+__device__ __forceinline__ void store_idx8_any(uint8_t* __restrict__ base, const uint32_t ix[8]) {
+    u32x2 a;
+    a.x = ix[0] | (ix[1] << 8) | (ix[2] << 16) | (ix[3] << 24);
+    a.y = ix[4] | (ix[5] << 8) | (ix[6] << 16) | (ix[7] << 24);
+    __builtin_nontemporal_store(a, gbl(reinterpret_cast<u32x2_a1*>(base)));
 }
 
 __device__ __forceinline__ RawIdx8 load_raw_idx8_elems(const uint8_t* __restrict__ base) {
@@ -555,22 +579,6 @@ __device__ __forceinline__ void stage_tables(SharedTables& s, const QTable* __re
         s.thr[kCodebookMax + tid] = __builtin_inff();
         s.bkt[kBuckets + tid] = t->bucket[kBuckets - 1];
     }
-}
-
-// Nearest index for x in [-1, 1] (never NaN).  Thresholds in later buckets
-// are > x, so the first two slots from the bucket's base can be compared
-// unconditionally; buckets holding more than two thresholds (`dense` tables
-// only) continue with the remaining ones.
-__device__ __forceinline__ uint32_t quant_fast(float x, const SharedTables& s, bool dense) {
-    const int b = (int)__builtin_fmaf(x, (float)(kBuckets / 2), (float)(kBuckets / 2));
-    const uint32_t e = s.bkt[b];
-    const uint32_t base = e & 0xffffu;
-    uint32_t idx = base + (s.thr[base] < x ? 1u : 0u) + (s.thr[base + 1] < x ? 1u : 0u);
-    if (dense) {
-        const uint32_t cnt = e >> 16;
-        for (uint32_t j = 2; j < cnt; ++j) idx += (s.thr[base + j] < x) ? 1u : 0u;
-    }
-    return idx;
 }
 
 struct SharedSR {

@@ -1133,30 +1133,19 @@ __device__ __forceinline__ void stats_block_wg(const TensorWork& w, int64_t wg) 
 }
 
 // ====================================================================
-// Apply: grid-stride over logical chunks of 8 elements with nwg workgroups.
-// MODE 0 factored, MODE 1 block.  FAST: contiguous p/grad, C % 8 == 0,
-// P % 8 == 0, aligned -- a chunk then never crosses a row or a block, and
-// (row, col, blk, pin) advance by constant strides (no per-chunk division).
+// General apply: any strides, C and P; grid-stride over logical chunks of 8
+// elements with nwg workgroups, element loads and stores.
+// MODE 0 factored, MODE 1 block.
 // ====================================================================
-struct Pos {
-    int64_t row, col, blk, pin;
-};
-
-template <int MODE>
-__device__ __forceinline__ Pos advance(const TensorWork& w, Pos q) {
-    if constexpr (MODE == 0) {
-        q.col += w.dC;
-        q.row += w.dR;
-        if (q.col >= w.C) { q.col -= w.C; ++q.row; }
-    }
-    q.pin += w.dP;
-    q.blk += w.dB;
-    if (q.pin >= w.P) { q.pin -= w.P; ++q.blk; }
-    return q;
-}
-
 __device__ __forceinline__ void load_vcol(const float* __restrict__ vc, float v[8]) {
     const GX_GLOBAL f32x4* q = gbl(reinterpret_cast<const f32x4*>(vc));
+    const f32x4 v0 = q[0], v1 = q[1];
+    v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
+    v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
+}
+
+__device__ __forceinline__ void load_vcol_any(const float* __restrict__ vc, float v[8]) {
+    const GX_GLOBAL f32x4_a4* q = gbl(reinterpret_cast<const f32x4_a4*>(vc));
     const f32x4 v0 = q[0], v1 = q[1];
     v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
     v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
@@ -1168,81 +1157,12 @@ struct ApplyCtx {
     RefStep ref;      // fp32 factored: the reference-order stepsize
     bool wd;
     StepScalars sc;
-    bool dense;
     uint32_t kmax;
     int kk;
     uint64_t seed;
 };
 
-// One chunk of 8 elements sharing a row and a block (fast path).  u / m_new
-// goes through the block reciprocal (div_by_block's Markstein step) in every
-// lane; a wave where any lane is outside that step's safe range (tiny |u|;
-// zero, subnormal, huge, inf or NaN magnitude) redoes the chunk with the
-// fully guarded helpers.
 template <int DT, int MODE, bool SR>
-__device__ __forceinline__ void apply_chunk(const TensorWork& w, const SharedTables& st,
-                                            const SharedSR& ssr, const ApplyCtx& cx, int64_t e0,
-                                            const Pos& ps, const Raw8<DT>& gr, const Raw8<DT>& pr,
-                                            const RawIdx8& ir, const float vcv[kChunk],
-                                            uint32_t ix[kChunk], float pv[kChunk]) {
-    const float m_old = w.mag_old[ps.blk];
-    const float m_new = w.mag[ps.blk];
-    const float y = w.minv[ps.blk];
-    const float tb = 0x1.00001p-100f * fmaxf(m_new, 1.0f);
-    float xs[kChunk];
-    bool bad = (y == 0.0f);
-#pragma unroll
-    for (int k = 0; k < kChunk; ++k) {
-        const float u = momentum_value(st.cbr[raw_idx(ir, k)], m_old, raw_elem<DT>(gr, k), w.mc);
-        const float q0 = u * y;
-        const float r = __builtin_fmaf(-q0, m_new, u);
-        xs[k] = __builtin_fmaf(r, y, q0);
-        bad = bad || !(fabsf(u) >= tb);
-    }
-    if (__any(bad)) {
-        const bool nz = m_new > 0.0f;
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            const float u = momentum_value(st.cbr[raw_idx(ir, k)], m_old, raw_elem<DT>(gr, k), w.mc);
-            const float x = nz ? div_by_block(u, m_new, y) : 0.0f;
-            if constexpr (SR) ix[k] = quant_stochastic(x, ssr.cb, ssr.lut, cx.kk, cx.seed, e0 + k);
-            else ix[k] = quant_nearest(x, st.bkt, st.thr, cx.kmax);
-        }
-    } else {
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            if constexpr (SR) ix[k] = quant_stochastic(xs[k], ssr.cb, ssr.lut, cx.kk, cx.seed, e0 + k);
-            else ix[k] = quant_fast(xs[k], st, cx.dense);
-        }
-    }
-    if (w.write_p) {
-        float rs = 0.0f, bstep = 0.0f, vr = 0.0f;
-        if constexpr (MODE == 0) {
-            vr = w.v0[ps.row];
-            rs = vr * cx.row_scale;
-        } else {
-            bstep = w.step[ps.blk];
-        }
-#pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            const float q = st.cbr[ix[k]] * m_new;
-            float pw = raw_elem<DT>(pr, k);
-            if (cx.wd) pw = round_dt<DT>(pw * cx.sc.wdf);
-            if constexpr (MODE == 0) {
-                if (DT == F32 && cx.ref.on) {
-                    pv[k] = pw - (q * ref_step(cx.ref, vr, vcv[k])) * cx.sc.lr;
-                } else {
-                    const float h = __builtin_amdgcn_sqrtf(rs * vcv[k]) + w.eps;
-                    pv[k] = pw - q * (__builtin_amdgcn_rcpf(h) * cx.c1);
-                }
-            } else {
-                pv[k] = pw - (q * bstep) * cx.sc.lr;  // the reference's order (gefen.py:3806-3818)
-            }
-        }
-    }
-}
-
-template <int DT, int MODE, bool SR, bool FAST>
 __device__ __forceinline__ void apply_phase(const TensorWork& w, int64_t wg, int64_t nwg,
                                             const SharedTables& st, const SharedSR& ssr) {
     using T = typename Elem<DT>::T;
@@ -1250,7 +1170,6 @@ __device__ __forceinline__ void apply_phase(const TensorWork& w, int64_t wg, int
     cx.sc = read_scalars(w);
     cx.kmax = (uint32_t)(w.qt->k - 1);
     cx.kk = w.qt->k;
-    cx.dense = w.qt->max_cnt > 2;
     cx.seed = w.seed;
     if constexpr (SR) {
         if (w.seed_dev != nullptr) cx.seed = (uint64_t)w.seed_dev[0];
@@ -1270,161 +1189,107 @@ __device__ __forceinline__ void apply_phase(const TensorWork& w, int64_t wg, int
     const int64_t nchunks = (w.N + kChunk - 1) / kChunk;
     int64_t ch = wg * kThreads + threadIdx.x;
     const int64_t stride = nwg * kThreads;
-    if (ch >= nchunks) return;
-
-    if constexpr (FAST) {
-        // Two chunks per iteration (ch and ch + stride): both chunks' loads are
-        // issued before either is computed.
-        Pos pa;
+    for (; ch < nchunks; ch += stride) {
+        const int64_t e0 = ch * kChunk;
+        const int nvalid = (int)std::min<int64_t>(kChunk, w.N - e0);
+        int64_t row = div_floor(e0, w.C, w.invC);
+        int64_t col = e0 - row * w.C;
+        int64_t blk = div_floor(e0, w.P, w.invP);
+        int64_t pin = e0 - blk * w.P;
+        float gv[kChunk], pv[kChunk];
+        uint32_t ix[kChunk];
         {
-            const int64_t e0 = ch * kChunk;
-            pa.row = 0;
-            pa.col = e0;
-            if constexpr (MODE == 0) {
-                pa.row = div_floor(e0, w.C, w.invC);
-                pa.col = e0 - pa.row * w.C;
-            }
-            pa.blk = div_floor(e0, w.P, w.invP);
-            pa.pin = e0 - pa.blk * w.P;
-        }
-        for (; ch < nchunks; ch += 2 * stride) {
-            const bool has_b = ch + stride < nchunks;
-            const Pos pb = advance<MODE>(w, pa);
-            const int64_t ea = ch * kChunk, eb = (ch + stride) * kChunk;
-            Raw8<DT> rga, rpa, rgb, rpb;
-            RawIdx8 ria, rib;
-            float va[kChunk], vb[kChunk];
-            load_raw8<DT>(g + ea, rga);
-            ria = load_raw_idx8(w.idx + ea);
-            if (w.write_p) {
-                load_raw8<DT>(p + ea, rpa);
-                if constexpr (MODE == 0) load_vcol(w.v1 + pa.col, va);
-            }
-            if (has_b) {
-                load_raw8<DT>(g + eb, rgb);
-                rib = load_raw_idx8(w.idx + eb);
-                if (w.write_p) {
-                    load_raw8<DT>(p + eb, rpb);
-                    if constexpr (MODE == 0) load_vcol(w.v1 + pb.col, vb);
-                }
-            }
-            uint32_t ix[kChunk];
-            float pv[kChunk];
-            apply_chunk<DT, MODE, SR>(w, st, ssr, cx, ea, pa, rga, rpa, ria, va, ix, pv);
-            store_idx8(w.idx + ea, ix);
-            if (w.write_p) store8<DT>(p + ea, pv);
-            if (has_b) {
-                apply_chunk<DT, MODE, SR>(w, st, ssr, cx, eb, pb, rgb, rpb, rib, vb, ix, pv);
-                store_idx8(w.idx + eb, ix);
-                if (w.write_p) store8<DT>(p + eb, pv);
-            }
-            pa = advance<MODE>(w, pb);
-        }
-    } else {
-        for (; ch < nchunks; ch += stride) {
-            const int64_t e0 = ch * kChunk;
-            const int nvalid = (int)std::min<int64_t>(kChunk, w.N - e0);
-            int64_t row = div_floor(e0, w.C, w.invC);
-            int64_t col = e0 - row * w.C;
-            int64_t blk = div_floor(e0, w.P, w.invP);
-            int64_t pin = e0 - blk * w.P;
-            float gv[kChunk], pv[kChunk];
-            uint32_t ix[kChunk];
-            {
-                int64_t r = row, c = col;
-#pragma unroll
-                for (int k = 0; k < kChunk; ++k) {
-                    if (k < nvalid) {
-                        gv[k] = to_f32<DT>(g[r * w.gs0 + c * w.gs1]);
-                        pv[k] = w.write_p ? to_f32<DT>(p[r * w.ps0 + c * w.ps1]) : 0.0f;
-                        ix[k] = w.idx[e0 + k];
-                        if (++c == w.C) { c = 0; ++r; }
-                    } else {
-                        gv[k] = 0.0f;
-                        pv[k] = 0.0f;
-                        ix[k] = 0u;
-                    }
-                }
-            }
-            float m_old = w.mag_old[blk];
-            float m_new = w.mag[blk];
-            float y = w.minv[blk];
-            float bstep = 0.0f;
-            if constexpr (MODE == 1) bstep = w.step[blk];
-            float rs = 0.0f, vr = 0.0f;
-            if constexpr (MODE == 0) {
-                vr = w.v0[row];
-                rs = vr * cx.row_scale;
-            }
             int64_t r = row, c = col;
 #pragma unroll
             for (int k = 0; k < kChunk; ++k) {
                 if (k < nvalid) {
-                    const float u = momentum_value(st.cbr[ix[k]], m_old, gv[k], w.mc);
-                    const float x = (m_new > 0.0f) ? div_by_block(u, m_new, y) : 0.0f;
-                    uint32_t ni;
-                    if constexpr (SR) ni = quant_stochastic(x, ssr.cb, ssr.lut, cx.kk, cx.seed, e0 + k);
-                    else ni = quant_nearest(x, st.bkt, st.thr, cx.kmax);
-                    ix[k] = ni;
-                    if (w.write_p) {
-                        const float q = st.cbr[ni] * m_new;
-                        float pw = pv[k];
-                        if (cx.wd) pw = round_dt<DT>(pw * cx.sc.wdf);
-                        if constexpr (MODE == 0) {
-                            if (DT == F32 && cx.ref.on) {
-                                pv[k] = pw - (q * ref_step(cx.ref, vr, w.v1[c])) * cx.sc.lr;
-                            } else {
-                                const float h = __builtin_amdgcn_sqrtf(rs * w.v1[c]) + w.eps;
-                                pv[k] = pw - q * (__builtin_amdgcn_rcpf(h) * cx.c1);
-                            }
+                    gv[k] = to_f32<DT>(g[r * w.gs0 + c * w.gs1]);
+                    pv[k] = w.write_p ? to_f32<DT>(p[r * w.ps0 + c * w.ps1]) : 0.0f;
+                    ix[k] = w.idx[e0 + k];
+                    if (++c == w.C) { c = 0; ++r; }
+                } else {
+                    gv[k] = 0.0f;
+                    pv[k] = 0.0f;
+                    ix[k] = 0u;
+                }
+            }
+        }
+        float m_old = w.mag_old[blk];
+        float m_new = w.mag[blk];
+        float y = w.minv[blk];
+        float bstep = 0.0f;
+        if constexpr (MODE == 1) bstep = w.step[blk];
+        float rs = 0.0f, vr = 0.0f;
+        if constexpr (MODE == 0) {
+            vr = w.v0[row];
+            rs = vr * cx.row_scale;
+        }
+        int64_t r = row, c = col;
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+            if (k < nvalid) {
+                const float u = momentum_value(st.cbr[ix[k]], m_old, gv[k], w.mc);
+                const float x = (m_new > 0.0f) ? div_by_block(u, m_new, y) : 0.0f;
+                uint32_t ni;
+                if constexpr (SR) ni = quant_stochastic(x, ssr.cb, ssr.lut, cx.kk, cx.seed, e0 + k);
+                else ni = quant_nearest(x, st.bkt, st.thr, cx.kmax);
+                ix[k] = ni;
+                if (w.write_p) {
+                    const float q = st.cbr[ni] * m_new;
+                    float pw = pv[k];
+                    if (cx.wd) pw = round_dt<DT>(pw * cx.sc.wdf);
+                    if constexpr (MODE == 0) {
+                        if (DT == F32 && cx.ref.on) {
+                            pv[k] = pw - (q * ref_step(cx.ref, vr, w.v1[c])) * cx.sc.lr;
                         } else {
-                            pv[k] = pw - (q * bstep) * cx.sc.lr;
+                            const float h = __builtin_amdgcn_sqrtf(rs * w.v1[c]) + w.eps;
+                            pv[k] = pw - q * (__builtin_amdgcn_rcpf(h) * cx.c1);
                         }
+                    } else {
+                        pv[k] = pw - (q * bstep) * cx.sc.lr;
                     }
-                    if (++c == w.C) {
-                        c = 0;
-                        ++r;
-                        if constexpr (MODE == 0) {
-                            if (k + 1 < nvalid) {
-                                vr = w.v0[r];
-                                rs = vr * cx.row_scale;
-                            }
-                        }
-                    }
-                    if (++pin == w.P) {
-                        pin = 0;
-                        ++blk;
+                }
+                if (++c == w.C) {
+                    c = 0;
+                    ++r;
+                    if constexpr (MODE == 0) {
                         if (k + 1 < nvalid) {
-                            m_old = w.mag_old[blk];
-                            m_new = w.mag[blk];
-                            y = w.minv[blk];
-                            if constexpr (MODE == 1) bstep = w.step[blk];
+                            vr = w.v0[r];
+                            rs = vr * cx.row_scale;
                         }
+                    }
+                }
+                if (++pin == w.P) {
+                    pin = 0;
+                    ++blk;
+                    if (k + 1 < nvalid) {
+                        m_old = w.mag_old[blk];
+                        m_new = w.mag[blk];
+                        y = w.minv[blk];
+                        if constexpr (MODE == 1) bstep = w.step[blk];
                     }
                 }
             }
-            int64_t rr = row, cc = col;
+        }
+        int64_t rr = row, cc = col;
 #pragma unroll
-            for (int k = 0; k < kChunk; ++k) {
-                if (k < nvalid) {
-                    w.idx[e0 + k] = (uint8_t)ix[k];
-                    if (w.write_p) p[rr * w.ps0 + cc * w.ps1] = from_f32<DT>(pv[k]);
-                    if (++cc == w.C) { cc = 0; ++rr; }
-                }
+        for (int k = 0; k < kChunk; ++k) {
+            if (k < nvalid) {
+                w.idx[e0 + k] = (uint8_t)ix[k];
+                if (w.write_p) p[rr * w.ps0 + cc * w.ps1] = from_f32<DT>(pv[k]);
+                if (++cc == w.C) { cc = 0; ++rr; }
             }
         }
     }
 }
 
 // ====================================================================
-// Fast apply (the hot path): contiguous p/grad, C % 8 == 0, P % 8 == 0,
-// nearest rounding, a table with at most one threshold per bucket.
-// Workgroup `wg` owns chunks [wg*256*kApplyChunksPerThread, ...): thread t
-// takes chunks t, t+256, ... of that range, two at a time with all loads
-// issued before any math.  Per element the only LDS traffic is the old
-// codeword, one 8-byte quantiser entry {thr[base], base} and the new
-// codeword; the step uses sqrt(v_col) precomputed by finalize and one
-// sqrt(v_row * scale) per chunk.
+// Fast apply (the hot path): contiguous p and grad of any alignment, P >= 8,
+// nearest or stochastic rounding.  Per element the only LDS traffic of nearest
+// rounding is the old codeword, one 8-byte quantiser entry {thr[base], base}
+// and the new codeword (a table with several thresholds in one bucket takes
+// the exact search instead); the step uses sqrt(v_col) precomputed by finalize
+// and one sqrt(v_row * scale) per chunk.
 // ====================================================================
 struct FastTables {
     uint2 fq[kFqEntries];
@@ -1452,6 +1317,93 @@ __device__ __forceinline__ void stage_fast(FastTables& s, const QTable* __restri
     if (threadIdx.x < kCodebookMax) s.cbr[threadIdx.x] = c;
 }
 
+// Stochastic rounding.  Entry j (0..k) describes the codewords around insertion
+// point j: r = min(j, k-1), l = max(r-1, 0), {cb[l], cb[r], RN(1 / (cb[r] -
+// cb[l])) or 0 where that is not a normal number}; lut[b] packs the range of
+// insertion points of bucket b, first | last << 16.
+struct SrTables {
+    float cbr[kCodebookMax];
+    f32x4 e[kCodebookMax + 2];
+    uint32_t lut[kBuckets];
+};
+
+__device__ __forceinline__ void stage_tabs(FastTables& s, const QTable* __restrict__ t) { stage_fast(s, t); }
+__device__ __forceinline__ void stage_tabs(SrTables& s, const QTable* __restrict__ t) {
+    const int kk = t->k;
+    for (int j = threadIdx.x; j < kCodebookMax + 2; j += kThreads) {
+        const int r = j > kk - 1 ? kk - 1 : j, l = r - 1 < 0 ? 0 : r - 1;
+        const float lv = *gbl(t->cb + l), hv = *gbl(t->cb + r);
+        s.e[j] = f32x4{lv, hv, block_recip(hv - lv), 0.0f};
+    }
+    s.cbr[threadIdx.x % kCodebookMax] = *gbl(t->cbr + threadIdx.x % kCodebookMax);
+#pragma unroll 4
+    for (int b = threadIdx.x; b < kBuckets; b += kThreads) {
+        int lo = *gbl(t->lut + b), hi = *gbl(t->lut + b + 1);
+        lo = lo < 0 ? 0 : (lo > kk ? kk : lo);
+        hi = hi < lo ? lo : (hi > kk ? kk : hi);
+        s.lut[b] = (uint32_t)lo | ((uint32_t)hi << 16);
+    }
+}
+
+// quant_stochastic, bit for bit, for four elements at a time (z: their hash
+// inputs): one LUT read, the entries of the bucket's first insertion point and
+// of the next in one go (a bucket usually holds at most one codeword), the
+// probability of rounding up through the span's reciprocal with one Markstein
+// correction (exact where the offset and the quotient are at least 2^-100; a
+// smaller one divides), and the hash's top 24 bits, which need neither its last
+// xor-shift nor the low half of its last product.
+__device__ __forceinline__ void quant_sr4(const float* xs, const SrTables& s, int kk, uint64_t z0, uint64_t dz,
+                                          uint32_t* ix) {
+    uint32_t pk[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        int b = (int)floorf((xs[k] + 1.0f) * (float)(kBuckets / 2));
+        b = b < 0 ? 0 : (b > kBuckets - 1 ? kBuckets - 1 : b);
+        pk[k] = s.lut[b];
+    }
+    f32x4 e0[4], e1[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        e0[k] = s.e[pk[k] & 0xffffu];
+        e1[k] = s.e[(pk[k] & 0xffffu) + 1u];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float x = xs[k];
+        uint32_t j = pk[k] & 0xffffu;
+        const uint32_t hi = pk[k] >> 16;
+        bool up = j < hi && e0[k].y < x;
+        f32x4 e = e0[k];
+        if (up) { e = e1[k]; ++j; }
+        while (__any(up && j < hi)) {  // several codewords in one bucket
+            up = up && j < hi && e.y < x;
+            if (up) { ++j; e = s.e[j]; }
+        }
+        const uint32_t r = j > (uint32_t)(kk - 1) ? (uint32_t)(kk - 1) : j;
+        const uint32_t l = r > 0u ? r - 1u : 0u;
+        const float span = e.y - e.x;
+        const float v = x < e.x ? e.x : (x > e.y ? e.y : x);
+        const float d = v - e.x;
+        const float q0 = d * e.z;
+        float p_up = __builtin_fmaf(__builtin_fmaf(-q0, span, d), e.z, q0);
+        const bool odd = span > 0.0f && (e.z == 0.0f || (d != 0.0f && !(q0 >= 0x1p-100f && d >= 0x1p-100f)));
+        if (__builtin_expect(__any(odd), 0)) p_up = odd ? d / span : p_up;
+        if (!(span > 0.0f)) p_up = 0.0f;
+        uint64_t z = z0 + dz * (uint64_t)k;
+        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
+        z = z ^ (z >> 27);
+        const uint32_t zl = (uint32_t)z, zh = (uint32_t)(z >> 32);
+        const uint32_t h = __umulhi(zl, 0x133111EBu) + zl * 0x94D049BBu + zh * 0x133111EBu;
+        const float u01 = (float)(h >> 8) * (1.0f / 16777216.0f);
+        ix[k] = u01 < p_up ? r : l;  // one codeword (l == r): either
+    }
+}
+constexpr uint64_t kSrStep = 0x9E3779B97F4A7C15ULL;  // hash input: seed + kSrStep * (element + 1)
+
+struct Pos {
+    int64_t blk, pin;  // block of an element and its offset there
+};
+
 // Everything the fast loop touches, copied out of the descriptor once: the
 // stores to p / indices could alias the descriptor memory, so fields read
 // through it would be re-fetched after every store.
@@ -1468,9 +1420,11 @@ struct FastArgs {
     const float* vcs;    // factored: sqrt(v_col)
     const float* bstep;  // block: per-block stepsize
     const QTable* qt;
-    int64_t C, P, fR, fC, fB, fP;
+    int64_t P, fB, fP;
     float row_scale, c1, eps, wdf, lr;
     bool wd;
+    int kk;              // codebook size
+    uint64_t seed;       // stochastic rounding
     MomentumCoef mc;
     RefStep ref;         // fp32 factored: the reference-order stepsize (vcs then holds v_col itself)
 };
@@ -1484,13 +1438,8 @@ struct ChunkIn {
     float m_old, m_new, y, rv;  // rv: v_row (factored) or the block stepsize (block)
 };
 
-template <int DT, int MODE>
-__device__ __forceinline__ Pos advance_fast(const FastArgs<DT>& a, Pos q) {
-    if constexpr (MODE == 0) {
-        q.col += a.fC;
-        q.row += a.fR;
-        if (q.col >= a.C) { q.col -= a.C; ++q.row; }
-    }
+template <int DT>
+__device__ __forceinline__ Pos advance_flat(const FastArgs<DT>& a, Pos q) {
     q.pin += a.fP;
     q.blk += a.fB;
     if (q.pin >= a.P) { q.pin -= a.P; ++q.blk; }
@@ -1504,33 +1453,30 @@ __device__ __forceinline__ uint32_t quant_global(float x, const QTable* __restri
 
 // Issue the loads of one chunk: the small per-row/per-block values first, so
 // that waiting for them never waits for the streams issued after them.
-template <int DT, int MODE>
-__device__ __forceinline__ void fast_load(const FastArgs<DT>& a, const Pos& ps, int64_t e0, ChunkIn<DT>& in) {
+template <int DT>
+__device__ __forceinline__ void flat_load(const FastArgs<DT>& a, const Pos& ps, int64_t e0, ChunkIn<DT>& in) {
     in.m_old = *gbl(a.mag_old + ps.blk);
     in.m_new = *gbl(a.mag + ps.blk);
     in.y = *gbl(a.minv + ps.blk);
-    if constexpr (MODE == 0) {
-        in.rv = *gbl(a.vrow + ps.row);
-        load_vcol(a.vcs + ps.col, in.vc);
-    } else {
-        in.rv = *gbl(a.bstep + ps.blk);
-    }
-    load_raw8<DT>(a.g + e0, in.g);
-    in.i = load_raw_idx8(a.idx + e0);
-    load_raw8<DT>(a.p + e0, in.p);
+    in.rv = *gbl(a.bstep + ps.blk);
+    load_raw8_any<DT>(a.g + e0, in.g);
+    in.i = load_raw_idx8_any(a.idx + e0);
+    load_raw8_any<DT>(a.p + e0, in.p);
 }
 
 // Requantise and apply one chunk: new indices in ix, new parameter values
 // in pv.  g and p are the chunk's grads and parameters as floats, iv its old
 // indices, vc its columns' sqrt(v_col) (v_col on the fp32 reference path),
-// rv its v_row (factored) or block stepsize (block).  GENERAL_Q: the table
-// may hold several thresholds per bucket (the fq entries do not describe
-// it), so every element takes the exact search.
-template <int DT, int MODE, int LF>
-__device__ __forceinline__ void chunk_math(const FastArgs<DT>& a, const FastTables& ft, const float g[kChunk],
+// rv its v_row (factored) or block stepsize (block), e0 its first element
+// (stochastic rounding).  general_q: the table may hold several thresholds per
+// bucket (the fq entries do not describe it), so every element takes the exact
+// search.
+template <int DT, int MODE, int LF, class Tabs>
+__device__ __forceinline__ void chunk_math(const FastArgs<DT>& a, const Tabs& ft, const float g[kChunk],
                                            const float p[kChunk], const RawIdx8& iv, const float vc[kChunk],
                                            float m_old, float m_new, float y, float rv, bool general_q,
-                                           uint32_t ix[kChunk], float pv[kChunk]) {
+                                           int64_t e0, uint32_t ix[kChunk], float pv[kChunk]) {
+    constexpr bool SR = std::is_same_v<Tabs, SrTables>;
     const float tb = 0x1.00001p-100f * fmaxf(m_new, 1.0f);
     float xs[kChunk];
     bool bad = (y == 0.0f) || general_q;
@@ -1548,9 +1494,10 @@ __device__ __forceinline__ void chunk_math(const FastArgs<DT>& a, const FastTabl
         for (int k = 0; k < kChunk; ++k) {
             const float u = momentum_value<LF>(ft.cbr[raw_idx(iv, k)], m_old, g[k], a.mc);
             const float x = nz ? div_by_block(u, m_new, y) : 0.0f;
-            ix[k] = quant_global(x, a.qt);
+            if constexpr (SR) xs[k] = x;
+            else ix[k] = quant_global(x, a.qt);
         }
-    } else {
+    } else if constexpr (!SR) {
 #pragma unroll
         for (int k = 0; k < kChunk; ++k) {
             int b = (int)__builtin_fmaf(xs[k], (float)(kBuckets / 2), (float)(kBuckets / 2));
@@ -1558,6 +1505,12 @@ __device__ __forceinline__ void chunk_math(const FastArgs<DT>& a, const FastTabl
             const uint2 e = ft.fq[b];
             ix[k] = e.y + (__uint_as_float(e.x) < xs[k] ? 1u : 0u);
         }
+    }
+    if constexpr (SR) {
+        const uint64_t z0 = a.seed + kSrStep * ((uint64_t)e0 + 1ull);
+        quant_sr4(xs, ft, a.kk, z0, kSrStep, ix);
+        __builtin_amdgcn_sched_barrier(0);  // four at a time: registers
+        quant_sr4(xs + 4, ft, a.kk, z0 + 4ull * kSrStep, kSrStep, ix + 4);
     }
     if constexpr (MODE == 0 && DT == F32) {
         if (a.ref.on) {  // reference order; vc holds v_col
@@ -1586,31 +1539,30 @@ __device__ __forceinline__ void chunk_math(const FastArgs<DT>& a, const FastTabl
     }
 }
 
-template <int DT, int MODE, int LF>
-__device__ __forceinline__ void fast_math(const FastArgs<DT>& a, const FastTables& ft, const ChunkIn<DT>& in,
-                                          bool general_q, uint32_t ix[kChunk], float pv[kChunk]) {
+template <int DT, int MODE, int LF, class Tabs>
+__device__ __forceinline__ void fast_math(const FastArgs<DT>& a, const Tabs& ft, const ChunkIn<DT>& in,
+                                          bool general_q, int64_t e0, uint32_t ix[kChunk], float pv[kChunk]) {
     float g[kChunk], p[kChunk];
 #pragma unroll
     for (int k = 0; k < kChunk; ++k) {
         g[k] = raw_elem<DT>(in.g, k);
         p[k] = raw_elem<DT>(in.p, k);
     }
-    chunk_math<DT, MODE, LF>(a, ft, g, p, in.i, in.vc, in.m_old, in.m_new, in.y, in.rv, general_q, ix, pv);
+    chunk_math<DT, MODE, LF>(a, ft, g, p, in.i, in.vc, in.m_old, in.m_new, in.y, in.rv, general_q, e0,
+                             ix, pv);
 }
 
 // Requantise and apply one chunk, then store its indices and parameters.
-template <int DT, int MODE, int LF>
-__device__ __forceinline__ void fast_compute(const FastArgs<DT>& a, const FastTables& ft, int64_t e0,
+template <int DT, int MODE, int LF, class Tabs>
+__device__ __forceinline__ void fast_compute(const FastArgs<DT>& a, const Tabs& ft, int64_t e0,
                                              const ChunkIn<DT>& in) {
     uint32_t ix[kChunk];
     float pv[kChunk];
-    fast_math<DT, MODE, LF>(a, ft, in, false, ix, pv);
+    fast_math<DT, MODE, LF>(a, ft, in, false, e0, ix, pv);
     store_idx8(a.idx + e0, ix);
     store8<DT>(a.p + e0, pv);
 }
 
-// Workgroup `wg` of one parameter's fast apply.  Two chunks are computed per
-// iteration while the next two are already loading.
 template <int DT>
 __device__ __forceinline__ FastArgs<DT> make_fast_args(const TensorWork& w, float row_scale) {
     FastArgs<DT> a;
@@ -1625,13 +1577,15 @@ __device__ __forceinline__ FastArgs<DT> make_fast_args(const TensorWork& w, floa
     a.vcs = w.vcs;
     a.bstep = w.step;
     a.qt = w.qt;
-    a.C = w.C; a.P = w.P; a.fR = w.fR; a.fC = w.fC; a.fB = w.fB; a.fP = w.fP;
+    a.P = w.P; a.fB = w.fB; a.fP = w.fP;
     a.row_scale = row_scale;
     a.c1 = sc.inv_bc1 * sc.lr;
     a.eps = w.eps;
     a.wdf = sc.wdf;
     a.lr = sc.lr;
     a.wd = sc.wdf != 1.0f;
+    a.kk = w.qt->k;
+    a.seed = w.sr && w.seed_dev != nullptr ? (uint64_t)w.seed_dev[0] : w.seed;
     a.mc = w.mc;
     a.ref.on = false;
     if constexpr (DT == F32) {
@@ -1643,11 +1597,57 @@ __device__ __forceinline__ FastArgs<DT> make_fast_args(const TensorWork& w, floa
     return a;
 }
 
-template <int DT, int MODE, int LF>
-__device__ __forceinline__ void apply_fast(const TensorWork& w, int64_t wg, const FastTables& ft,
-                                           float row_scale) {
-    const FastArgs<DT> a = make_fast_args<DT>(w, row_scale);
-    const int64_t nchunks = w.N / kChunk;
+// One chunk of `nv` elements (8, or fewer at the end of a flat tensor) whose
+// first `na` lie in block blk and the rest in the next: math and stores.  A
+// lane whose chunk holds a border (na < nv) first stores what block blk gives
+// for the whole chunk, then the elements of the next block over it (a wave's
+// stores to one address stay in order, and no other wave touches the chunk):
+// keeping the first results for a select instead cost the registers of the
+// fourth wave per SIMD.
+// BORDERS false: na and nv are 8.
+template <int DT, int MODE, int LF, bool BORDERS, class Tabs>
+__device__ __forceinline__ void chunk_step(const FastArgs<DT>& a, const Tabs& ft, ChunkIn<DT>& in, int64_t blk,
+                                           int na, int nv, bool store, bool write_p, bool general_q, int64_t e0) {
+    uint32_t ix[kChunk];
+    float pv[kChunk];
+    fast_math<DT, MODE, LF>(a, ft, in, general_q, e0, ix, pv);
+    if (store && (!BORDERS || nv == kChunk)) {
+        store_idx8_any(a.idx + e0, ix);
+        if (write_p) store8_any<DT>(a.p + e0, pv);
+    }
+    if constexpr (!BORDERS) return;
+    const bool border = na < nv;
+    if (__builtin_expect(!__any(border || nv < kChunk), 1)) return;
+    auto put = [&](int k0, int k1) {
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+            if (k < k0 || k >= k1) continue;
+            *gbl(a.idx + e0 + k) = (uint8_t)ix[k];
+            if (write_p) *gbl(a.p + e0 + k) = from_f32<DT>(pv[k]);
+        }
+    };
+    if (store && nv < kChunk) put(0, nv);
+    if (!__any(border)) return;
+    const int64_t b = border ? blk + 1 : blk;
+    in.m_old = *gbl(a.mag_old + b);
+    in.m_new = *gbl(a.mag + b);
+    in.y = *gbl(a.minv + b);
+    if constexpr (MODE == 1) in.rv = *gbl(a.bstep + b);
+    fast_math<DT, MODE, LF>(a, ft, in, general_q, e0, ix, pv);
+    if (store && border) put(na, nv);
+}
+
+// Block path, contiguous p and grad, a linear walk.  Workgroup wg owns chunks
+// [wg*256*kApplyChunksPerThread, ...), thread t takes t, t+256, ... of them.
+// HOT: P and N multiples of 8, everything aligned, nearest rounding.  Otherwise
+// any alignment, N and P >= 8; two chunks are computed while the next two load.
+template <int DT, int LF, bool HOT, class Tabs>
+__device__ __forceinline__ void apply_flat(const TensorWork& w, int64_t wg, const Tabs& ft) {
+    constexpr int MODE = 1;
+    const FastArgs<DT> a = make_fast_args<DT>(w, 0.0f);
+    const bool general_q = !std::is_same_v<Tabs, SrTables> && w.qt->max_cnt > 1;
+    const bool write_p = w.write_p != 0;
+    const int64_t N = w.N, nchunks = (N + kChunk - 1) / kChunk;
     const int64_t first = wg * (kThreads * kApplyChunksPerThread) + threadIdx.x;
     if (first >= nchunks) return;
     // chunks of this thread: first + i*256 for i < n (n >= 1)
@@ -1655,147 +1655,225 @@ __device__ __forceinline__ void apply_fast(const TensorWork& w, int64_t wg, cons
     Pos p0;
     {
         const int64_t e0 = first * kChunk;
-        p0.row = 0;
-        p0.col = e0;
-        if constexpr (MODE == 0) {
-            p0.row = div_floor(e0, w.C, w.invC);
-            p0.col = e0 - p0.row * w.C;
-        }
         p0.blk = div_floor(e0, w.P, w.invP);
         p0.pin = e0 - p0.blk * w.P;
     }
-    Pos p1 = advance_fast<DT, MODE>(a, p0);
+    Pos p1 = advance_flat<DT>(a, p0);
     ChunkIn<DT> A, B;
-    if ((wg + 1) * (kThreads * kApplyChunksPerThread) <= nchunks) {
-        // A full workgroup (all but a tensor's last): straight-line code with
-        // every load and store unconditional, so each wait names exactly the
-        // chunk about to be computed and the next two chunks stay in flight.
-        // (A load or store behind a branch makes the compiler assume, at the
-        // join, the path with fewer operations in flight, and the waits then
-        // drain the prefetched chunks as well.)
-        fast_load<DT, MODE>(a, p0, first * kChunk, A);
-        fast_load<DT, MODE>(a, p1, (first + kThreads) * kChunk, B);
+    if constexpr (HOT) {
+        if ((wg + 1) * (kThreads * kApplyChunksPerThread) <= nchunks && write_p && !general_q) {
+            // A full workgroup: straight-line code with every load and store
+            // unconditional, so each wait names exactly the chunk about to be
+            // computed and the next two chunks stay in flight.  (A load or store
+            // behind a branch makes the compiler assume, at the join, the path
+            // with fewer operations in flight, and the waits then drain the
+            // prefetched chunks as well.)
+            flat_load<DT>(a, p0, first * kChunk, A);
+            flat_load<DT>(a, p1, (first + kThreads) * kChunk, B);
 #pragma unroll
-        for (int i = 0; i < (int)kApplyChunksPerThread; i += 2) {
-            const int64_t ea = (first + (int64_t)i * kThreads) * kChunk;
-            const int64_t eb = ea + kThreads * kChunk;
-            const Pos p2 = advance_fast<DT, MODE>(a, p1);
-            const Pos p3 = advance_fast<DT, MODE>(a, p2);
-            fast_compute<DT, MODE, LF>(a, ft, ea, A);
-            if (i + 2 < (int)kApplyChunksPerThread) fast_load<DT, MODE>(a, p2, ea + 2 * kThreads * kChunk, A);
-            fast_compute<DT, MODE, LF>(a, ft, eb, B);
-            if (i + 3 < (int)kApplyChunksPerThread) fast_load<DT, MODE>(a, p3, eb + 2 * kThreads * kChunk, B);
-            p1 = p3;
+            for (int i = 0; i < (int)kApplyChunksPerThread; i += 2) {
+                const int64_t ea = (first + (int64_t)i * kThreads) * kChunk;
+                const int64_t eb = ea + kThreads * kChunk;
+                const Pos p2 = advance_flat<DT>(a, p1);
+                const Pos p3 = advance_flat<DT>(a, p2);
+                fast_compute<DT, MODE, LF>(a, ft, ea, A);
+                if (i + 2 < (int)kApplyChunksPerThread) flat_load<DT>(a, p2, ea + 2 * kThreads * kChunk, A);
+                fast_compute<DT, MODE, LF>(a, ft, eb, B);
+                if (i + 3 < (int)kApplyChunksPerThread) flat_load<DT>(a, p3, eb + 2 * kThreads * kChunk, B);
+                p1 = p3;
+            }
+            return;
+        }
+#pragma unroll 1
+        for (int i = 0; i < n; ++i) {
+            const int64_t e0 = (first + (int64_t)i * kThreads) * kChunk;
+            flat_load<DT>(a, p0, e0, A);
+            chunk_step<DT, MODE, LF, false>(a, ft, A, p0.blk, kChunk, kChunk, true, write_p, general_q, e0);
+            p0 = advance_flat<DT>(a, p0);
         }
         return;
     }
-    fast_load<DT, MODE>(a, p0, first * kChunk, A);
-    if (n > 1) fast_load<DT, MODE>(a, p1, (first + kThreads) * kChunk, B);
+    auto load = [&](const Pos& q, int64_t e0, ChunkIn<DT>& in) {
+        if (e0 + kChunk <= N) {
+            flat_load<DT>(a, q, e0, in);
+            return;
+        }
+        // the tensor's last elements, one by one (the last one again past its end)
+        in.m_old = *gbl(a.mag_old + q.blk);
+        in.m_new = *gbl(a.mag + q.blk);
+        in.y = *gbl(a.minv + q.blk);
+        in.rv = *gbl(a.bstep + q.blk);
+        const int64_t last = N - 1 - e0;
+        auto at = [&](int k) { return e0 + (k < last ? k : last); };
+        uint32_t lo = 0u, hi = 0u;
+#pragma unroll
+        for (int k = 0; k < kChunk; ++k) {
+            const uint32_t v = *gbl(a.idx + at(k));
+            if (k < 4) lo |= v << (8 * k);
+            else hi |= v << (8 * (k - 4));
+        }
+        in.i = RawIdx8{lo, hi};
+        if constexpr (DT == F32) {
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {
+                in.g.f[k] = *gbl(a.g + at(k));
+                in.p.f[k] = *gbl(a.p + at(k));
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                in.g.w[k] = (uint32_t)*gbl(a.g + at(2 * k)) | ((uint32_t)*gbl(a.g + at(2 * k + 1)) << 16);
+                in.p.w[k] = (uint32_t)*gbl(a.p + at(2 * k)) | ((uint32_t)*gbl(a.p + at(2 * k + 1)) << 16);
+            }
+        }
+    };
+    auto compute = [&](const Pos& q, int64_t e0, ChunkIn<DT>& in) {
+        const int na = (int)std::min<int64_t>(kChunk, a.P - q.pin);
+        const int nv = (int)std::min<int64_t>(kChunk, N - e0);
+        chunk_step<DT, MODE, LF, true>(a, ft, in, q.blk, na, nv, true, write_p, general_q, e0);
+    };
+    load(p0, first * kChunk, A);
+    if (n > 1) load(p1, (first + kThreads) * kChunk, B);
 #pragma unroll 1
     for (int i = 0; i < n; i += 2) {
         const int64_t ea = (first + (int64_t)i * kThreads) * kChunk;
         const int64_t eb = ea + kThreads * kChunk;
-        const Pos p2 = advance_fast<DT, MODE>(a, p1);
-        const Pos p3 = advance_fast<DT, MODE>(a, p2);
-        fast_compute<DT, MODE, LF>(a, ft, ea, A);
-        if (i + 2 < n) fast_load<DT, MODE>(a, p2, ea + 2 * kThreads * kChunk, A);
-        if (i + 1 < n) fast_compute<DT, MODE, LF>(a, ft, eb, B);
-        if (i + 3 < n) fast_load<DT, MODE>(a, p3, eb + 2 * kThreads * kChunk, B);
+        const Pos p2 = advance_flat<DT>(a, p1);
+        const Pos p3 = advance_flat<DT>(a, p2);
+        compute(p0, ea, A);
+        if (i + 2 < n) load(p2, ea + 2 * kThreads * kChunk, A);
+        if (i + 1 < n) compute(p1, eb, B);
+        if (i + 3 < n) load(p3, eb + 2 * kThreads * kChunk, B);
         p0 = p2;
         p1 = p3;
     }
 }
 
-// Factored apply over row segments (contiguous p and grad, C >= 512).  The
-// tasks are 512-column segments of 8 rows, segment-fastest; wave v of
-// workgroup wg takes task 4*wg + v.  A lane keeps its 8 columns' sqrt(v_col)
-// in registers for the task's rows, v_row is a scalar load per row, and when
-// the segment lies inside one block in every row of the task, so are the
-// block's magnitudes and reciprocal: per 8 elements the lane loads only g, p
-// and the indices (the per-chunk v_col and block loads of apply_fast cost
-// ~6% of the apply time).  Two rows are in flight while one is computed.
-
-template <int DT, int LF>
-__device__ __forceinline__ void apply_rows(const TensorWork& w, int64_t wg, const FastTables& ft, float row_scale) {
+// Factored apply, contiguous p and grad.  A row is cut into w.a_segs even
+// segments of w.a_cols <= 512 columns; 1 << w.a_lg lanes take a segment, 8
+// columns each, a wave 64 >> a_lg rows at a time.  A task is w.a_steps such row
+// steps of one segment, segment-fastest; wave v of workgroup wg takes task 4*wg
+// + v.  Lanes past the segment's last whole chunk repeat the segment's last 8
+// columns: in each step every lane has loaded before any stores, and
+// overlapping lanes store the same values, so no chunk needs a mask.  A lane
+// keeps its 8 columns' sqrt(v_col) in registers.
+// HOT (C >= 512, C and P multiples of 8, blocks of at least kShortPeriod,
+// everything aligned, nearest rounding): a task whose segment lies inside one
+// block in every row takes v_row and the block's magnitudes and reciprocal as
+// scalar loads; per 8 elements the lane loads only g, p and the indices (the
+// per-chunk v_col and block loads of a linear walk cost ~6% of the apply time).
+// Two rows are in flight while two are computed.  Otherwise (any alignment, C >=
+// 8, P >= 8, stochastic rounding) each lane loads its row's and block's values
+// with its chunk (43M fp16 elements with stochastic rounding: 166 us + 81 for
+// the odd-sized two through element loads -> 195 in one launch).  The two are kernels of their own: in one, the borders'
+// registers cost the HOT tasks their fourth wave per SIMD (1.05e9 elements 1530
+// -> 1592 us).
+template <int DT, int LF, bool HOT, class Tabs>
+__device__ __forceinline__ void apply_tasks(const TensorWork& w, int64_t wg, const Tabs& ft, float row_scale) {
     const FastArgs<DT> a = make_fast_args<DT>(w, row_scale);
+    const bool general_q = !std::is_same_v<Tabs, SrTables> && w.qt->max_cnt > 1;
+    const bool write_p = w.write_p != 0;
     const int64_t C = w.C, R = w.R, P = w.P;
-    const int64_t nseg = (C + kRowSegCols - 1) / kRowSegCols;
     const int64_t t = wg * kWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t rt = t / nseg;
-    const int64_t cs = (t - rt * nseg) * kRowSegCols;
-    const int64_t r0 = rt * kRowsPerTask;
+    const int64_t rt = t / w.a_segs;
+    const int64_t cs = (t - rt * w.a_segs) * w.a_cols;
+    const int64_t ce = std::min<int64_t>(cs + w.a_cols, C);
+    const int lane = threadIdx.x & 63, lg = w.a_lg, rpw = 64 >> lg, steps = w.a_steps;
+    const int64_t r0 = rt * steps * rpw;
     if (r0 >= R) return;
-    const int64_t seglen = std::min<int64_t>(kRowSegCols, C - cs);
-    const int64_t c = cs + (int64_t)(threadIdx.x & 63) * kChunk;
-    const bool active = c < C;
-    const int64_t cl = active ? c : cs;  // idle lanes of a short segment re-read its first chunk
-    const int nrows = (int)std::min<int64_t>(kRowsPerTask, R - r0);
-    // block and offset of the segment's first element, row by row
-    // (wave-uniform): one block per row when pin + seglen <= P
-    const int64_t e_first = r0 * C + cs;
-    int64_t bk[kRowsPerTask];
-    bool uniform = true;
-    {
-        int64_t b = div_floor(e_first, P, w.invP);
-        int64_t pin = e_first - b * P;
-        const int64_t dB = div_floor(C, P, w.invP);
-        const int64_t dP = C - dB * P;
+    const int64_t c = std::min<int64_t>(cs + (lane & ((1 << lg) - 1)) * kChunk, ce - kChunk);
+    float vc[kChunk];
+    load_vcol_any(a.vcs + c, vc);
+    if (HOT && rpw == 1 && steps == kRowsPerTask && r0 + kRowsPerTask <= R && write_p && !general_q) {
+        // block and offset of the segment's first element, row by row
+        // (wave-uniform): one block per row when pin + seglen <= P
+        int64_t bk[kRowsPerTask];
+        bool uniform = true;
+        {
+            const int64_t e_first = r0 * C + cs;
+            int64_t b = div_floor(e_first, P, w.invP);
+            int64_t pin = e_first - b * P;
+            const int64_t dB = div_floor(C, P, w.invP);
+            const int64_t dP = C - dB * P;
 #pragma unroll
-        for (int i = 0; i < kRowsPerTask; ++i) {
-            bk[i] = b;
-            uniform = uniform && (i >= nrows || pin + seglen <= P);
-            pin += dP;
-            b += dB;
-            if (pin >= P) { pin -= P; ++b; }
+            for (int i = 0; i < kRowsPerTask; ++i) {
+                bk[i] = b;
+                uniform = uniform && pin + (ce - cs) <= P;
+                pin += dP;
+                b += dB;
+                if (pin >= P) { pin -= P; ++b; }
+            }
+        }
+        if (uniform) {
+            auto load_row = [&](int i, ChunkIn<DT>& in) {
+                const int64_t r = r0 + i;
+                const int64_t e0 = r * C + c;
+                in.m_old = sload(a.mag_old + bk[i]);
+                in.m_new = sload(a.mag + bk[i]);
+                in.y = sload(a.minv + bk[i]);
+                in.rv = sload(a.vrow + r);
+                load_raw8<DT>(a.g + e0, in.g);
+                in.i = load_raw_idx8(a.idx + e0);
+                load_raw8<DT>(a.p + e0, in.p);
+            };
+            ChunkIn<DT> A, B;
+            load_row(0, A);
+            load_row(1, B);
+#pragma unroll
+            for (int i = 0; i < kRowsPerTask; i += 2) {
+#pragma unroll
+                for (int k = 0; k < kChunk; ++k) { A.vc[k] = vc[k]; B.vc[k] = vc[k]; }
+                fast_compute<DT, 0, LF>(a, ft, (r0 + i) * C + c, A);
+                if (i + 2 < kRowsPerTask) load_row(i + 2, A);
+                fast_compute<DT, 0, LF>(a, ft, (r0 + i + 1) * C + c, B);
+                if (i + 3 < kRowsPerTask) load_row(i + 3, B);
+            }
+            return;
         }
     }
-    if (nrows == kRowsPerTask && seglen == kRowSegCols && uniform) {
-        float vc[kChunk];
-        load_vcol(a.vcs + c, vc);
-        auto load_row = [&](int i, ChunkIn<DT>& in) {
-            const int64_t r = r0 + i;
-            const int64_t e0 = r * C + c;
-            in.m_old = sload(a.mag_old + bk[i]);
-            in.m_new = sload(a.mag + bk[i]);
-            in.y = sload(a.minv + bk[i]);
-            in.rv = sload(a.vrow + r);
-            load_raw8<DT>(a.g + e0, in.g);
-            in.i = load_raw_idx8(a.idx + e0);
-            load_raw8<DT>(a.p + e0, in.p);
-        };
-        ChunkIn<DT> A, B;
-        load_row(0, A);
-        load_row(1, B);
+    // rows of step i: r0 + i * rpw + sub; a lane past R loads row R - 1 and stores nothing
+    const int sub = lane >> lg;
+    const int n = (int)std::min<int64_t>(steps, (R - r0 + rpw - 1) / rpw);
+    struct At {
+        int64_t blk;
+        int na;  // elements of the chunk in that block (8: all)
+    };
+    auto load = [&](int i, ChunkIn<DT>& in, At& at) {
+        const int64_t r = std::min<int64_t>(r0 + (int64_t)i * rpw + sub, R - 1);
+        const int64_t e0 = r * C + c;
+        at.blk = div_floor(e0, P, w.invP);
+        at.na = HOT ? kChunk : (int)std::min<int64_t>(kChunk, P - (e0 - at.blk * P));
+        in.m_old = *gbl(a.mag_old + at.blk);
+        in.m_new = *gbl(a.mag + at.blk);
+        in.y = *gbl(a.minv + at.blk);
+        in.rv = *gbl(a.vrow + r);
+        load_raw8_any<DT>(a.g + e0, in.g);
+        in.i = load_raw_idx8_any(a.idx + e0);
+        load_raw8_any<DT>(a.p + e0, in.p);
+    };
+    auto compute = [&](int i, ChunkIn<DT>& in, const At& at) {
+        const int64_t r = r0 + (int64_t)i * rpw + sub;
 #pragma unroll
-        for (int i = 0; i < kRowsPerTask; i += 2) {
-#pragma unroll
-            for (int k = 0; k < kChunk; ++k) { A.vc[k] = vc[k]; B.vc[k] = vc[k]; }
-            fast_compute<DT, 0, LF>(a, ft, (r0 + i) * C + c, A);
-            if (i + 2 < kRowsPerTask) load_row(i + 2, A);
-            fast_compute<DT, 0, LF>(a, ft, (r0 + i + 1) * C + c, B);
-            if (i + 3 < kRowsPerTask) load_row(i + 3, B);
-        }
-        return;
-    }
-    // a short segment, fewer rows, or a block boundary inside the segment:
-    // one row at a time, per-lane block values
+        for (int k = 0; k < kChunk; ++k) in.vc[k] = vc[k];
+        chunk_step<DT, 0, LF, !HOT>(a, ft, in, at.blk, at.na, kChunk, r < R, write_p, general_q, r * C + c);
+    };
+    ChunkIn<DT> A, B;
+    At pa, pb;
+    if constexpr (HOT) {  // a block border inside the segment, or fewer rows: one row at a time
 #pragma unroll 1
-    for (int i = 0; i < nrows; ++i) {
-        const int64_t r = r0 + i;
-        const int64_t e0 = r * C + cl;
-        Pos ps;
-        ps.row = r;
-        ps.col = cl;
-        ps.blk = div_floor(e0, P, w.invP);
-        ps.pin = e0 - ps.blk * P;
-        ChunkIn<DT> in;
-        fast_load<DT, 0>(a, ps, e0, in);
-        uint32_t ix[kChunk];
-        float pv[kChunk];
-        fast_math<DT, 0, LF>(a, ft, in, false, ix, pv);
-        if (active) {
-            store_idx8(a.idx + e0, ix);
-            store8<DT>(a.p + e0, pv);
+        for (int i = 0; i < n; ++i) {
+            load(i, A, pa);
+            compute(i, A, pa);
+        }
+    } else {
+        load(0, A, pa);
+        if (n > 1) load(1, B, pb);
+#pragma unroll 1
+        for (int i = 0; i < n; i += 2) {
+            compute(i, A, pa);
+            if (i + 2 < n) load(i + 2, A, pa);
+            if (i + 1 < n) compute(i + 1, B, pb);
+            if (i + 3 < n) load(i + 3, B, pb);
         }
     }
 }
@@ -1899,7 +1977,7 @@ __device__ __forceinline__ void apply_tv(const TensorWork& w, int64_t wg, const 
             uint32_t ix[kChunk];
             float pn[kChunk];
             chunk_math<DT, MODE, LF>(a, ft, gj, pj, iv[j], vc, mo[j], mn[j], y[j], MODE == 0 ? vr[j] : bs[j],
-                                     general_q, ix, pn);
+                                     general_q, 0, ix, pn);
             if (ok) store_idx8(a.idx + (r + j) * C + c, ix);
 #pragma unroll
             for (int k = 0; k < kChunk; ++k) po[k][j] = pn[k];
@@ -1924,46 +2002,44 @@ __device__ __forceinline__ void apply_tv_wg(const TensorWork& w, int64_t wg, Fas
     else apply_tv<DT, MODE, kLerpLarge>(w, wg, ft, row_scale);
 }
 
-// LDS of the apply kernels: the fast tables or the general ones, never both.
-union ApplyLds {
-    FastTables f;
-    struct {
-        SharedTables st;
-        SharedSR ssr;
-    } g;
+// LDS of the apply kernels.
+template <bool SR, int FAST>
+struct ApplyLds {
+    std::conditional_t<SR, SrTables, FastTables> f;
+};
+template <bool SR>
+struct ApplyLds<SR, 0> {
+    SharedTables st;
+    SharedSR ssr;
 };
 
-// One apply workgroup: the fast path when the parameter and the table allow
-// it, the general path (grid-stride over all chunks, any strides, stochastic
-// rounding, dense tables) otherwise.
-template <int DT, int MODE, bool SR, bool FAST>
-__device__ __forceinline__ void apply_wg(const TensorWork& w, int64_t wg, int64_t nwg, ApplyLds& lds) {
+// One apply workgroup.  FAST as w.fast_apply: 1 the HOT forms, 3 contiguous p
+// and grad of any alignment, 0 any strides (grid-stride over all chunks).
+template <int DT, int MODE, bool SR, int FAST>
+__device__ __forceinline__ void apply_wg(const TensorWork& w, int64_t wg, int64_t nwg, ApplyLds<SR, FAST>& lds) {
     const QTable* qt = w.qt;
-    if constexpr (FAST && !SR) {
-        if (w.write_p && qt->max_cnt <= 1) {
-            stage_fast(lds.f, qt);
-            float row_scale = 0.0f;
-            if constexpr (MODE == 0) {
-                const StepScalars sc = read_scalars(w);
-                row_scale = (1.0f / stored_mean(w)) * sc.inv_bc2;
-            }
-            __syncthreads();
-            if constexpr (MODE == 0) {
-                if (w.row_apply) {
-                    if (w.mc.small) apply_rows<DT, kLerpSmall>(w, wg, lds.f, row_scale);
-                    else apply_rows<DT, kLerpLarge>(w, wg, lds.f, row_scale);
-                    return;
-                }
-            }
-            if (w.mc.small) apply_fast<DT, MODE, kLerpSmall>(w, wg, lds.f, row_scale);
-            else apply_fast<DT, MODE, kLerpLarge>(w, wg, lds.f, row_scale);
-            return;
+    if constexpr (FAST != 0) {
+        constexpr bool HOT = FAST == 1;
+        stage_tabs(lds.f, qt);
+        float row_scale = 0.0f;
+        if constexpr (MODE == 0) {
+            const StepScalars sc = read_scalars(w);
+            row_scale = (1.0f / stored_mean(w)) * sc.inv_bc2;
         }
+        __syncthreads();
+        if constexpr (MODE == 0) {
+            if (w.mc.small) apply_tasks<DT, kLerpSmall, HOT>(w, wg, lds.f, row_scale);
+            else apply_tasks<DT, kLerpLarge, HOT>(w, wg, lds.f, row_scale);
+        } else {
+            if (w.mc.small) apply_flat<DT, kLerpSmall, HOT>(w, wg, lds.f);
+            else apply_flat<DT, kLerpLarge, HOT>(w, wg, lds.f);
+        }
+    } else {
+        stage_tables(lds.st, qt);
+        if constexpr (SR) stage_sr(lds.ssr, qt);
+        __syncthreads();
+        apply_phase<DT, MODE, SR>(w, wg, nwg, lds.st, lds.ssr);
     }
-    stage_tables(lds.g.st, qt);
-    if constexpr (SR) stage_sr(lds.g.ssr, qt);
-    __syncthreads();
-    apply_phase<DT, MODE, SR, FAST>(w, wg, nwg, lds.g.st, lds.g.ssr);
 }
 
 // ====================================================================
@@ -2015,9 +2091,9 @@ __global__ void __launch_bounds__(kThreads) k_block_stats(TensorWork w) {
     stats_block_wg<DT>(w, blockIdx.x);
 }
 
-template <int DT, int MODE, bool SR, bool FAST>
+template <int DT, int MODE, bool SR, int FAST>
 __global__ void __launch_bounds__(kThreads) k_apply(TensorWork w) {
-    __shared__ ApplyLds lds;
+    __shared__ ApplyLds<SR, FAST> lds;
     apply_wg<DT, MODE, SR, FAST>(w, blockIdx.x, gridDim.x, lds);
 }
 
@@ -2056,13 +2132,13 @@ __global__ void __launch_bounds__(kThreads) k_mt_apply_tv(const TensorWork* __re
 
 // Apply of a launch group; with MODE 0 the group's block-path tensors of the
 // same dtype and variant (not transposed views) ride in the same launch.
-template <int DT, int MODE, bool SR, bool FAST>
+template <int DT, int MODE, bool SR, int FAST>
 // Each XCD runs a contiguous range of the launch's workgroups, i.e. streams
 // its own part of each tensor (measured on the Llama-3-8B set: apply
 // 11.51-11.61 -> 11.42-11.44 ms, with a smaller spread between processes).
-__global__ void __launch_bounds__(kThreads) k_mt_apply(const TensorWork* __restrict__ ws,
+__global__ void __launch_bounds__(kThreads, FAST == 1 ? 4 : SR ? 2 : 3) k_mt_apply(const TensorWork* __restrict__ ws,
                                                        SegTable tb) {
-    __shared__ ApplyLds lds;
+    __shared__ ApplyLds<SR, FAST> lds;
     const int64_t L = xcd_contiguous(blockIdx.x, gridDim.x);
     const Seg sg = find_seg(tb, L);
     const TensorWork& w = ws[sg.t];
@@ -2089,12 +2165,14 @@ void StepKernels<DT>::stats(const TensorWork& w, hipStream_t s) {
 template <int DT, int MODE>
 static void launch_apply(const TensorWork& w, hipStream_t s) {
     const dim3 grid((unsigned)w.apply_wgs), block(kThreads);
-    if (w.fast_apply) {
-        if (w.sr) hipLaunchKernelGGL((k_apply<DT, MODE, true, true>), grid, block, 0, s, w);
-        else hipLaunchKernelGGL((k_apply<DT, MODE, false, true>), grid, block, 0, s, w);
+    if (w.fast_apply == 1) {
+        hipLaunchKernelGGL((k_apply<DT, MODE, false, 1>), grid, block, 0, s, w);
+    } else if (w.fast_apply) {
+        if (w.sr) hipLaunchKernelGGL((k_apply<DT, MODE, true, 3>), grid, block, 0, s, w);
+        else hipLaunchKernelGGL((k_apply<DT, MODE, false, 3>), grid, block, 0, s, w);
     } else {
-        if (w.sr) hipLaunchKernelGGL((k_apply<DT, MODE, true, false>), grid, block, 0, s, w);
-        else hipLaunchKernelGGL((k_apply<DT, MODE, false, false>), grid, block, 0, s, w);
+        if (w.sr) hipLaunchKernelGGL((k_apply<DT, MODE, true, 0>), grid, block, 0, s, w);
+        else hipLaunchKernelGGL((k_apply<DT, MODE, false, 0>), grid, block, 0, s, w);
     }
 }
 
@@ -2122,13 +2200,15 @@ void StepKernels<DT>::mt_apply(int key_mode, int fast, int sr, dim3 grid, hipStr
     if (fast == 2) {
         if (key_mode == 0) hipLaunchKernelGGL((k_mt_apply_tv<DT, 0>), grid, block, 0, s, ws, sg);
         else hipLaunchKernelGGL((k_mt_apply_tv<DT, 1>), grid, block, 0, s, ws, sg);
+    } else if (fast == 1) {
+        // factored and block-path tensors together (the kernels branch per tensor)
+        hipLaunchKernelGGL((k_mt_apply<DT, 0, false, 1>), grid, block, 0, s, ws, sg);
     } else if (fast) {
-        // factored and block-path tensors together (the kernel branches per tensor)
-        if (sr) hipLaunchKernelGGL((k_mt_apply<DT, 0, true, true>), grid, block, 0, s, ws, sg);
-        else hipLaunchKernelGGL((k_mt_apply<DT, 0, false, true>), grid, block, 0, s, ws, sg);
+        if (sr) hipLaunchKernelGGL((k_mt_apply<DT, 0, true, 3>), grid, block, 0, s, ws, sg);
+        else hipLaunchKernelGGL((k_mt_apply<DT, 0, false, 3>), grid, block, 0, s, ws, sg);
     } else {
-        if (sr) hipLaunchKernelGGL((k_mt_apply<DT, 0, true, false>), grid, block, 0, s, ws, sg);
-        else hipLaunchKernelGGL((k_mt_apply<DT, 0, false, false>), grid, block, 0, s, ws, sg);
+        if (sr) hipLaunchKernelGGL((k_mt_apply<DT, 0, true, 0>), grid, block, 0, s, ws, sg);
+        else hipLaunchKernelGGL((k_mt_apply<DT, 0, false, 0>), grid, block, 0, s, ws, sg);
     }
 }
 

@@ -354,8 +354,13 @@ static int build_work(const WorkInput& in, TensorWork& w) {
             w.ct = t.ct_l; w.rt = t.rt_l; w.tile_rows = t.l_rows; w.tile_cols = t.l_cols;
             w.stats_wgs = t.ct_l * t.rt_l;
         }
-        w.fast_apply = contig_g && contig_p && (in.C % kChunk == 0) && (in.period % kChunk == 0) &&
-                       aligned(in.grad, 16) && aligned(in.p, 16) && aligned(in.idx, 8) && aligned(in.v1, 16);
+        w.fast_apply = 0;
+        if (contig_g && contig_p && in.C >= kChunk && in.period >= kChunk) {
+            const bool hot = !in.sr && in.C >= kRowSegCols && in.C % kChunk == 0 && in.period % kChunk == 0 &&
+                             in.period >= kShortPeriod && aligned(in.grad, 16) && aligned(in.p, 16) &&
+                             aligned(in.idx, 8);
+            w.fast_apply = hot ? 1 : 3;
+        }
         if (!w.fast_stats && tv_shape && tv_g) {
             w.fast_stats = 2;
             w.ct = t.ct_tv; w.rt = t.rt_tv;
@@ -396,8 +401,12 @@ static int build_work(const WorkInput& in, TensorWork& w) {
         w.nbw = std::max<int64_t>(1, std::min<int64_t>(4096, ceil_div(nb, kThreads)));
         w.fin_wgs = w.nbw;
         w.fast_stats = aligned(in.grad, 16) && aligned(in.idx, 8);
-        w.fast_apply = (in.period % kChunk == 0) && aligned(in.grad, 16) && aligned(in.p, 16) &&
-                       aligned(in.idx, 8);
+        w.fast_apply = 0;
+        if (in.period >= kChunk) {
+            const bool hot = !in.sr && in.period % kChunk == 0 && aligned(in.grad, 16) && aligned(in.p, 16) &&
+                             aligned(in.idx, 8);
+            w.fast_apply = hot ? 1 : 3;
+        }
         if (in.R > 1) {
             // a 2D descriptor that is not contiguous (the callers flatten the
             // contiguous ones): the grad must be contiguous (flat stats) or a
@@ -428,25 +437,36 @@ static int build_work(const WorkInput& in, TensorWork& w) {
         }
     }
     w.apply_wgs = std::max<int64_t>(1, ceil_div(nchunks, kThreads * kApplyChunksPerThread));
-    // contiguous factored tensors of at least one 512-column segment per row:
-    // row segments (apply_rows); any grid size works for the general apply
-    w.row_apply = (in.mode == 0 && w.fast_apply == 1 && in.R > 1 && in.C >= kRowSegCols) ? 1 : 0;
-    if (w.row_apply)
-        w.apply_wgs = ceil_div(ceil_div(in.C, kRowSegCols) * ceil_div(in.R, (int64_t)kRowsPerTask), (int64_t)kWaves);
+    if (in.mode == 0 && (w.fast_apply & 1)) {  // 1 or 3
+        // even segments of at most 512 columns, a whole number of chunks each
+        // but the last; short rows share a wave.  kRowsPerTask row steps a
+        // task, fewer where the launch would leave CUs idle.
+        w.a_segs = ceil_div(in.C, kRowSegCols);
+        w.a_cols = ceil_div(ceil_div(in.C, w.a_segs), (int64_t)kChunk) * kChunk;
+        w.a_segs = ceil_div(in.C, w.a_cols);
+        // no last segment of fewer than 8 columns: its lanes would step back
+        // into the segment before it, which another wave updates
+        while (w.a_segs > 1 && in.C - (w.a_segs - 1) * w.a_cols < kChunk) {
+            w.a_cols -= kChunk;
+            w.a_segs = ceil_div(in.C, w.a_cols);
+        }
+        w.a_lg = 0;
+        while ((kChunk << w.a_lg) < w.a_cols) ++w.a_lg;
+        w.a_steps = in.launch_elems < kSmallApplyElems ? 2 : kRowsPerTask;
+        const int64_t task_rows = (int64_t)w.a_steps * (64 >> w.a_lg);
+        w.apply_wgs = ceil_div(w.a_segs * ceil_div(in.R, task_rows), (int64_t)kWaves);
+    }
     if (w.fast_apply == 2)
         w.apply_wgs = ceil_div(ceil_div(in.R, kTv) * ceil_div(in.C, kTv), (int64_t)kWaves * kTvTilesPerWave);
-    const int64_t S = w.apply_wgs * kThreads * kChunk;
-    w.dR = S / w.C;
-    w.dC = S - w.dR * w.C;
-    w.dB = S / w.P;
-    w.dP = S - w.dB * w.P;
     const int64_t F = kThreads * kChunk;
-    w.fR = F / w.C;
-    w.fC = F - w.fR * w.C;
     w.fB = F / w.P;
     w.fP = F - w.fB * w.P;
     return GEFENX_OK;
 }
+
+// 8% of the apply of so many 16-bit elements (8 B each at ~5.5 TB/s) are about
+// the 5 us of a launch.
+constexpr int64_t kMergeApplyElems = (int64_t)1 << 25;
 
 // Algorithmic bytes of one parameter's step: p r/w, g r, idx r/w per element
 // plus the fp32 state vectors read and written.
@@ -1133,6 +1153,19 @@ static int desc_to_work(const gefenx_tensor_desc& d, int i, const void* const* q
     return build_work(in, w);
 }
 
+// Tensors of the HOT apply join the launch of the others (which takes every
+// tensor, some 8% slower) where they are few: a launch of their own costs ~5 us.
+static void merge_small_applies(std::vector<TensorWork>& works) {
+    for (int dt : {F32, F16, BF16}) {
+        int64_t hot = 0, any = 0;
+        for (const TensorWork& w : works)
+            if (w.dtype == dt) (w.fast_apply == 1 ? hot : any) += (w.fast_apply & 1) ? w.N : 0;
+        if (any == 0 || hot > kMergeApplyElems) continue;
+        for (TensorWork& w : works)
+            if (w.dtype == dt && w.fast_apply == 1) w.fast_apply = 3;
+    }
+}
+
 static int build_layout(const gefenx_tensor_desc* descs, int n, const void* const* qtables, int sr,
                         int64_t seed, const float* const* step_scalars, const int64_t* seed_dev, MtLayout& L) {
     if (n < 0 || (n > 0 && (!descs || !qtables)))
@@ -1149,6 +1182,7 @@ static int build_layout(const gefenx_tensor_desc* descs, int n, const void* cons
         if (rc) return rc;
         works.push_back(w);
     }
+    merge_small_applies(works);
     plan_multi(works, L);
     return GEFENX_OK;
 }

@@ -17,8 +17,9 @@ constexpr int64_t kFinBlocksPerWg = 1024;
 constexpr int64_t kDefaultCohortElems = 0;  // one cohort per step (see cohort_limit)
 constexpr int kTv = 64;                        // transposed views: square tiles of this side
 constexpr int kTvTilesPerWave = 2;             // apply: consecutive tiles per wave
-constexpr int64_t kRowSegCols = 64 * kChunk;   // apply_rows: columns of a task
-constexpr int kRowsPerTask = 8;                // apply_rows: rows of a task
+constexpr int64_t kRowSegCols = 64 * kChunk;   // apply_tasks: most columns of a task
+constexpr int kRowsPerTask = 8;                // apply_tasks: row steps of a task
+constexpr int64_t kSmallApplyElems = 1 << 22;  // ... in launches of at least so many elements, else 2
 constexpr int kDetIters = 8;                   // block stats: items per thread
 // Stats records per block from which the block finalize takes a workgroup per block.
 constexpr int64_t kFinWideRecords = 32;
@@ -57,14 +58,14 @@ struct TensorWork {
     int64_t ct, rt, tile_rows, tile_cols, shards;  // tile_cols: lane tiles and transposed views
     int64_t stats_wgs, nr, nc, nbw, fin_wgs, apply_wgs;
     int64_t det_elems;   // block stats: elements per workgroup
-    int64_t dR, dC, dB, dP;  // apply: chunk advance for a stride of apply_wgs*256*8 elements
-    int64_t fR, fC, fB, fP;  // fast apply: advance for a stride of 256*8 elements
+    int64_t fB, fP;          // flat apply: block advance for a stride of 256*8 elements
+    int64_t a_segs, a_cols;  // apply_tasks: segments per row, columns of a segment
+    int32_t a_lg, a_steps;   // ... log2 lanes per segment, row steps of a task
     uint64_t seed;
     int32_t dtype, mode;
-    int32_t fast_stats, fast_apply;  // kernel variant: 0 general, 1 contiguous, 2 transposed view
+    int32_t fast_stats, fast_apply;  // kernel variant: 0 general, 1 contiguous (apply: HOT), 2 transposed view, 3 apply of any alignment
     int32_t write_p, sr, bf16_mean, det_epl;  // det_epl: block stats elements per item (8 or 1)
     int32_t det_vec;     // block stats items: vector loads (grad 16-byte, indices 8-byte aligned)
-    int32_t row_apply;   // factored contiguous apply over row segments (apply_rows)
     int32_t partial;     // block path with the caller's per-block stepsize (no vmean)
     int32_t fin_wide;    // block finalize: one workgroup per block (blocks span many stats records)
     int32_t lg_lanes;    // factored contiguous stats on lane tiles: log2 lanes per row (stats_lanes), else -1

@@ -56,6 +56,22 @@ CASES = [
     ((64, 512), 8, BF16, "c", {}),
     ((66, 2048), 1, F32, "c", {}),
     ((48, 600), 72, BF16, "t", {}),
+    # apply: segments of any width, chunks that hold a block border, a task's
+    # rows cut by the last row, stochastic rounding, the flat walk's last chunk
+    ((9, 513), 513, BF16, "c", {}),
+    ((17, 1543), 1543 * 17, F16, "o", {}),
+    ((24, 1030), 10, BF16, "c", {}),
+    ((45, 768), 9, F32, "o", {}),
+    ((20, 16392), 16392, BF16, "c", {}),
+    ((33, 1025), 1025, BF16, "c", {"sr": True}),
+    ((50, 40), 8, F32, "c", {"sr": True}),
+    ((64, 1024), 2048, F16, "c", {"sr": True}),
+    ((41, 1031), 1031, BF16, "c", {"factored": False}),
+    ((41, 1031), 1031, F16, "o", {"factored": False, "sr": True}),
+    ((4097 * 9,), 9, F32, "c", {}),
+    ((999,), 27, BF16, "c", {}),
+    ((3047,), 277, F16, "c", {}),
+    ((2048 * 11 + 8,), 8, BF16, "o", {}),
     # fewer than 8 columns: element loads
     ((500, 7), 35, BF16, "c", {}),
 ]
