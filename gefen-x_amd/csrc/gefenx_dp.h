@@ -66,16 +66,14 @@ inline double dp_cost(const double* pw, const double* pwx, const double* pwx2, i
     return swx2 - sq / sw;
 }
 
-// Walk the first-minimum starts back from bin n: the centres are the segment
-// means (forced endpoints -1 / +1), sorted.  bt row c, column end: start of
-// centre c's segment when it ends at `end`.  Returns false when a segment is
-// missing (infeasible).
-inline bool dp_backtrack(const DpPrefix& p, const int32_t* bt, size_t W, int n, int k, int force_endpoints,
-                         float* out) {
+// The centres of the segments path[c] .. (end of centre c), c = k .. 1, from bin
+// n down: segment means (forced endpoints -1 / +1), sorted.  Returns false when
+// a segment is missing (infeasible).
+inline bool dp_centres(const DpPrefix& p, const int32_t* path, int n, int k, int force_endpoints, float* out) {
     std::vector<float> cb((size_t)k);
     int64_t end = n;
     for (int c = k; c >= 1; --c) {
-        const int64_t s = bt[(size_t)c * W + (size_t)end];
+        const int64_t s = path[c];
         if (force_endpoints && c == 1) cb[(size_t)c - 1] = -1.0f;
         else if (force_endpoints && c == k) cb[(size_t)c - 1] = 1.0f;
         else {
@@ -89,6 +87,19 @@ inline bool dp_backtrack(const DpPrefix& p, const int32_t* bt, size_t W, int n, 
     std::sort(cb.begin(), cb.end());
     std::copy(cb.begin(), cb.end(), out);
     return true;
+}
+
+// The same from the first-minimum starts: bt row c, column end is the start of
+// centre c's segment when it ends at `end`.
+inline bool dp_backtrack(const DpPrefix& p, const int32_t* bt, size_t W, int n, int k, int force_endpoints,
+                         float* out) {
+    std::vector<int32_t> path((size_t)k + 1, -1);
+    int64_t end = n;
+    for (int c = k; c >= 1 && end >= 0; --c) {
+        path[(size_t)c] = bt[(size_t)c * W + (size_t)end];
+        end = path[(size_t)c] - 1;
+    }
+    return dp_centres(p, path.data(), n, k, force_endpoints, out);
 }
 
 }  // namespace gx

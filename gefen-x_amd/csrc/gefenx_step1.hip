@@ -413,24 +413,72 @@ __global__ void __launch_bounds__(kT) k_vmean(float* vmean, const void* g, int64
 
 // ---------------------------------------------------------- exact DP
 // Level c of the exact-DP codebook solver (quantization.py:75-139) for every
-// segment end at once: one wave per end, lanes over the segment starts s,
-// each lane keeping its first strict minimum of prev[s-1] + cost(s, end); the
-// wave then takes the (value, start) lexicographic minimum, which is the
-// sequential scan's first minimum.  Costs are the host solver's operations
-// in the same order (dp_cost), so values and choices are bit-identical.
+// segment end at once: one wave per end, the first minimum over the segment
+// starts s of prev[s-1] + cost(s, end).  Costs are the host solver's operations
+// in the same order (dp_cost) and the minimum is the (value, start)
+// lexicographic one, so values and choices are the sequential scan's, bit for
+// bit.
+// Most starts cannot win: prev grows and cost shrinks with s, so no start of a
+// group of 64, s1 .. s2, beats prev[s1-1] + cost(s2, end).  The wave takes this
+// bound for up to 64 groups at a time, one per lane, evaluates the group with
+// the smallest bound, and after it only the groups whose bound does not exceed
+// the best value so far by more than `margin` (rounding: the prefix sums
+// deviate from exact, monotone ones by at most n 2^-53 pw[n] each, a cost by a
+// few times that; the caller passes 2^-38 pw[n], 8 n 2^-53 pw[n] for n = 4096).
+// Every start of every group took 23.6 us a level at n = 4096, this takes 8.8.
 __global__ void __launch_bounds__(kT) k_dp_level(const double* __restrict__ pw, const double* __restrict__ pwx,
                                                 const double* __restrict__ pwx2, const double* __restrict__ prev,
                                                 double* __restrict__ cur, int32_t* __restrict__ bt_row, int c, int n,
-                                                int endpoint, double fc) {
+                                                int endpoint, double fc, double margin) {
     const int lane = threadIdx.x & 63;
     const int64_t w = ((int64_t)blockIdx.x * kT + threadIdx.x) >> 6;
     const int end = c + (int)w;
     if (end > n) return;  // whole waves
-    double best = __builtin_huge_val();
+    double best = __builtin_huge_val();  // of this lane's starts; combined in wave_min
     int best_s = -1;
-    for (int s = c + lane; s <= end; s += 64) {
+    auto wave_min = [&]() {
+        double m = best;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const double o = __shfl_xor(m, off, 64);
+            m = o < m ? o : m;
+        }
+        return m;
+    };
+    auto eval = [&](int grp) {
+        const int s = c + 64 * grp + lane;
+        if (s > end) return;
         const double cand = prev[s - 1] + dp_cost(pw, pwx, pwx2, s, end, endpoint != 0, fc);
-        if (cand < best) { best = cand; best_s = s; }
+        if (cand < best || (cand == best && s < best_s)) { best = cand; best_s = s; }
+    };
+    const int groups = (end - c) / 64 + 1;
+    double top = __builtin_huge_val();  // best value of the wave so far
+    for (int g0 = 0; g0 < groups; g0 += 64) {
+        double lb = __builtin_huge_val();
+        if (g0 + lane < groups) {
+            const int s1 = c + 64 * (g0 + lane);
+            const int s2 = s1 + 63 < end ? s1 + 63 : end;
+            lb = prev[s1 - 1] + dp_cost(pw, pwx, pwx2, s2, end, endpoint != 0, fc);
+        }
+        double m = lb;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) {
+            const double o = __shfl_xor(m, off, 64);
+            m = o < m ? o : m;
+        }
+        const uint64_t low = (uint64_t)__ballot(lb == m && lb < __builtin_huge_val());
+        if (low == 0ull) continue;  // no finite start here
+        const int first = __ffsll((unsigned long long)low) - 1;
+        if (m <= top + margin) {
+            eval(g0 + first);
+            top = wave_min();
+        }
+        uint64_t rest = (uint64_t)__ballot(lb <= top + margin) & ~(1ull << first);
+        while (rest != 0ull) {
+            eval(g0 + __ffsll((unsigned long long)rest) - 1);
+            rest &= rest - 1ull;
+        }
+        top = wave_min();
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
@@ -444,6 +492,21 @@ __global__ void __launch_bounds__(kT) k_dp_level(const double* __restrict__ pw, 
     if (lane == 0) {
         cur[end] = best;
         bt_row[end] = best_s;
+    }
+}
+
+// path[c] = start of centre c's segment (c = k .. 1), walking the choices back
+// from bin n; stops at a missing one.  Rows c of bt hold ends c .. n.
+__global__ void k_dp_path(const int32_t* __restrict__ bt, int64_t W, int n, int k, int32_t* __restrict__ path) {
+    int end = n;
+    for (int c = k; c >= 1; --c) {
+        const int s = end >= c ? bt[(int64_t)c * W + end] : -1;
+        path[c] = s;
+        if (s < 1) {
+            for (int q = c - 1; q >= 1; --q) path[q] = -1;
+            return;
+        }
+        end = s - 1;
     }
 }
 
@@ -638,46 +701,54 @@ int gefenx_exact_dp_device(const float* active_centers, const float* active_coun
     const DpPrefix pre = dp_prefix(active_centers, active_counts, n);
     const size_t W = (size_t)n + 1;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    // device: pw, pwx, pwx2, prev, cur (double [W] each), bt (int32 [k+1][W])
+    // device: pw, pwx, pwx2, prev, cur (double [W] each), bt (int32 [k+1][W]),
+    // path (int32 [k+1]); stream-ordered memory
     const size_t dbytes = sizeof(double) * 5 * W;
     const size_t btbytes = sizeof(int32_t) * (size_t)(k + 1) * W;
     char* dev = nullptr;
-    if (hipMalloc((void**)&dev, dbytes + btbytes) != hipSuccess)
-        return set_error(GEFENX_ENOMEM, "gefenx_exact_dp_device: hipMalloc(%zu) failed", dbytes + btbytes);
+    if (hipMallocAsync((void**)&dev, dbytes + btbytes + sizeof(int32_t) * (size_t)(k + 1), s) != hipSuccess)
+        return set_error(GEFENX_ENOMEM, "gefenx_exact_dp_device: allocation of %zu bytes failed", dbytes + btbytes);
     double* d_pw = reinterpret_cast<double*>(dev);
     double* d_pwx = d_pw + W;
     double* d_pwx2 = d_pwx + W;
     double* d_prev = d_pwx2 + W;
     double* d_cur = d_prev + W;
     int32_t* d_bt = reinterpret_cast<int32_t*>(dev + dbytes);
-    std::vector<double> prev0(W, std::numeric_limits<double>::infinity());
-    prev0[0] = 0.0;
-    std::vector<int32_t> bt((size_t)(k + 1) * W, -1);
+    int32_t* d_path = d_bt + (size_t)(k + 1) * W;
+    // one upload: the three prefix sums and level 0 (only the empty prefix)
+    std::vector<double> up;
+    up.reserve(4 * W);
+    up.insert(up.end(), pre.pw.begin(), pre.pw.end());
+    up.insert(up.end(), pre.pwx.begin(), pre.pwx.end());
+    up.insert(up.end(), pre.pwx2.begin(), pre.pwx2.end());
+    up.push_back(0.0);
+    up.resize(4 * W, std::numeric_limits<double>::infinity());
+    std::vector<int32_t> path((size_t)(k + 1), -1);
+    const double margin = std::ldexp(pre.pw[(size_t)n], -38) * std::max(1.0, (double)n / 4096.0);
     int rc = GEFENX_OK;
-    if (hipMemcpyAsync(d_pw, pre.pw.data(), sizeof(double) * W, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(d_pwx, pre.pwx.data(), sizeof(double) * W, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(d_pwx2, pre.pwx2.data(), sizeof(double) * W, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(d_prev, prev0.data(), sizeof(double) * W, hipMemcpyHostToDevice, s) != hipSuccess ||
-        hipMemcpyAsync(d_bt, bt.data(), btbytes, hipMemcpyHostToDevice, s) != hipSuccess)
+    if (hipMemcpyAsync(d_pw, up.data(), sizeof(double) * 4 * W, hipMemcpyHostToDevice, s) != hipSuccess)
         rc = set_error(GEFENX_ELAUNCH, "gefenx_exact_dp_device: upload failed");
     for (int c = 1; c <= k && rc == GEFENX_OK; ++c) {
-        const int ends = n - c + 1;
-        if (ends > 0) {
-            const bool endpoint = force_endpoints && (c == 1 || c == k);
-            const double fc = (c == 1) ? -1.0 : 1.0;
-            hipLaunchKernelGGL(k_dp_level, dim3((unsigned)(((int64_t)ends * 64 + kT - 1) / kT)), dim3(kT), 0, s,
-                               d_pw, d_pwx, d_pwx2, d_prev, d_cur, d_bt + (size_t)c * W, c, n, endpoint ? 1 : 0, fc);
-            rc = check("exact DP level");
-        }
+        const int ends = n - c + 1;  // > 0: k <= n
+        const bool endpoint = force_endpoints && (c == 1 || c == k);
+        const double fc = (c == 1) ? -1.0 : 1.0;
+        hipLaunchKernelGGL(k_dp_level, dim3((unsigned)(((int64_t)ends * 64 + kT - 1) / kT)), dim3(kT), 0, s,
+                           d_pw, d_pwx, d_pwx2, d_prev, d_cur, d_bt + (size_t)c * W, c, n, endpoint ? 1 : 0, fc, margin);
+        rc = check("exact DP level");
         std::swap(d_prev, d_cur);
     }
-    if (rc == GEFENX_OK && (hipMemcpyAsync(bt.data(), d_bt, btbytes, hipMemcpyDeviceToHost, s) != hipSuccess ||
-                            hipStreamSynchronize(s) != hipSuccess))
+    if (rc == GEFENX_OK) {
+        hipLaunchKernelGGL(k_dp_path, dim3(1), dim3(1), 0, s, d_bt, (int64_t)W, n, k, d_path);
+        rc = check("exact DP path");
+    }
+    if (rc == GEFENX_OK && hipMemcpyAsync(path.data(), d_path, sizeof(int32_t) * (size_t)(k + 1),
+                                          hipMemcpyDeviceToHost, s) != hipSuccess)
         rc = set_error(GEFENX_ELAUNCH, "gefenx_exact_dp_device: download failed");
-    hipStreamSynchronize(s);
-    hipFree(dev);
+    (void)hipFreeAsync(dev, s);
+    if (hipStreamSynchronize(s) != hipSuccess && rc == GEFENX_OK)
+        rc = set_error(GEFENX_ELAUNCH, "gefenx_exact_dp_device: download failed");
     if (rc) return rc;
-    if (!dp_backtrack(pre, bt.data(), W, n, k, force_endpoints, codebook_out))
+    if (!dp_centres(pre, path.data(), n, k, force_endpoints, codebook_out))
         return set_error(GEFENX_EINVAL, "gefenx_exact_dp_device: infeasible segmentation");
     return GEFENX_OK;
 }
