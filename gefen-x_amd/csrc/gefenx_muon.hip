@@ -617,7 +617,14 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const f32x16 (&
     const int tid = threadIdx.x;
 #pragma unroll
     for (int h = 0; h < WM; ++h) {
-        if (wm == h / (WM / 2)) {
+        if constexpr (WM == 1) {  // one slab, both wave rows
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r)
+                    sOut[(wm * 32 + (r >> 2) * 8 + lhi * 4 + (r & 3)) * kOutPitch + wn * (32 * WN) + j * 32 + l32] =
+                        acc[0][j][r];
+        } else if (wm == h / (WM / 2)) {
 #pragma unroll
             for (int ii = 0; ii < 2; ++ii) {
                 const int i = 2 * (h % (WM / 2)) + ii;
@@ -723,6 +730,12 @@ __device__ __forceinline__ int epi_at(int row, int col) {
 template <int WM>
 __device__ __forceinline__ void put_acc32(const f32x16 (&acc)[WM][WM], float* sOut, int h, int wm, int wn, int l32,
                                           int lhi) {
+    if constexpr (WM == 1) {  // one slab, both wave rows
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+            sOut[epi_at<1>(wm * 32 + (r >> 2) * 8 + lhi * 4 + (r & 3), wn * 32 + l32)] = acc[0][0][r];
+        return;
+    } else {
     if (wm != h / (WM / 2)) return;
 #pragma unroll
     for (int ii = 0; ii < 2; ++ii) {
@@ -735,6 +748,7 @@ __device__ __forceinline__ void put_acc32(const f32x16 (&acc)[WM][WM], float* sO
                 const int col = wn * (32 * WM) + j * 32 + l32;
                 sOut[epi_at<WM>(row, col)] = acc[i][j][r];
             }
+    }
     }
 }
 
@@ -979,6 +993,92 @@ __global__ void __launch_bounds__(kT) k_gemm_dl(GemmArgs g) {
     for (int64_t kt = 0; kt < nk; ++kt) {
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): step kt's loads, the only ones in flight
         __syncthreads();  // every wave's loads of step kt landed; step kt-1's buffer is free
+        if (kt + S - 1 < nk)
+            dl_load_stage<TILE, BK>(A, g.lda, g.M, B, g.ldb, g.N, m0, n0, (kt + S - 1) * BK,
+                                    smem + ((kt + S - 1) % S) * kStage);
+        const uint16_t* a_s = smem + (kt % S) * kStage;
+        const uint16_t* b_s = a_s + TILE * BK;
+#pragma unroll
+        for (int ks = 0; ks < BK / 16; ++ks) {
+            const int c = ks * 2 + lhi;
+            bf16x8 av[WM], bv[WM];
+#pragma unroll
+            for (int i = 0; i < WM; ++i) {
+                const int row = wm * (32 * WM) + i * 32 + l32;
+                av[i] = *reinterpret_cast<const bf16x8*>(a_s + row * BK + dl_slot<BK>(row, c) * 8);
+            }
+#pragma unroll
+            for (int j = 0; j < WM; ++j) {
+                const int row = wn * (32 * WM) + j * 32 + l32;
+                bv[j] = *reinterpret_cast<const bf16x8*>(b_s + row * BK + dl_slot<BK>(row, c) * 8);
+            }
+#pragma unroll
+            for (int i = 0; i < WM; ++i)
+#pragma unroll
+                for (int j = 0; j < WM; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[i], bv[j], acc[i][j], 0, 0, 0);
+        }
+    }
+    __syncthreads();
+    if (m0 + TILE <= g.M && n0 + TILE <= g.N && epi_aligned(g.C, g.ldc, g.sC) && epi_aligned(g.D, g.ldd, g.sD) &&
+        epi_aligned(g.Dt, g.lddt, g.sDt)) {
+        float* sOut = reinterpret_cast<float*>(smem);
+        gemm_epilogue_full<WM>(g, [&](int h) { put_acc32<WM>(acc, sOut, h, wm, wn, l32, lhi); }, sOut, bz, tm == tn,
+                               m0, n0);
+    } else
+        gemm_epilogue<WM, WM>(g, acc, reinterpret_cast<float*>(smem), bz, tm == tn, m0, n0, wm, wn, l32, lhi);
+}
+
+// 64 x 64 tiles (WM 1) with a ring of four stages (64 KB of LDS, two
+// workgroups per CU), for grids too small to fill the CUs with 128 x 128 tiles:
+// four times the workgroups, a quarter of the MFMAs in each one's serial chain
+// of K steps, three steps of loads in flight.  The wait at the top of a step
+// leaves the later stages' loads (kL instructions per wave and stage) in
+// flight; the bare barrier keeps the compiler from draining them.  Measured
+// against k_gemm_dl, us: 9 tiles of 128 x 128 (320 x 320, K 320) 13.2 -> 5.8;
+// 49 (1152 x 832, K 832) 19.5 -> 9.8; 133 21.2 -> 12.9; but 136 with K 6144 (a
+// lower triangle of 2048 x 2048) 71 -> 84, twice the operand traffic then
+// being what counts, and 272 42 -> 69.  (128 x 128 tiles in the same ring: no
+// gain, 13.2, 18.8 and 64 us.)
+template <int WM, int BK>
+__global__ void __launch_bounds__(kT) k_gemm_ring(GemmArgs g) {
+    constexpr int S = 4;
+    int64_t bz, tm, tn;
+    if (!gemm_tile(g, bz, tm, tn)) return;  // upper triangle: the mirror of a lower tile
+    constexpr int TILE = 64 * WM;
+    constexpr int kStage = 2 * TILE * BK;         // bf16 per stage: A then B
+    constexpr int kEpi = 2 * 64 * (TILE + 1);     // the epilogue's fp32 slab, in bf16 units
+    constexpr int kSmem = S * kStage > kEpi ? S * kStage : kEpi;
+    constexpr int kL = 2 * (TILE * BK * 2 / 1024) / (kT / 64);  // load instructions per wave and stage
+    __shared__ __attribute__((aligned(16))) uint16_t smem[kSmem];
+    const uint16_t* A = g.A + bz * g.sA;
+    const uint16_t* B = g.B + bz * g.sB;
+    const int64_t m0 = tm * TILE;
+    const int64_t n0 = tn * TILE;
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int wm = wave >> 1, wn = wave & 1;
+    const int l32 = lane & 31, lhi = lane >> 5;
+    f32x16 acc[WM][WM];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WM; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+    const int64_t nk = g.K / BK;
+#pragma unroll
+    for (int st = 0; st < S - 1; ++st)
+        if (st < nk) dl_load_stage<TILE, BK>(A, g.lda, g.M, B, g.ldb, g.N, m0, n0, st * BK, smem + st * kStage);
+#pragma unroll 1
+    for (int64_t kt = 0; kt < nk; ++kt) {
+        const int64_t later = nk - 1 - kt;  // stages after this one; at most two of them are in flight
+        // vmcnt(n) alone: bits 3:0 and 15:14
+        if (later >= 2) __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * kL) & 15) | (((2 * kL) >> 4) << 14));
+        else if (later == 1) __builtin_amdgcn_s_waitcnt(0x0F70 | (kL & 15) | ((kL >> 4) << 14));
+        else __builtin_amdgcn_s_waitcnt(0x0F70);
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        // every wave's loads of step kt landed; step kt-1's buffer is free
         if (kt + S - 1 < nk)
             dl_load_stage<TILE, BK>(A, g.lda, g.M, B, g.ldb, g.N, m0, n0, (kt + S - 1) * BK,
                                     smem + ((kt + S - 1) % S) * kStage);
@@ -1321,8 +1421,9 @@ static int gemm_nt(const GemmArgs& g, int64_t batch, hipStream_t s) {
     // 256 tiles (lower triangle only when symmetric) fill the 256 CUs at least
     // once take a 256 x 256 kernel (16x16x32 MFMAs when every tile is full,
     // the 32x32x16 kernel with its clamped loads and guarded epilogue
-    // otherwise); smaller grids keep 128 x 128 tiles (four times the
-    // workgroups).
+    // otherwise); smaller grids take 128 x 128 tiles (four times the
+    // workgroups), and grids that leave about half of the CUs without one 64 x
+    // 64 tiles.
     const auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool dl = a.vec && g.K % 64 == 0 && al16(g.A) && al16(g.B);
     constexpr int bm = 128, bn = 128;
@@ -1344,7 +1445,12 @@ static int gemm_nt(const GemmArgs& g, int64_t batch, hipStream_t s) {
     a.nt_m = cdiv(g.M, bm);
     a.nt_n = cdiv(g.N, bn);
     const dim3 grid((unsigned)(a.nt_m * a.nt_n * batch));
-    if (dl)
+    const int64_t tiles = (g.tri ? a.nt_m * (a.nt_m + 1) / 2 : a.nt_m * a.nt_n) * batch;
+    if (dl && tiles <= (g.K <= 1024 ? 192 : 128)) {  // k_gemm_ring's comment has both sides
+        a.nt_m = cdiv(g.M, 64);
+        a.nt_n = cdiv(g.N, 64);
+        hipLaunchKernelGGL((k_gemm_ring<1, 64>), dim3((unsigned)(a.nt_m * a.nt_n * batch)), dim3(kT), 0, s, a);
+    } else if (dl)
         hipLaunchKernelGGL((k_gemm_dl<2, 64, 2>), grid, dim3(kT), 0, s, a);
     else if (a.vec)
         hipLaunchKernelGGL((k_gemm_nt<2, 2, 64, true>), grid, dim3(kT), 0, s, a);

@@ -15,7 +15,7 @@ TUNED3 = [(5.0067, -14.4125, 10.6001), (3.7534, -6.8083, 3.3840), (3.2080, -4.35
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("shape", [(1, 9), (63, 65), (64, 64), (65, 129), (130, 40), (200, 333), (511, 257),
-                                   (300, 1030)])
+                                   (300, 1030), (1408, 1409), (1700, 900)])
 def test_shapes_around_the_padding(shape, dtype):
     if not torch.cuda.is_available():
         pytest.skip("no HIP device")
