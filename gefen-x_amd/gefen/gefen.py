@@ -26,10 +26,13 @@ same kernels, bit for bit as if it lived on the device.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
+import functools
 import logging
 import math
 import os
+import struct
 import warnings
 import weakref
 from collections import OrderedDict
@@ -71,8 +74,25 @@ _CAPT_PLAN_CACHE = 4
 
 _LR_DTYPE_CODES = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2, torch.float64: 3}
 
-# numpy image of gefenx_tensor_desc (field order and offsets of the C struct)
+# numpy image of gefenx_tensor_desc (field order and offsets of the C struct),
+# and the same as a struct format, for packing one descriptor at a time
 _DESC_DTYPE = np.dtype(_native.TensorDesc)
+_DESC_STRUCT = struct.Struct("<" + "".join({"c_void_p": "Q", "c_long": "q", "c_int": "i", "c_float": "f"}[t.__name__]
+                                           for _, t in _native.TensorDesc._fields_))
+_DESC_BYTES = ctypes.sizeof(_native.TensorDesc)
+_STEP_DTYPES = frozenset((torch.float32, torch.float16, torch.bfloat16))
+
+
+@functools.lru_cache(maxsize=4096)
+def _workspace_bytes(kind: int, rows: int, cols: int, nb: int) -> int:
+    return int(_native.load().gefenx_workspace_bytes(kind, rows, cols, nb))
+
+
+def _on_device(device):
+    """torch.cuda.device(device), or nothing where it is the current one."""
+    if device.index == torch.cuda.current_device():
+        return contextlib.nullcontext()
+    return torch.cuda.device(device)
 
 
 def automatic_partition_view(flat_tensor: torch.Tensor, period: int) -> torch.Tensor:
@@ -659,6 +679,10 @@ class Gefen(torch.optim.Optimizer):
                 g = p.grad
                 if g is None:
                     continue
+                dt, dev = p.dtype, p.device
+                if (g.dtype is dt and dt in _STEP_DTYPES and g.layout is torch.strided and g.shape == p.shape
+                        and g.device == dev and dev.type == "cuda"):
+                    continue  # every check below holds
                 if getattr(g, "is_sparse", False) or g.layout != torch.strided:
                     raise RuntimeError("Gefen does not support sparse gradients")
                 if torch.is_complex(g):
@@ -771,7 +795,7 @@ class Gefen(torch.optim.Optimizer):
 
     def _workspace(self, state, kind, rows, cols, nb, device):
         ws = state.get("_gefenx_ws")
-        need = int(_native.load().gefenx_workspace_bytes(kind, rows, cols, nb))
+        need = _workspace_bytes(kind, rows, cols, nb)
         if ws is None or ws.numel() < need or ws.device != device:
             ws = torch.zeros(max(need, 256), dtype=torch.uint8, device=device)
             state["_gefenx_ws"] = ws
@@ -939,20 +963,27 @@ class Gefen(torch.optim.Optimizer):
         (stats, finalize and apply phases each launched once per kernel
         variant instead of once per parameter)."""
         lib = _native.load()
-        descs = np.array(rows, dtype=_DESC_DTYPE)
+        n = len(rows)
+        descs = bytearray(n * _DESC_BYTES)
+        try:
+            for i, row in enumerate(rows):
+                _DESC_STRUCT.pack_into(descs, i * _DESC_BYTES, *row)
+        except OverflowError:  # a scalar beyond fp32: infinite, as a cast makes it
+            with np.errstate(over="ignore"):
+                descs = bytearray(np.array(rows, dtype=_DESC_DTYPE).tobytes())
         cb = self._gefen_codebook_on(device)
         qt = [0, 0, 0]
         for dt in dtypes:
             qt[_fused._dtype_code(dt)] = _fused.quant_table(cb, dt).data_ptr()
         qt_arr = (ctypes.c_void_p * 3)(*qt)
-        need = int(lib.gefenx_multi_tensor_scratch_bytes(len(rows)))
+        need = int(lib.gefenx_multi_tensor_scratch_bytes(n))
         scratch = self._mt_scratch.get(device)
         if scratch is None or scratch.numel() < need:
             scratch = torch.empty(need, dtype=torch.uint8, device=device)
             self._mt_scratch[device] = scratch
-        with torch.cuda.device(device):
+        with _on_device(device):
             _native.check(lib.gefenx_multi_tensor_step(
-                descs.ctypes.data, len(rows), qt_arr, 1 if self._stochastic_round else 0,
+                ctypes.addressof(ctypes.c_char.from_buffer(descs)), n, qt_arr, 1 if self._stochastic_round else 0,
                 self._gefen_global_step, scratch.data_ptr(), scratch.numel(),
                 torch.cuda.current_stream(device).cuda_stream), "multi-tensor step")
 
@@ -1159,7 +1190,8 @@ class Gefen(torch.optim.Optimizer):
                 grad = p.grad
                 if grad is None or grad.numel() == 0:
                     continue
-                factored = self._factored_v_2d and p.ndim == 2 and not hasattr(p, "placements")
+                factored = (self._factored_v_2d and p.ndim == 2
+                            and (type(p) is nn.Parameter or not hasattr(p, "placements")))
                 if capturing and "step" not in self.state[p]:
                     raise RuntimeError("Gefen capturable: parameter {} has no state yet; its first step runs "
                                        "eagerly".format(name))
