@@ -72,7 +72,10 @@ inline bool lane_tiles(int64_t cols, int64_t period) {
     return cols >= 8 && (cols <= kNarrowMaxCols || (period < kShortPeriod && period < cols));
 }
 
-// As launch_elems: the largest tiles whatever the launch.
+// As launch_elems: the largest tiles whatever the launch, for the scratch of
+// fixed size.  Short blocks of wide matrices then stay on 1024-column tiles: the
+// twice as many row partials of the lane tiles would take shapes out of it
+// (21920 x 21920 in 512-element blocks 30.3 -> 34.0 MB of 33.6).
 constexpr int64_t kCoarseTiles = (int64_t)1 << 62;
 
 // Transposed-view stats (strides (1, ld)): tiles of up to four 64-row bands,
@@ -110,7 +113,7 @@ struct FactTiles {
         t.lg_lanes = -1;
         t.ct_l = t.rt_l = 0;
         t.l_rows = t.l_cols = 0;
-        if (lane_tiles(cols, period)) {
+        if (lane_tiles(cols, period) && (cols <= kNarrowMaxCols || launch_elems < kCoarseTiles)) {
             t.l_cols = (ceil_div(cols, ceil_div(cols, kLaneTileCols)) + 7) & ~int64_t(7);  // even column tiles
             t.lg_lanes = 0;
             while ((8 << t.lg_lanes) < t.l_cols) ++t.lg_lanes;

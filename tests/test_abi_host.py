@@ -256,6 +256,24 @@ def test_noalloc_rejects_shapes_beyond_the_static_scratch(lib):
     assert "static scratch" in _native.last_error()
 
 
+@pytest.mark.parametrize("rows,cols,period", [(21920, 21920, 512), (1408, 100720, 64), (233004, 608, 64)])
+def test_noalloc_takes_short_blocks_up_to_the_static_scratch(lib, rows, cols, period):
+    """Short blocks of wide matrices whose 1024-column row partials fit the
+    static scratch pass the size check (the tiles of short blocks in a
+    workspace would need more than it holds).  The call that passes the check
+    ends at its first HIP call, so this runs without a device only."""
+    import torch
+    from gefen.kernels import _native
+    if torch.cuda.is_available():
+        pytest.skip("the pointers are not real")
+    fake = 4096
+    rc = lib.gefenx_factored_update_noalloc(fake, fake, _native.DT_BF16, rows, cols, cols, 1, cols, 1,
+                                            fake, fake, fake, fake, period, fake, 0.9, 0.999, 1e-3, 1e-8, 1.0,
+                                            1.0, 1.0, 0, 0, None, None, None)
+    assert rc != _native.GEFENX_EINVAL
+    assert "static scratch" not in _native.last_error()
+
+
 def test_gemm_rejects_empty_contraction_before_any_launch(lib):
     """K == 0 is refused on the host (the kernels read the first K step of A
     and B before their loop); here on a machine without a GPU the call
