@@ -422,10 +422,9 @@ __global__ void __launch_bounds__(kT) k_vmean(float* vmean, const void* g, int64
 // group of 64, s1 .. s2, beats prev[s1-1] + cost(s2, end).  The wave takes this
 // bound for up to 64 groups at a time, one per lane, evaluates the group with
 // the smallest bound, and after it only the groups whose bound does not exceed
-// the best value so far by more than `margin` (rounding: the prefix sums
-// deviate from exact, monotone ones by at most n 2^-53 pw[n] each, a cost by a
-// few times that; the caller passes 2^-38 pw[n], 8 n 2^-53 pw[n] for n = 4096).
-// Every start of every group took 23.6 us a level at n = 4096, this takes 8.8.
+// the best value so far by more than `margin`, which covers what rounding may
+// take from these two orders (dp_margin).  Every start of every group took
+// 23.6 us a level at n = 4096, this takes 8.8.
 __global__ void __launch_bounds__(kT) k_dp_level(const double* __restrict__ pw, const double* __restrict__ pwx,
                                                 const double* __restrict__ pwx2, const double* __restrict__ prev,
                                                 double* __restrict__ cur, int32_t* __restrict__ bt_row, int c, int n,
@@ -453,7 +452,9 @@ __global__ void __launch_bounds__(kT) k_dp_level(const double* __restrict__ pw, 
     };
     const int groups = (end - c) / 64 + 1;
     double top = __builtin_huge_val();  // best value of the wave so far
-    for (int g0 = 0; g0 < groups; g0 += 64) {
+    if (!(margin < __builtin_huge_val())) {
+        for (int grp = 0; grp < groups; ++grp) eval(grp);
+    } else for (int g0 = 0; g0 < groups; g0 += 64) {
         double lb = __builtin_huge_val();
         if (g0 + lane < groups) {
             const int s1 = c + 64 * (g0 + lane);
@@ -508,6 +509,25 @@ __global__ void k_dp_path(const int32_t* __restrict__ bt, int64_t W, int n, int 
         }
         end = s - 1;
     }
+}
+
+// Margin of k_dp_level.  With d = n 2^-53 sum w max(1, x^2), which bounds what a
+// prefix sum deviates from its exact value, a cost deviates by a few d, and so
+// does prev: the deviations of its segments' costs telescope over the segment
+// ends to d times the total variation of the means, at most 2 max |x| while the
+// centres ascend.  That takes weights well above d (the squared deviation of
+// sum w x is divided by a segment's weight).  Other inputs take every start.
+static double dp_margin(const float* centers, const float* counts, int n, double total) {
+    double top = 1.0, least = std::numeric_limits<double>::infinity();
+    bool ascending = true;
+    for (int i = 0; i < n; ++i) {
+        const double x = (double)centers[i];
+        top = std::max(top, x * x);
+        least = std::min(least, (double)counts[i]);
+        ascending = ascending && x - x == 0.0 && (i == 0 || centers[i - 1] <= centers[i]);
+    }
+    const double d = std::ldexp((double)n * total * top, -53);
+    return ascending && 16.0 * d <= least ? 32.0 * d : std::numeric_limits<double>::infinity();
 }
 
 static int grid_cap(int64_t items, int per, int cap) {
@@ -724,7 +744,7 @@ int gefenx_exact_dp_device(const float* active_centers, const float* active_coun
     up.push_back(0.0);
     up.resize(4 * W, std::numeric_limits<double>::infinity());
     std::vector<int32_t> path((size_t)(k + 1), -1);
-    const double margin = std::ldexp(pre.pw[(size_t)n], -38) * std::max(1.0, (double)n / 4096.0);
+    const double margin = dp_margin(active_centers, active_counts, n, pre.pw[(size_t)n]);
     int rc = GEFENX_OK;
     if (hipMemcpyAsync(d_pw, up.data(), sizeof(double) * 4 * W, hipMemcpyHostToDevice, s) != hipSuccess)
         rc = set_error(GEFENX_ELAUNCH, "gefenx_exact_dp_device: upload failed");

@@ -93,6 +93,41 @@ def test_device_exact_dp_matches_host_and_golden(dev):
                                   quantization.exact_dp(st, 256, True).numpy(), err_msg="ties")
 
 
+@pytest.mark.parametrize("name", ["spread", "unsorted", "wide", "fractions"])
+def test_device_exact_dp_on_any_histogram(dev, name):
+    """The device solver leaves out starts by bounds that rest on ascending
+    centres and on weights above the prefix sums' rounding; histograms without
+    these (weights over 31 decades, centres in any order) take every start,
+    and bit for bit the host solver's choices."""
+    from gefen import quantization
+    rng = np.random.default_rng(11)
+    n, k = 700, 40
+    grid = (np.arange(4096) + 0.5) / 2048 - 1
+    c, w = np.sort(rng.choice(grid, n, replace=False)), np.floor(rng.pareto(1.2, n) * 50 + 1)
+    if name == "spread":
+        w = 10.0 ** rng.uniform(-25, 6, n)
+    elif name == "unsorted":
+        c = rng.permutation(c)
+    elif name == "wide":
+        c = np.sort(rng.normal(0, 1e6, n))
+    else:
+        w = rng.uniform(1e-3, 1, n)
+    st = {"active_centers": torch.from_numpy(c.astype(np.float32)),
+          "active_counts": torch.from_numpy(w.astype(np.float32))}
+    for force in (False, True):
+        results = []
+        for device in (None, dev):
+            try:
+                results.append(quantization.exact_dp(st, k, force, device=device).numpy())
+            except (RuntimeError, ValueError) as e:  # no finite segmentation: both refuse it
+                results.append(type(e))
+        host, devr = results
+        if isinstance(host, type) or isinstance(devr, type):
+            assert host is devr
+        else:
+            np.testing.assert_array_equal(devr, host)
+
+
 def test_period_search_matches_reference_golden(dev):
     from gefen import partitioning
     z = np.load(os.path.join(GOLD, "period.npz"))
