@@ -526,27 +526,50 @@ struct GemmArgs {
 // tiles, and order the tiles of a matrix in bands of kGroupM tile rows,
 // column by column inside a band.  The ~32 tiles an XCD holds at once then
 // read kGroupM A panels and ~32/kGroupM B panels per K step, instead of
-// tiles scattered over the whole grid.  Returns false for the upper-triangle
-// tiles of a symmetric product (their values are the lower tiles' mirrors).
+// tiles scattered over the whole grid.  A symmetric product counts its lower
+// triangle only (the rest are mirrors): with all tiles counted and the upper
+// ones left at once, the XCDs' ranges held 10 to 122 of the 528 live tiles of
+// 32 x 32, and the fullest set the time.
 constexpr int64_t kXcds = 8;
 constexpr int64_t kGroupM = 4;
 
-__device__ __forceinline__ bool gemm_tile(const GemmArgs& g, int64_t& bz, int64_t& tm, int64_t& tn) {
-    const int64_t T = g.nt_m * g.nt_n * g.batch;
+// Tiles of one matrix.
+__host__ __device__ inline int64_t gemm_tiles(int64_t nt_m, int64_t nt_n, int tri) {
+    return tri ? nt_m * (nt_m + 1) / 2 : nt_m * nt_n;
+}
+
+__device__ __forceinline__ void gemm_tile(const GemmArgs& g, int64_t& bz, int64_t& tm, int64_t& tn) {
+    const int64_t per = gemm_tiles(g.nt_m, g.nt_n, g.tri);
+    const int64_t T = per * g.batch;
     const int64_t wid = blockIdx.x;
     const int64_t q = T / kXcds, r = T % kXcds;
     const int64_t x = wid % kXcds;
     const int64_t L = x * q + (x < r ? x : r) + wid / kXcds;
-    const int64_t per = g.nt_m * g.nt_n;
     bz = L / per;
-    const int64_t t = L - bz * per;
-    const int64_t band = g.nt_n * kGroupM;
-    const int64_t m0 = (t / band) * kGroupM;
+    int64_t t = L - bz * per;
+    int64_t m0 = 0;  // first row of the band
+    if (g.tri) {     // kGroupM rows from m0: m0 + 1 tiles in the first, one more in each that follows
+        for (;;) {
+            const int64_t in_band = kGroupM * m0 + kGroupM * (kGroupM + 1) / 2;
+            if (t < in_band || m0 + kGroupM >= g.nt_m) break;
+            t -= in_band;
+            m0 += kGroupM;
+        }
+    } else {
+        const int64_t b = t / (g.nt_n * kGroupM);
+        m0 = b * kGroupM;
+        t -= b * (g.nt_n * kGroupM);
+    }
     const int64_t gm = g.nt_m - m0 < kGroupM ? g.nt_m - m0 : kGroupM;
-    const int64_t tin = t - (t / band) * band;
-    tm = m0 + tin % gm;
-    tn = tin / gm;
-    return !(g.tri && tn > tm);
+    tm = m0 + t % gm;
+    tn = t / gm;
+    if (g.tri && tn > m0) {  // past the columns that all rows of the band hold: column m0 + c has rows c ..
+        t -= gm * (m0 + 1);
+        int64_t c = 1;
+        while (t >= gm - c) { t -= gm - c; ++c; }
+        tn = m0 + c;
+        tm = m0 + c + t;
+    }
 }
 
 __device__ __forceinline__ float bf16f(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
@@ -850,7 +873,7 @@ __global__ void __launch_bounds__(kT) k_gemm_nt(GemmArgs g) {
     uint16_t (*sB)[BN * kPitch] = reinterpret_cast<uint16_t (*)[BN * kPitch]>(smem + sizeof(uint16_t) * 2 * BM * kPitch);
     float* sOut = reinterpret_cast<float*>(smem);
     int64_t bz, tm, tn;
-    if (!gemm_tile(g, bz, tm, tn)) return;  // upper triangle: the mirror of a lower tile
+    gemm_tile(g, bz, tm, tn);
     const uint16_t* A = g.A + bz * g.sA;
     const uint16_t* B = g.B + bz * g.sB;
     const int64_t m0 = tm * BM;
@@ -965,7 +988,7 @@ template <int WM, int BK, int S>
 __global__ void __launch_bounds__(kT) k_gemm_dl(GemmArgs g) {
     static_assert(S == 2, "two-stage ring: the loop waits for every load in flight at each step");
     int64_t bz, tm, tn;
-    if (!gemm_tile(g, bz, tm, tn)) return;  // upper triangle: the mirror of a lower tile
+    gemm_tile(g, bz, tm, tn);
     constexpr int TILE = 64 * WM;
     constexpr int kStage = 2 * TILE * BK;                        // bf16 per stage: A then B
     constexpr int kEpi = 2 * 64 * (TILE + 1);                    // the epilogue's fp32 slab, in bf16 units
@@ -1044,7 +1067,7 @@ template <int WM, int BK>
 __global__ void __launch_bounds__(kT) k_gemm_ring(GemmArgs g) {
     constexpr int S = 4;
     int64_t bz, tm, tn;
-    if (!gemm_tile(g, bz, tm, tn)) return;  // upper triangle: the mirror of a lower tile
+    gemm_tile(g, bz, tm, tn);
     constexpr int TILE = 64 * WM;
     constexpr int kStage = 2 * TILE * BK;         // bf16 per stage: A then B
     constexpr int kEpi = 2 * 64 * (TILE + 1);     // the epilogue's fp32 slab, in bf16 units
@@ -1160,7 +1183,7 @@ __device__ __forceinline__ void dl_load_one(const uint16_t* __restrict__ A, int6
 __global__ void __launch_bounds__(kT) k_gemm_big(GemmArgs g) {
     constexpr int WM = 4, TILE = 256, BK = 64, KS = BK / 16;
     int64_t bz, tm, tn;
-    if (!gemm_tile(g, bz, tm, tn)) return;  // upper triangle: the mirror of a lower tile
+    gemm_tile(g, bz, tm, tn);
     constexpr int kStage = 2 * TILE * BK;
     constexpr int kIpw = 2 * (TILE * BK * 2 / 1024) / (kT / 64);  // 16 load instructions per wave and stage
     constexpr int kLoadKs = 2;
@@ -1306,7 +1329,7 @@ __device__ __forceinline__ void put_acc16(const f32x16 (&acc4)[8][2], float* sOu
 __global__ void __launch_bounds__(kT) k_gemm_big16(GemmArgs g) {
     constexpr int TILE = 256, BK = 64;
     int64_t bz, tm, tn;
-    if (!gemm_tile(g, bz, tm, tn)) return;  // upper triangle: the mirror of a lower tile
+    gemm_tile(g, bz, tm, tn);
     constexpr int kStage = 2 * TILE * BK;
     constexpr int kIpw = 2 * (TILE * BK * 2 / 1024) / (kT / 64);  // 16 load instructions per wave and stage
     constexpr int kEpi = 2 * 64 * (TILE + 1);
@@ -1432,24 +1455,24 @@ static int gemm_nt(const GemmArgs& g, int64_t batch, hipStream_t s) {
                          (long long)g.M, (long long)g.N, (long long)batch);
     a.batch = batch;
     const int64_t t256m = cdiv(g.M, 256), t256n = cdiv(g.N, 256);
-    const int64_t big_tiles = (g.tri ? t256m * (t256m + 1) / 2 : t256m * t256n) * batch;
+    const int64_t big_tiles = gemm_tiles(t256m, t256n, g.tri) * batch;
     if (dl && big_tiles >= 256) {
         a.nt_m = t256m;
         a.nt_n = t256n;
         const bool full = g.M % 256 == 0 && g.N % 256 == 0 && epi_aligned(g.C, g.ldc, g.sC) &&
                           epi_aligned(g.D, g.ldd, g.sD) && epi_aligned(g.Dt, g.lddt, g.sDt);
-        if (full) hipLaunchKernelGGL(k_gemm_big16, dim3((unsigned)(t256m * t256n * batch)), dim3(kT), 0, s, a);
-        else hipLaunchKernelGGL(k_gemm_big, dim3((unsigned)(t256m * t256n * batch)), dim3(kT), 0, s, a);
+        if (full) hipLaunchKernelGGL(k_gemm_big16, dim3((unsigned)big_tiles), dim3(kT), 0, s, a);
+        else hipLaunchKernelGGL(k_gemm_big, dim3((unsigned)big_tiles), dim3(kT), 0, s, a);
         return launch_check("newton-schulz gemm");
     }
     a.nt_m = cdiv(g.M, bm);
     a.nt_n = cdiv(g.N, bn);
-    const dim3 grid((unsigned)(a.nt_m * a.nt_n * batch));
-    const int64_t tiles = (g.tri ? a.nt_m * (a.nt_m + 1) / 2 : a.nt_m * a.nt_n) * batch;
+    const int64_t tiles = gemm_tiles(a.nt_m, a.nt_n, g.tri) * batch;
+    const dim3 grid((unsigned)tiles);
     if (dl && tiles <= (g.K <= 1024 ? 192 : 128)) {  // k_gemm_ring's comment has both sides
         a.nt_m = cdiv(g.M, 64);
         a.nt_n = cdiv(g.N, 64);
-        hipLaunchKernelGGL((k_gemm_ring<1, 64>), dim3((unsigned)(a.nt_m * a.nt_n * batch)), dim3(kT), 0, s, a);
+        hipLaunchKernelGGL((k_gemm_ring<1, 64>), dim3((unsigned)(gemm_tiles(a.nt_m, a.nt_n, g.tri) * batch)), dim3(kT), 0, s, a);
     } else if (dl)
         hipLaunchKernelGGL((k_gemm_dl<2, 64, 2>), grid, dim3(kT), 0, s, a);
     else if (a.vec)
