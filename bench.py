@@ -80,7 +80,7 @@ def fill_grads(torch, params, step_seed, device):
 
 
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "gefen_step_llama3_8b_traffic.json")
-APPLY_KERNEL = "k_mt_apply<2, 0, false, true>"  # bf16, factored, nearest rounding, contiguous fast path
+APPLY_KERNEL = "k_mt_apply<2, 0, false, 1>"  # bf16, factored, nearest rounding, contiguous fast path
 KERNEL_SOURCES = ("gefenx_update.hip", "gefenx_step_kernels.h", "gefenx_work.h", "gefenx_device.h", "gefenx_common.h")
 
 
