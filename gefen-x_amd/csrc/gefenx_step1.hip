@@ -38,6 +38,20 @@ constexpr int64_t kThreadPeriod = 64;   // below: a thread per block
 constexpr int64_t kGroupPeriod = 512;   // below: 8 lanes per block; from here a wave per block
 constexpr int64_t kSeg = 65536;  // elements per workgroup segment of a large block
 constexpr int kVarGrid = 2048;   // workgroups (and partials) per small-period pass
+constexpr int kVarBatch = 32;    // candidate periods per launch
+
+// The candidates of one launch.  A pass over a few million elements takes no
+// longer than its launch, and large blocks leave most CUs without a segment
+// (64 workgroups for 4M elements), so candidates share launches; each one's
+// sums are those of a launch of its own.  First step of a layer of hidden
+// size 2048 (nine tensors, 22 to 24 candidates each): 8.0 -> 6.05 ms.
+struct VarPeriods {
+    int64_t P[kVarBatch], nb[kVarBatch];
+    int64_t first[kVarBatch];  // k_var_seg: first workgroup
+    int64_t off[kVarBatch];    // k_var_seg, k_var_finish: first block sum
+    int32_t slot[kVarBatch];   // index among the caller's periods
+    int32_t n;
+};
 
 __device__ __forceinline__ void var_partial(double acc, double* part) {
     __shared__ double sh[kT / 64];
@@ -69,9 +83,11 @@ struct VarTile {
 };
 
 template <int DT, bool SQ = true>
-__global__ void __launch_bounds__(kT) k_var_tile(const void* g, int64_t nb, int64_t P, double* part) {
+__global__ void __launch_bounds__(kT) k_var_tile(const void* g, VarPeriods vp, double* parts) {
     using T = typename Elem<DT>::T;
     using VT = VarTile<DT>;
+    const int64_t nb = vp.nb[blockIdx.y], P = vp.P[blockIdx.y];
+    double* part = parts + (int64_t)vp.slot[blockIdx.y] * kVarGrid;
     __shared__ T sx[kVarTile + kVarTile / 2];
     const T* gt = static_cast<const T*>(g);
     const int Pi = (int)P;
@@ -213,12 +229,17 @@ __global__ void __launch_bounds__(64) k_var_sum(const double* part, int n, doubl
 // Segments whose start is 16-byte aligned and whose length is a multiple of
 // 8 read 8 elements per load (two loads in flight per thread).
 template <int DT, bool SQ = true>
-__global__ void __launch_bounds__(kT) k_var_seg(const void* g, int64_t P, int64_t segs_per_block,
-                                               double* s1, double* s2) {
+__global__ void __launch_bounds__(kT) k_var_seg(const void* g, VarPeriods vp, double* sums1, double* sums2) {
     using T = typename Elem<DT>::T;
     __shared__ double sh[2][kT / 64];
-    const int64_t b = (int64_t)blockIdx.x / segs_per_block;
-    const int64_t sg = (int64_t)blockIdx.x - b * segs_per_block;
+    int at = 0;
+    while (at + 1 < vp.n && (int64_t)blockIdx.x >= vp.first[at + 1]) ++at;
+    const int64_t P = vp.P[at], segs_per_block = (P + kSeg - 1) / kSeg;
+    double* s1 = sums1 + vp.off[at];
+    double* s2 = sums2 + vp.off[at];
+    const int64_t wg = (int64_t)blockIdx.x - vp.first[at];
+    const int64_t b = wg / segs_per_block;
+    const int64_t sg = wg - b * segs_per_block;
     const int64_t lo = b * P + sg * kSeg;
     const int64_t hi = std::min<int64_t>(lo + kSeg, (b + 1) * P);
     double a1 = 0.0, a2 = 0.0, c1 = 0.0, c2 = 0.0;
@@ -267,8 +288,11 @@ __global__ void __launch_bounds__(kT) k_var_seg(const void* g, int64_t P, int64_
     }
 }
 
-__global__ void __launch_bounds__(kT) k_var_finish(double* s1, double* s2, int64_t nb, int64_t P,
-                                                  double* total) {
+__global__ void __launch_bounds__(kT) k_var_finish(double* sums1, double* sums2, VarPeriods vp, double* totals) {
+    const int64_t nb = vp.nb[blockIdx.y], P = vp.P[blockIdx.y];
+    double* s1 = sums1 + vp.off[blockIdx.y];
+    double* s2 = sums2 + vp.off[blockIdx.y];
+    double* total = totals + vp.slot[blockIdx.y];
     double acc = 0.0;
     const double fP = (double)P;
     for (int64_t b = (int64_t)blockIdx.x * kT + threadIdx.x; b < nb; b += (int64_t)gridDim.x * kT) {
@@ -581,50 +605,79 @@ int gefenx_block_variance_errors_ex(const void* grad, int dtype, int64_t numel, 
     if (!grad || !periods || !err_host || numel <= 0 || n_periods < 0)
         return set_error(GEFENX_EINVAL, "gefenx_block_variance_errors: bad arguments");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    int64_t max_nb = 0;
     for (int i = 0; i < n_periods; ++i) {
         const int64_t P = periods[i];
         if (P <= 0 || numel % P != 0)
             return set_error(GEFENX_EINVAL, "period %lld does not divide numel %lld", (long long)P, (long long)numel);
-        if (P > kWavePeriod) max_nb = std::max<int64_t>(max_nb, numel / P);
+    }
+    // batches of up to kVarBatch candidates: blocks of at most kWavePeriod
+    // elements by tiles, larger ones by segments
+    std::vector<VarPeriods> tiled, segmented;
+    std::vector<int64_t> wgs;  // of each segmented batch
+    int64_t sums = 0;          // most block sums of a segmented batch
+    int64_t used = 0;          // of the present one
+    for (int i = 0; i < n_periods; ++i) {
+        const int64_t P = periods[i], nb = numel / P;
+        if (P == 1) continue;  // single-element blocks have zero variance
+        std::vector<VarPeriods>& to = P <= kWavePeriod ? tiled : segmented;
+        const int64_t need = nb * ((P + kSeg - 1) / kSeg);
+        if (to.empty() || to.back().n == kVarBatch || (P > kWavePeriod && wgs.back() + need > 2147483647LL)) {
+            to.emplace_back();
+            to.back().n = 0;
+            if (P > kWavePeriod) {
+                wgs.push_back(0);
+                used = 0;
+            }
+        }
+        VarPeriods& v = to.back();
+        v.P[v.n] = P;
+        v.nb[v.n] = nb;
+        v.slot[v.n] = i;
+        v.first[v.n] = v.off[v.n] = 0;
+        if (P > kWavePeriod) {
+            v.first[v.n] = wgs.back();
+            v.off[v.n] = used;
+            wgs.back() += need;
+            used += nb;
+            sums = std::max(sums, used);
+        }
+        ++v.n;
     }
     // [n_periods] totals, [n_periods][kVarGrid] small-period partials (zero
-    // where a pass uses fewer workgroups), then 2 * max_nb block sums
+    // where a pass uses fewer workgroups), then 2 * sums block sums; stream-ordered memory
     double* dev = nullptr;
     const int64_t n_part = (int64_t)n_periods * kVarGrid;
-    const size_t bytes = sizeof(double) * ((size_t)n_periods + (size_t)n_part + 2 * (size_t)max_nb + 1);
-    if (hipMalloc(&dev, bytes) != hipSuccess)
-        return set_error(GEFENX_ENOMEM, "gefenx_block_variance_errors: hipMalloc(%zu) failed", bytes);
+    const size_t bytes = sizeof(double) * ((size_t)n_periods + (size_t)n_part + 2 * (size_t)sums + 1);
+    if (hipMallocAsync((void**)&dev, bytes, s) != hipSuccess)
+        return set_error(GEFENX_ENOMEM, "gefenx_block_variance_errors: allocation of %zu bytes failed", bytes);
     double* totals = dev;
     double* part = dev + n_periods;
     double* s1 = part + n_part;
-    double* s2 = s1 + max_nb;
-    const int64_t fill = (int64_t)n_periods + n_part + 2 * max_nb;
+    double* s2 = s1 + sums;
+    const int64_t fill = (int64_t)n_periods + n_part + 2 * sums;
     hipLaunchKernelGGL(k_zero_f64, dim3(grid_cap(fill, kT, 4096)), dim3(kT), 0, s, dev, fill);
-    bool any_small = false;
-    for (int i = 0; i < n_periods && rc == GEFENX_OK; ++i) {
-        const int64_t P = periods[i];
-        const int64_t nb = numel / P;
-        if (P == 1) continue;  // single-element blocks have zero variance
-        double* pi = part + (int64_t)i * kVarGrid;
-        if (P <= kWavePeriod) {
-            const int64_t tiles = (nb + kVarTile / P - 1) / (kVarTile / P);
-            if (input_is_squared)
-                GX_DISPATCH_SQ(dtype, k_var_tile, dim3(grid_cap(tiles, 1, kVarGrid)), dim3(kT), s, grad, nb, P, pi);
-            else
-                GX_DISPATCH(dtype, k_var_tile, dim3(grid_cap(tiles, 1, kVarGrid)), dim3(kT), s, grad, nb, P, pi);
-            any_small = true;
-        } else {
-            const int64_t spb = (P + kSeg - 1) / kSeg;
-            if (input_is_squared)
-                GX_DISPATCH_SQ(dtype, k_var_seg, dim3((unsigned)(nb * spb)), dim3(kT), s, grad, P, spb, s1, s2);
-            else
-                GX_DISPATCH(dtype, k_var_seg, dim3((unsigned)(nb * spb)), dim3(kT), s, grad, P, spb, s1, s2);
-            hipLaunchKernelGGL(k_var_finish, dim3(grid_cap(nb, kT, 4096)), dim3(kT), 0, s, s1, s2, nb, P, totals + i);
+    for (const VarPeriods& v : tiled) {
+        int grid = 1;
+        for (int i = 0; i < v.n; ++i) {
+            const int64_t per = kVarTile / v.P[i];
+            grid = std::max(grid, grid_cap(v.nb[i], (int)per, kVarGrid));
         }
-        rc = check("block variance");
+        const dim3 g2((unsigned)grid, (unsigned)v.n);
+        if (input_is_squared) GX_DISPATCH_SQ(dtype, k_var_tile, g2, dim3(kT), s, grad, v, part);
+        else GX_DISPATCH(dtype, k_var_tile, g2, dim3(kT), s, grad, v, part);
+        if (rc == GEFENX_OK) rc = check("block variance");
     }
-    if (rc == GEFENX_OK && any_small && n_periods > 0) {
+    for (size_t k = 0; k < segmented.size(); ++k) {
+        const VarPeriods& v = segmented[k];
+        const dim3 gs((unsigned)wgs[k]);
+        if (input_is_squared) GX_DISPATCH_SQ(dtype, k_var_seg, gs, dim3(kT), s, grad, v, s1, s2);
+        else GX_DISPATCH(dtype, k_var_seg, gs, dim3(kT), s, grad, v, s1, s2);
+        const int64_t most = *std::max_element(v.nb, v.nb + v.n);
+        hipLaunchKernelGGL(k_var_finish, dim3((unsigned)grid_cap(most, kT, 4096), (unsigned)v.n), dim3(kT), 0, s, s1,
+                           s2, v, totals);
+        if (rc == GEFENX_OK) rc = check("block variance");
+    }
+    if (rc == GEFENX_OK && !tiled.empty()) {
         hipLaunchKernelGGL(k_var_sum, dim3((unsigned)n_periods), dim3(64), 0, s, part, kVarGrid, totals);
         rc = check("block variance sum");
     }
@@ -634,8 +687,9 @@ int gefenx_block_variance_errors_ex(const void* grad, int dtype, int64_t numel, 
             hipStreamSynchronize(s) != hipSuccess)
             rc = set_error(GEFENX_ELAUNCH, "gefenx_block_variance_errors: copy-back failed");
     }
-    hipStreamSynchronize(s);
-    hipFree(dev);
+    (void)hipFreeAsync(dev, s);
+    if (hipStreamSynchronize(s) != hipSuccess && rc == GEFENX_OK)
+        rc = set_error(GEFENX_ELAUNCH, "gefenx_block_variance_errors: synchronisation failed");
     if (rc) return rc;
     for (int i = 0; i < n_periods; ++i) {
         const double nb = (double)(numel / periods[i]);

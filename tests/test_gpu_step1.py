@@ -154,6 +154,27 @@ def test_period_errors_large_blocks(dev, dt):
     np.testing.assert_allclose(got, ref, rtol=1e-10)
 
 
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("numel", [1441440, 4097, 12288])
+def test_period_errors_many_candidates(dev, dt, numel):
+    """Candidates that share launches (1441440 has 288 divisors: several full
+    batches of either kind; the others a single large one or few) have the
+    errors they have alone, at any alignment.  1e-12: the order of the float64
+    atomics; 1e-10 against the oracle as above (one-pass large blocks)."""
+    from gefen import partitioning
+    gen = torch.Generator().manual_seed(numel)
+    g = (torch.randn(numel + 1, generator=gen) * 1e-3).to(dt)
+    d = g.to(dev)[1:]
+    divs = partitioning.divisors(numel)
+    got = partitioning.block_variance_errors_device(d, divs)
+    vals = (g[1:].float().numpy() ** 2).astype(np.float32).astype(np.float64)
+    ref = [np.sqrt(vals.reshape(-1, p).var(axis=1).mean()) for p in divs]
+    np.testing.assert_allclose(got, ref, rtol=1e-10, atol=1e-300)
+    some = list(range(0, len(divs), 9))
+    alone = [partitioning.block_variance_errors_device(d, [divs[i]])[0] for i in some]
+    np.testing.assert_allclose([got[i] for i in some], alone, rtol=1e-12, atol=1e-300)
+
+
 def test_gefen_class_first_steps_match_oracle(dev):
     """Gefen.step on the GPU: periods from the search, the learned codebook
     and three steps of state against the oracle run on the same inputs."""
