@@ -44,7 +44,7 @@ constexpr int kVarBatch = 32;    // candidate periods per launch
 // longer than its launch, and large blocks leave most CUs without a segment
 // (64 workgroups for 4M elements), so candidates share launches; each one's
 // sums are those of a launch of its own.  First step of a layer of hidden
-// size 2048 (nine tensors, 22 to 24 candidates each): 8.0 -> 6.05 ms.
+// size 2048 (nine tensors, 12 to 46 candidates each): 8.0 -> 6.05 ms.
 struct VarPeriods {
     int64_t P[kVarBatch], nb[kVarBatch];
     int64_t first[kVarBatch];  // k_var_seg: first workgroup
