@@ -37,29 +37,34 @@ static_assert(sizeof(QTable) % 16 == 0, "QTable must stay 16-byte aligned in siz
 // zero on entry and left zero on exit by the finalize kernels.
 inline size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-// Factored stats tiling: a workgroup covers kFactTileCols columns (64 lanes x
-// two 8-column chunks) of `tile_rows` consecutive rows.  A tile's size has two
-// bounds.  Per tensor: about N/32 elements, between 64K and 1M (in a launch of
-// billions of elements larger tiles spend less of the pass on set-up and
-// flushes: on the Llama-3-8B set caps of 256K / 512K / 1M / 2M measured
-// 4.30 / 4.08 / 3.97 / 3.96 ms).  Per launch: launch_elems / kFactLaunchWgs,
-// so that a launch of any size fills the 256 CUs' four workgroups each (the
-// LDS of a workgroup allows four); with N/32 alone a single tensor is 32
-// workgroups and a decoder layer 298, one wave per SIMD and most of the chip
-// idle.  Not below kFactTileSmallElems, where a tile's set-up and its column
-// partials cost more than the waves it adds.  Measured (stats kernel, us;
-// N/32 alone -> launch_elems / 512, / 1024, / 2048 with 16K): one decoder
-// layer (218M bf16) 282 -> 154, 129, 136; 4096x4096 fp32 140 -> 28, 30, 35;
-// 43M fp16 elements in odd sizes 470 -> 57, 46, 47; 7.5M bf16 in 8 matrices
-// 258 -> 76, 75, 75.
-// Tiles start at multiples of 32 rows, so the rows whose squares meet in one
-// fp32 column partial are the same in every launch; the launch decides the
-// order of the float64 additions of those partials only.
+// Factored stats tiling.  A tensor's sums of squares are added up in an order
+// that its shape and block length alone decide, whatever else the call holds:
+// fp32 over 8 rows (float64 for fp32 grads), four such values to a granule,
+// granules in order to a tile, tiles in order to the total.  Granules and tiles
+// are rows of a column tile (transposed views: columns of a row band).
+// How the launch is cut is another matter: a workgroup takes a tile, or, where
+// that would leave CUs idle, a granule, whose sum then goes to scratch of the
+// call and which finalize adds up in the same order.
+//   tiles: about N/32 elements, between 64K and 1M.  In a launch of billions of
+// elements large ones spend less of the pass on set-up and flushes (on the
+// Llama-3-8B set caps of 256K / 512K / 1M / 2M measured 4.30 / 4.08 / 3.97 /
+// 3.96 ms), and their sums are what stays resident per tensor.
+//   granules: multiples of 32 rows (each of the 4 waves 8), at least 8K elements,
+// as many as leave a tensor at most kFactGranules of them, the workgroups that the
+// CUs hold: a second round of a few costs as much as the first (11008 x 4096 in
+// 256-element blocks, stats kernel: 920 workgroups 59.9 us, 1376 of them 69.7; in
+// rows as blocks 688 of them 36.9, 460 45.4).  A workgroup on a tile meets after
+// each (about 2 us: twenty of 4096 x 4096 in 32 rows 239 us against 201 without),
+// so 1024-column tiles take 128 rows where that leaves kFactGranulesOf128 of them
+// (the Llama-3-8B set's step 15.89 ms against 16.08 in 64 rows).
+// Tiles hold equal numbers of them (14336 x 4096 in 1024 rows against 1056 and a
+// short last tile: 3% of the stats of twelve).
 constexpr int64_t kFactTileCols = 1024;
 constexpr int64_t kFactTileMinElems = 1 << 16;
 constexpr int64_t kFactTileMaxElems = 1 << 20;
-constexpr int64_t kFactTileSmallElems = 1 << 14;
-constexpr int64_t kFactLaunchWgs = 1024;
+constexpr int64_t kFactGranules = 1024;
+constexpr int64_t kFactGranulesOf128 = 448;
+constexpr int64_t kFactGranuleElems = 1 << 13;
 
 // Contiguous matrices (C >= 8) of at most kNarrowMaxCols columns, or with
 // blocks shorter than kShortPeriod, take tiles of up to kLaneTileCols columns
@@ -72,60 +77,68 @@ inline bool lane_tiles(int64_t cols, int64_t period) {
     return cols >= 8 && (cols <= kNarrowMaxCols || (period < kShortPeriod && period < cols));
 }
 
-// As launch_elems: the largest tiles whatever the launch, for the scratch of
-// fixed size.  Short blocks of wide matrices then stay on 1024-column tiles: the
-// twice as many row partials of the lane tiles would take shapes out of it
-// (21920 x 21920 in 512-element blocks 30.3 -> 34.0 MB of 33.6).
-constexpr int64_t kCoarseTiles = (int64_t)1 << 62;
-
-// Transposed-view stats (strides (1, ld)): tiles of up to four 64-row bands,
-// one for each wave of the workgroup, and a multiple of 64 columns, half as
-// many elements as the contiguous tiles (a wave walks its columns one 64 x 64
-// tile at a time, with nothing else in flight: on 51M elements of a decoder
-// layer 1024-column tiles 59 us, the share of 1/1024 of the launch 42 us, of
-// 1/2048 37 us).
+// Transposed-view stats (strides (1, ld)): bands of up to 256 rows, 64 for each
+// wave of the workgroup, tiles of 1024 columns, granules of 64 to 512.  A wave
+// walks its columns one 64 x 64 tile at a time, with nothing else in flight, so
+// half as large a share of the launch as for the contiguous tiles is the faster
+// one (on 51M elements of a decoder layer 1024-column tiles 59 us, 1/1024 of the
+// launch 42 us, 1/2048 37 us).  Not below 16K elements: with few rows, one
+// finalize workgroup adds up all partials of a row (16 x 100000 in 64 columns
+// 154 us a step against 88 in 1024).  The block path leaves no such partials and
+// takes 64 columns there (49 against 92).
 constexpr int64_t kTvStatsMaxRows = 256;
+constexpr int64_t kTvGranules = 512;
+
+struct Tiling {
+    int64_t ct, rt;      // tiles: columns, rows
+    int64_t rows, cols;  // of a tile
+    int64_t gran, ng;    // granule: rows (views: columns) and count
+};
 
 struct FactTiles {
-    int64_t ct, rt, tile_rows;                            // 1024-column tiles
-    int64_t ct_l, rt_l, l_rows, l_cols, lg_lanes;         // lane tiles (lg_lanes: log2 lanes per row; -1: not taken)
-    int64_t ct_tv, rt_tv, tv_rows, tv_cols;               // transposed-view tiles
-    // launch_elems: elements of all tensors of the launch (>= rows * cols)
-    static FactTiles make(int64_t rows, int64_t cols, int64_t period, int64_t launch_elems) {
+    Tiling wide, lane, tv;  // 1024-column tiles, lane tiles, transposed views
+    int64_t lg_lanes;       // lane tiles: log2 lanes per row; -1: not taken
+    static FactTiles make(int64_t rows, int64_t cols, int64_t period, bool factored = true) {
         FactTiles t;
         const auto ceil_div = [](int64_t x, int64_t d) { return x > 0 ? (x + d - 1) / d : 1; };
-        int64_t elems = rows * cols / 32;
+        const int64_t N = rows * cols;
+        int64_t elems = N / 32;
         elems = elems < kFactTileMinElems ? kFactTileMinElems : (elems > kFactTileMaxElems ? kFactTileMaxElems : elems);
-        int64_t share = launch_elems / kFactLaunchWgs;
-        if (share < kFactTileSmallElems) share = kFactTileSmallElems;
-        if (elems > share) elems = share;
-        // rows of a tile of `width` columns: whole 8-row fp32 column groups of
-        // each wave (lane tiles: of each lane), `gran` rows together
-        const auto tile_rows = [&](int64_t width, int64_t gran) {
+        // tiles of `width` columns; `unit` rows hold 8 rows of every wave (lane tiles: of every lane)
+        const auto tiling = [&](int64_t width, int64_t unit) {
+            Tiling q;
             const int64_t w = cols < width ? (cols < 1 ? 1 : cols) : width;
-            int64_t r = ceil_div(ceil_div(elems, w), gran) * gran;
-            if (r > rows) r = rows;
-            return r < 1 ? 1 : r;
+            q.gran = unit;
+            while (q.gran * w < kFactGranuleElems) q.gran *= 2;
+            q.gran *= ceil_div(N, kFactGranules * q.gran * w);
+            if (width == kFactTileCols && q.gran < 128 && N >= kFactGranulesOf128 * 128 * w) q.gran = 128;
+            q.cols = width;
+            q.ct = ceil_div(cols, width);
+            q.ng = ceil_div(rows, q.gran);
+            q.rt = ceil_div(q.ng, ceil_div(elems, q.gran * w));
+            q.rows = ceil_div(q.ng, q.rt) * q.gran;
+            q.rt = ceil_div(rows, q.rows);
+            if (q.rows > rows) q.rows = rows < 1 ? 1 : rows;
+            return q;
         };
-        t.ct = ceil_div(cols, kFactTileCols);
-        t.tile_rows = tile_rows(kFactTileCols, 32);
-        t.rt = ceil_div(rows, t.tile_rows);
+        t.wide = tiling(kFactTileCols, 32);
         t.lg_lanes = -1;
-        t.ct_l = t.rt_l = 0;
-        t.l_rows = t.l_cols = 0;
-        if (lane_tiles(cols, period) && (cols <= kNarrowMaxCols || launch_elems < kCoarseTiles)) {
-            t.l_cols = (ceil_div(cols, ceil_div(cols, kLaneTileCols)) + 7) & ~int64_t(7);  // even column tiles
+        t.lane = Tiling{};
+        if (lane_tiles(cols, period)) {
+            const int64_t width = (ceil_div(cols, ceil_div(cols, kLaneTileCols)) + 7) & ~int64_t(7);  // even column tiles
             t.lg_lanes = 0;
-            while ((8 << t.lg_lanes) < t.l_cols) ++t.lg_lanes;
-            t.ct_l = ceil_div(cols, t.l_cols);
-            t.l_rows = tile_rows(t.l_cols, 32 * (64 >> t.lg_lanes));
-            t.rt_l = ceil_div(rows, t.l_rows);
+            while ((8 << t.lg_lanes) < width) ++t.lg_lanes;
+            t.lane = tiling(width, 32 * (64 >> t.lg_lanes));
         }
-        t.tv_rows = rows < 1 ? 1 : (rows < kTvStatsMaxRows ? rows : kTvStatsMaxRows);
-        t.rt_tv = ceil_div(rows, t.tv_rows);
-        const int64_t vc = (share / (2 * kTvStatsMaxRows) + 63) & ~int64_t(63);
-        t.tv_cols = vc < 64 ? 64 : vc > kFactTileCols ? kFactTileCols : vc;
-        t.ct_tv = ceil_div(cols, t.tv_cols);
+        t.tv.rows = rows < 1 ? 1 : (rows < kTvStatsMaxRows ? rows : kTvStatsMaxRows);
+        t.tv.rt = ceil_div(rows, t.tv.rows);
+        t.tv.cols = kFactTileCols;
+        t.tv.ct = ceil_div(cols, kFactTileCols);
+        t.tv.gran = 64;
+        while (t.tv.gran < kFactTileCols &&
+               ((factored && t.tv.rows * t.tv.gran < kFactGranuleElems) || 2 * t.tv.rows * t.tv.gran <= N / kTvGranules))
+            t.tv.gran *= 2;
+        t.tv.ng = ceil_div(cols, t.tv.gran);
         return t;
     }
 };
@@ -142,31 +155,51 @@ inline int64_t mag_shards(int64_t nb) { return nb <= kMagShardMaxBlocks ? kMagSh
 // sum(v_row) each; the apply kernel adds the partials in a fixed order).
 constexpr int64_t kFinRowsPerWg = 256;
 
+// Static scratch of gefenx_factored_update_noalloc.
+constexpr size_t kNoallocScratch = (size_t)32 << 20;
+
 struct FactoredWs {
-    // double row_part[max of the tilings' ct][rows], double col_part[max rt][cols] (per-tile
-    // partial sums, fully rewritten every step; launch_elems = rows * cols sizes them for the
-    // smallest tiles, so one workspace serves the tensor in every launch), uint32 magbits[shards][nb] (zero
+    // double row_part[most ct of the tilings][rows], double col_part[most rt][cols] (per-tile
+    // partial sums, fully rewritten every step), uint32 magbits[shards][nb] (zero
     // between steps), float mag_old[nb], float minv[nb],
     // double vrow_sum[ceil(rows/256)] (partials of sum(v_row)), float vcs[cols] (sqrt(v_col)),
     // {uint32 finalize counter (zero between steps), float mean(v_row)}
+    FactTiles tiles;
     size_t off_rowp, off_colp, off_magbits, off_magold, off_minv, off_vsum, off_vcs, off_fin, total;
-    static FactoredWs make(int64_t rows, int64_t cols, int64_t nb, int64_t launch_elems) {
+    // The lane tiles of short blocks have twice the row partials of 1024-column
+    // tiles.  Where these alone would take a tensor out of the static scratch
+    // (21920 x 21920 in 512-element blocks 30.3 -> 34.0 MB of 33.6), it keeps
+    // the 1024-column tiles, in every entry point.
+    static FactoredWs make(int64_t rows, int64_t cols, int64_t nb) {
         FactoredWs w;
-        const FactTiles t = FactTiles::make(rows, cols, nb > 0 ? rows * cols / nb : 1, launch_elems);
+        w.tiles = FactTiles::make(rows, cols, nb > 0 ? rows * cols / nb : 1);
+        w.lay_out(rows, cols, nb);
+        if (w.tiles.lg_lanes >= 0 && cols > kNarrowMaxCols && w.total > kNoallocScratch) {
+            FactoredWs v = w;
+            v.tiles.lg_lanes = -1;
+            v.tiles.lane = Tiling{};
+            v.lay_out(rows, cols, nb);
+            if (v.total <= kNoallocScratch) return v;
+        }
+        return w;
+    }
+
+private:
+    void lay_out(int64_t rows, int64_t cols, int64_t nb) {
         size_t o = 0;
         // any of the three tilings fits
-        const auto max3 = [](int64_t x, int64_t y, int64_t z) { return x > y ? (x > z ? x : z) : (y > z ? y : z); };
-        const int64_t ct = max3(t.ct, t.ct_l, t.ct_tv), rt = max3(t.rt, t.rt_l, t.rt_tv);
-        w.off_rowp = o;    o += align256(sizeof(double) * (size_t)(ct * rows));
-        w.off_colp = o;    o += align256(sizeof(double) * (size_t)(rt * cols));
-        w.off_magbits = o; o += align256(sizeof(uint32_t) * (size_t)(nb * mag_shards(nb)));
-        w.off_magold = o;  o += align256(sizeof(float) * (size_t)nb);
-        w.off_minv = o;    o += align256(sizeof(float) * (size_t)nb);
-        w.off_vsum = o;    o += align256(sizeof(double) * (size_t)((rows + kFinRowsPerWg - 1) / kFinRowsPerWg));
-        w.off_vcs = o;     o += align256(sizeof(float) * (size_t)cols);
-        w.off_fin = o;     o += 256;
-        w.total = o;
-        return w;
+        const auto most = [](int64_t x, int64_t y) { return x > y ? x : y; };
+        const int64_t ct = most(tiles.wide.ct, tiles.lane.ct);
+        const int64_t rt = most(most(tiles.wide.rt, tiles.lane.rt), tiles.tv.rt);
+        off_rowp = o;    o += align256(sizeof(double) * (size_t)(ct * rows));
+        off_colp = o;    o += align256(sizeof(double) * (size_t)(rt * cols));
+        off_magbits = o; o += align256(sizeof(uint32_t) * (size_t)(nb * mag_shards(nb)));
+        off_magold = o;  o += align256(sizeof(float) * (size_t)nb);
+        off_minv = o;    o += align256(sizeof(float) * (size_t)nb);
+        off_vsum = o;    o += align256(sizeof(double) * (size_t)((rows + kFinRowsPerWg - 1) / kFinRowsPerWg));
+        off_vcs = o;     o += align256(sizeof(float) * (size_t)cols);
+        off_fin = o;     o += 256;
+        total = o;
     }
 };
 

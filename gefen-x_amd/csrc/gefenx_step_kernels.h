@@ -37,7 +37,8 @@ __device__ __forceinline__ void wavemax_flush63(uint32_t* __restrict__ mb, WaveM
 // w takes rows r0 + w, r0 + w + 4, ... two at a time.  Per row: squares and
 // the momentum max over the lane's 16 elements, then a float64 DPP reduction
 // of the row sum (one value per row per column tile).  Column sums: fp32 in
-// registers over 8 rows, then float64; the 4 waves combine in LDS at the end.
+// registers over 8 rows, then float64 in LDS, where the 4 waves meet after each
+// granule and join the tile's partial (FactTiles has the order).
 // Both go out as float64 partials (no float atomics, deterministic).
 // FAST: contiguous grad and C >= 8, any alignment, any C and P (the vector
 // loads take any address; a row's last chunk, when C % 8 != 0, loads the row's
@@ -48,9 +49,26 @@ __device__ __forceinline__ void wavemax_flush63(uint32_t* __restrict__ mb, WaveM
 // element loads in a launch of their own) -> 49; 7.5M bf16 elements with
 // 256-element blocks 75 -> 40.
 // ====================================================================
+// A granule's column sum joins the tile's partial, which one thread owns: a
+// plain store of the first, then atomics that return nothing, performed in
+// order (a sum in registers would cost 8 of the stats kernel's 128).
+__device__ __forceinline__ void put_granule(double* p, double v, bool first) {
+    if (first) *gbl(p) = v;
+    else gatomic_add(p, v);
+}
+
+// v, as far as the compiler knows another value each time: what follows from it
+// is computed where it is used instead of held in registers across a loop.
+__device__ __forceinline__ int opaque(int v) {
+    asm volatile("" : "+v"(v));
+    return v;
+}
+
 struct FactStatsLds {
     float cbr[kCodebookMax];
-    double col[kWaves][kChunk][2][64];  // float64 column sums: [wave][k][h][lane]
+    // float64 column sums of a granule: [wave][k][64 h + lane]; the padding puts
+    // the 64 columns that a wave reads in order into different banks
+    double col[kWaves][kChunk][2 * 64 + 8];
     int64_t wblk[kWaves];
     uint32_t wbits[kWaves];
 };
@@ -73,7 +91,7 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
     const uint8_t* idxp = wr.idx;
     const float* mag_old = wr.mag;
     double* row_part = wr.row_part;
-    double* col_part = wr.col_part;
+    double* col_part = col_partials(wr);
     const int64_t R = wr.R, C = wr.C, P = wr.P, gs0 = wr.gs0, gs1 = wr.gs1;
     const int64_t ct = wr.ct, tile_rows = wr.tile_rows, nb = wr.nb;
     const double invP = wr.invP;
@@ -113,21 +131,47 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
     const int64_t dP4 = d4 - dB4 * P;
 
     // column sums: in registers over 8 rows, then added into the wave's
-    // float64 slots in LDS (each lane owns its 16 columns' slots)
+    // float64 slots in LDS (each lane owns its 16 columns' slots); the first of
+    // a granule is stored
     Acc colf[H][kChunk];
 #pragma unroll
     for (int h = 0; h < H; ++h)
 #pragma unroll
-        for (int k = 0; k < kChunk; ++k) { colf[h][k] = 0; s_col[wave][k][h][lane] = 0.0; }
+        for (int k = 0; k < kChunk; ++k) { colf[h][k] = 0; s_col[wave][k][64 * h + lane] = 0.0; }
     auto flush_cols = [&]() {
 #pragma unroll
         for (int h = 0; h < H; ++h)
 #pragma unroll
             for (int k = 0; k < kChunk; ++k) {
-                s_col[wave][k][h][lane] += (double)colf[h][k];
+                s_col[wave][k][64 * h + lane] += (double)colf[h][k];
                 colf[h][k] = 0;
             }
     };
+    // A granule's end: waves summed in order 0..3 (and cleared, where the tile
+    // goes on); thread t takes columns t, t + 256, ...  The bare barriers leave
+    // the next rows' loads in flight.
+    double* const col_out = col_part + rtile * C + tc0;
+    auto fold = [&](bool first, auto goes_on) {
+        lds_barrier();
+        const unsigned t = (unsigned)opaque((int)threadIdx.x);
+        double* src = &s_col[0][t % kChunk][t / kChunk];
+        constexpr int kWaveStride = kChunk * (2 * 64 + 8), kStride = kThreads / kChunk;
+#pragma unroll 2
+        for (int j = 0; j < kFactTileCols / kThreads; ++j) {
+            double sum = src[j * kStride];
+#pragma unroll
+            for (int ww = 1; ww < kWaves; ++ww) sum += src[ww * kWaveStride + j * kStride];
+            if constexpr (decltype(goes_on)::value) {
+#pragma unroll
+                for (int ww = 0; ww < kWaves; ++ww) src[ww * kWaveStride + j * kStride] = 0.0;
+            }
+            const int c = (int)t + j * kThreads;
+            if (c < span) put_granule(col_out + c, sum, first);
+        }
+        if constexpr (decltype(goes_on)::value) lds_barrier();
+    };
+    const int gran = (int)wr.gran;
+    int64_t fold_at = r_begin + gran;  // first row of the next granule
     int nrows_f = 0;
     WaveMax wm{-1, 0u};
     float mag_cur = 0.0f;
@@ -339,6 +383,15 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
     };
 
     constexpr int64_t kStep = 2 * kWaves;
+    // A granule ends inside the tile before row r - wave.  Every wave comes here
+    // with that row: one that left the loop before has r >= r_end, so r_end lies
+    // within the 3 rows after an r - wave below it.  A granule is a multiple of 32 rows, 8 of each wave, so the fp32
+    // sums are flushed.
+    auto granule_ends = [&](int64_t r) { return r - wave == fold_at && fold_at < r_end; };
+    auto end_granule = [&]() {
+        fold(fold_at - gran == r_begin, std::true_type{});
+        fold_at += gran;
+    };
     int64_t r0 = r_begin + wave;
     if (r0 < r_end) {
         Batch ba, bb;
@@ -356,12 +409,14 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
                 load_batch(r0 + kStep, ba);
                 reduce_batch(r0, bb);
                 r0 += kStep;
+                if (granule_ends(r0)) end_granule();
                 if (r0 >= r_end) break;
             }
         } else {
             for (;;) {
                 reduce_batch(r0, ba);
                 r0 += kStep;
+                if (granule_ends(r0)) end_granule();
                 if (r0 >= r_end) break;
                 load_batch(r0, ba);
             }
@@ -390,18 +445,7 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
                 if (s_wblk[ww] >= 0 && s_wbits[ww]) gatomic_max(mb + s_wblk[ww], s_wbits[ww]);
         }
     }
-    // column partials of the tile: waves summed in order 0..3; thread t
-    // stores columns t, t + 256, ... (coalesced)
-#pragma unroll
-    for (int j = 0; j < kFactTileCols / kThreads; ++j) {
-        const int c = threadIdx.x + j * kThreads;
-        const int h = c / (kFactTileCols / 2), cl = c % (kFactTileCols / 2);
-        const int ln = cl / kChunk, k = cl % kChunk;
-        double sum = s_col[0][k][h][ln];
-#pragma unroll
-        for (int ww = 1; ww < kWaves; ++ww) sum += s_col[ww][k][h][ln];
-        if (c < span) *gbl(col_part + rtile * C + tc0 + c) = sum;
-    }
+    fold(fold_at - gran == r_begin, std::false_type{});  // the last granule
 }
 
 // ====================================================================
@@ -412,7 +456,7 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
 // time, four such steps in flight, each lane's old magnitude loaded with its
 // chunk.  A row's lanes add up its sum of squares, a lane keeps its columns'
 // sums (fp32 over 8 rows, then float64), the lanes of one column meet in LDS
-// at the end in a fixed order.  stats_factored would leave all but C / 16 of a
+// after each granule in a fixed order.  stats_factored would leave all but C / 16 of a
 // wave's lanes idle on few columns and walk the rows one by one (a set of
 // 16-column and 16-row fp32 adapters 246 -> 16 us), and would wait for the
 // magnitudes of every row whose blocks end inside it (7.5M bf16 elements with
@@ -448,11 +492,37 @@ __device__ __forceinline__ void stats_lanes(const TensorWork& wr, int64_t wg, Fa
     const int64_t r_end = std::min<int64_t>(r_begin + wr.tile_rows, R);
     __syncthreads();
     Acc colf[kChunk];
-    double cold[kChunk];
 #pragma unroll
-    for (int k = 0; k < kChunk; ++k) { colf[k] = 0; cold[k] = 0.0; }
+    for (int k = 0; k < kChunk; ++k) colf[k] = 0;
+    bool fresh = true;
+    auto flush_cols = [&]() {  // as in stats_factored
+        const auto flush = [&](auto add) {
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {
+                double& slot = lds.col[wave][k][lane];
+                slot = fresh ? (double)colf[k] : slot + (double)colf[k];
+                colf[k] = 0;
+            }
+        };
+        flush(std::true_type{});
+        fresh = false;
+    };
+    // A granule's end: per column the waves in order, and the rows of a wave
+    double* const col_part = col_partials(wr) + rtile * C + tc0;
+    auto fold = [&](bool first) {
+        lds_barrier();
+        for (int col = opaque(threadIdx.x); col < span; col += kThreads) {
+            const int j = col / kChunk, k = col % kChunk;
+            double sum = 0.0;
+            for (int ww = 0; ww < kWaves; ++ww)
+                for (int s = 0; s < rpw; ++s) sum += lds.col[ww][k][s * L + j];
+            put_granule(col_part + col, sum, first);
+        }
+    };
+    constexpr int64_t kStep = Q * kWaves;
+    int64_t fold_at = r_begin + wr.gran;  // first row of the next granule
     int nf = 0;
-    for (int64_t r0 = r_begin + wave * rpw; r0 < r_end; r0 += (int64_t)Q * kWaves * rpw) {
+    for (int64_t r0 = r_begin + wave * rpw; r0 < r_end; r0 += kStep * rpw) {
         Raw8<DT> gr[Q];
         RawIdx8 ir[Q];
         int64_t bb[Q], pp[Q];
@@ -506,21 +576,21 @@ __device__ __forceinline__ void stats_lanes(const TensorWork& wr, int64_t wg, Fa
             if ((lane & (L - 1)) == 0 && r < r_end) *gbl(wr.row_part + ctile * R + r) = rsum;
             if (++nf == 8) {
                 nf = 0;
-#pragma unroll
-                for (int k = 0; k < kChunk; ++k) { cold[k] += (double)colf[k]; colf[k] = 0; }
+                flush_cols();
             }
         }
+        // every wave comes here for each granule that ends inside the tile
+        // (one that left the loop has its r0, so every later granule, past r_end)
+        const int64_t next = r0 - wave * rpw + kStep * rpw;
+        if (next == fold_at && fold_at < r_end) {
+            fold(fold_at - wr.gran == r_begin);
+            lds_barrier();
+            fresh = true;
+            fold_at += wr.gran;
+        }
     }
-#pragma unroll
-    for (int k = 0; k < kChunk; ++k) lds.col[wave][k][0][lane] = cold[k] + (double)colf[k];
-    __syncthreads();
-    for (int col = threadIdx.x; col < span; col += kThreads) {
-        const int j = col / kChunk, k = col % kChunk;
-        double sum = 0.0;
-        for (int ww = 0; ww < kWaves; ++ww)
-            for (int s = 0; s < rpw; ++s) sum += lds.col[ww][k][0][s * L + j];
-        *gbl(wr.col_part + rtile * C + tc0 + col) = sum;
-    }
+    flush_cols();
+    fold(fold_at - wr.gran == r_begin);  // the last granule
 }
 
 // ====================================================================
@@ -538,7 +608,6 @@ __device__ __forceinline__ void stats_lanes(const TensorWork& wr, int64_t wg, Fa
 // (8 elements of one logical row) lies in one block since P % 8 == 0.
 // Requires R, C, P multiples of 8 and 16-byte aligned storage rows.
 // ====================================================================
-constexpr int kTvLdsBlocks = 512;   // stats: LDS block accumulators per workgroup
 constexpr int kTvFew = 4;           // blocks a tile may touch on the scalar-load path
 
 // A value every lane of the wave holds, moved to scalar registers.
@@ -631,8 +700,8 @@ struct TvStatsLds {
 // than 4 waves on 4 column ranges) and a wave reads the two halves of each
 // 128-byte index line in consecutive tiles.  MODE 0 (factored): squares in
 // fp32 over a chunk's 8 columns and over a vector's 8 rows (float64 for fp32
-// grads), then float64: a row's sum over the columns collects in its lanes
-// and leaves as the row partial (reduce-scatter over the 8 column groups),
+// grads), then float64: a row's sum over a granule's columns collects in its
+// lanes and joins the row partial (reduce-scatter over the 8 column groups),
 // a column's over the band in one lane (reduce-scatter over the 8 row
 // groups of each tile), and the 4 bands' column sums meet in LDS in band
 // order.  Block max |u| (and, MODE 1, the block's sum of squares, each square
@@ -655,7 +724,7 @@ __device__ __forceinline__ void stats_tv(const TensorWork& wr, int64_t wg, TvSta
     const T* g = static_cast<const T*>(wr.grad);
     const uint8_t* idxp = wr.idx;
     const float* mag_old = wr.mag;
-    double* row_part = wr.row_part;
+    double* row_part = row_partials(wr);
     double* col_part = wr.col_part;
     const int64_t R = wr.R, C = wr.C, P = wr.P, ld = wr.gs1, nb = wr.nb;
     const double invP = wr.invP;
@@ -715,7 +784,9 @@ __device__ __forceinline__ void stats_tv(const TensorWork& wr, int64_t wg, TvSta
         for (int j = 0; j < kChunk; ++j) t.iv[j] = load_raw_idx8_cached(idxp + (rl + j) * C + cl);
     };
 
-    double racc[kChunk];  // MODE 0: row sums of the lane's 8 rows over the columns so far
+    int left = (int)(wr.gran / kTv);  // 64-column tiles to the granule's end
+    double rtot = 0.0;    // MODE 0: sum of row 8a + b over the granules so far
+    double racc[kChunk];  // MODE 0: row sums of the lane's 8 rows over the granule's columns so far
 #pragma unroll
     for (int j = 0; j < kChunk; ++j) racc[j] = 0.0;
 
@@ -812,10 +883,16 @@ __device__ __forceinline__ void stats_tv(const TensorWork& wr, int64_t wg, TvSta
             for (int k = 0; k < kChunk; ++k) cv[k] = (double)colf[k];
             const double col = tv_scatter_lo(cv, la);
             lds.colp[wave][cs * kTv + 8 * lb + la] = col;
-            if (cs == ncs - 1) {
-                const double row = tv_scatter_hi(racc, lb);
+            const bool last = cs == ncs - 1;
+            if (--left == 0 || last) {
+                left = (int)(wr.gran / kTv);
+                rtot += tv_scatter_hi(racc, lb);
+#pragma unroll
+                for (int j = 0; j < kChunk; ++j) racc[j] = 0.0;
+            }
+            if (last) {
                 const int64_t rr = r0 + 8 * la + lb;
-                if (rr < r_end) *gbl(row_part + ctile * R + rr) = row;
+                if (rr < r_end) *gbl(row_part + ctile * R + rr) = rtot;
             }
         }
     };
@@ -976,12 +1053,18 @@ __device__ __forceinline__ void stats_block_one(const TensorWork& w, int64_t wg,
     }
 }
 
+struct BlockStatsLds {
+    float cbr[kCodebookMax];
+    int64_t key[2 * kDetIters * kWaves];
+    double sum[2 * kDetIters * kWaves];
+};
+
 template <int DT, int EPL>
-__device__ __forceinline__ void stats_block_det(const TensorWork& w, int64_t wg) {
+__device__ __forceinline__ void stats_block_det(const TensorWork& w, int64_t wg, BlockStatsLds& lds) {
     using T = typename Elem<DT>::T;
-    __shared__ float s_cbr[kCodebookMax];
-    __shared__ int64_t s_key[2 * kDetIters * kWaves];
-    __shared__ double s_sum[2 * kDetIters * kWaves];
+    float* s_cbr = lds.cbr;
+    int64_t* s_key = lds.key;
+    double* s_sum = lds.sum;
     const int64_t N = w.N, P = w.P, nb = w.nb;
     constexpr int64_t E = (int64_t)kDetIters * kThreads * EPL;
     const int64_t base = wg * E;
@@ -1127,9 +1210,9 @@ __device__ __forceinline__ bool block_stats_fast_ok(const TensorWork& w) {
 }
 
 template <int DT>
-__device__ __forceinline__ void stats_block_wg(const TensorWork& w, int64_t wg) {
-    if (block_stats_fast_ok(w)) stats_block_det<DT, kChunk>(w, wg);
-    else stats_block_det<DT, 1>(w, wg);
+__device__ __forceinline__ void stats_block_wg(const TensorWork& w, int64_t wg, BlockStatsLds& lds) {
+    if (block_stats_fast_ok(w)) stats_block_det<DT, kChunk>(w, wg, lds);
+    else stats_block_det<DT, 1>(w, wg, lds);
 }
 
 // ====================================================================
@@ -2054,11 +2137,15 @@ __device__ __forceinline__ int64_t xcd_contiguous(int64_t b, int64_t G) {
     return x * q + (x < r ? x : r) + b / 8;
 }
 
-// One LDS image for both lerp forms (each instantiation would otherwise
-// declare its own).
+// One LDS image for every form (each instantiation would otherwise declare its
+// own): four workgroups per CU with it.
+union StatsLds {
+    FactStatsLds f;
+    BlockStatsLds b;
+};
+
 template <int DT, bool FAST>
-__device__ __forceinline__ void stats_factored_wg(const TensorWork& w, int64_t wg) {
-    __shared__ FactStatsLds lds;
+__device__ __forceinline__ void stats_factored_wg(const TensorWork& w, int64_t wg, FactStatsLds& lds) {
     if constexpr (FAST) {
         if (w.lg_lanes >= 0) {
             if (w.mc.small) stats_lanes<DT, kLerpSmall>(w, wg, lds);
@@ -2072,7 +2159,8 @@ __device__ __forceinline__ void stats_factored_wg(const TensorWork& w, int64_t w
 
 template <int DT, bool FAST>
 __global__ void __launch_bounds__(kThreads) k_factored_stats(TensorWork w) {
-    stats_factored_wg<DT, FAST>(w, blockIdx.x);
+    __shared__ FactStatsLds lds;
+    stats_factored_wg<DT, FAST>(w, blockIdx.x, lds);
 }
 
 template <int DT>
@@ -2088,7 +2176,8 @@ __global__ void __launch_bounds__(kThreads) k_apply_tv(TensorWork w) {
 
 template <int DT>
 __global__ void __launch_bounds__(kThreads) k_block_stats(TensorWork w) {
-    stats_block_wg<DT>(w, blockIdx.x);
+    __shared__ BlockStatsLds lds;
+    stats_block_wg<DT>(w, blockIdx.x, lds);
 }
 
 template <int DT, int MODE, bool SR, int FAST>
@@ -2105,11 +2194,12 @@ __global__ void __launch_bounds__(kThreads, FAST && DT != F32 ? 4 : 2) k_mt_fact
     const Seg sg = find_seg(tb, blockIdx.x);
     const TensorWork& w = ws[sg.t];
     const int64_t local = (int64_t)blockIdx.x - sg.wg_begin;
+    __shared__ StatsLds lds;
     if (w.mode != 0) {
-        stats_block_wg<DT>(w, local);
+        stats_block_wg<DT>(w, local, lds.b);
         return;
     }
-    stats_factored_wg<DT, FAST>(w, local);
+    stats_factored_wg<DT, FAST>(w, local, lds.f);
 }
 
 template <int DT, int MODE>

@@ -46,29 +46,44 @@ __device__ __forceinline__ void finalize_magnitude(const TensorWork& w, int64_t 
     w.minv[b] = block_recip(m);
 }
 
-// Sum of p[0], p[stride], ..., p[(n-1)*stride] in index order (the sequential
-// sum, bit for bit), the loads issued four at a time.
-__device__ __forceinline__ double ordered_sum(const double* __restrict__ p, int64_t n, int64_t stride) {
-    double s = 0.0;
-    int64_t t = 0;
-    for (; t + 4 <= n; t += 4) {
-        double a[4];
+// Sum of the tiles [t0, t1), in order, of n partials p[0], p[stride], ..., of
+// which `per` in order make a tile; the loads issued eight at a time.
+__device__ __forceinline__ double tile_sum(const double* __restrict__ p, int64_t t0, int64_t t1, int64_t per, int64_t n,
+                                           int64_t stride) {
+    const int64_t end = t1 * per < n ? t1 * per : n;
+    double s = 0.0, t = 0.0;
+    int left = (int)per;
+    const auto add = [&](double a) {  // 0 + a is a: with one partial to a tile, s += a
+        t += a;
+        if (--left == 0) {
+            s += t;
+            t = 0.0;
+            left = (int)per;
+        }
+    };
+    int64_t i = t0 * per;
+    const auto run = [&](auto n_loads) {
+        constexpr int kLoads = decltype(n_loads)::value;
+        for (; i + kLoads <= end; i += kLoads) {
+            double a[kLoads];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) a[k] = *gbl(p + (t + k) * stride);
+            for (int k = 0; k < kLoads; ++k) a[k] = *gbl(p + (i + k) * stride);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) s += a[k];
-    }
-    for (; t < n; ++t) s += *gbl(p + t * stride);
-    return s;
+            for (int k = 0; k < kLoads; ++k) add(a[k]);
+        }
+    };
+    run(std::integral_constant<int, 8>{});
+    run(std::integral_constant<int, 2>{});
+    for (; i < end; ++i) add(*gbl(p + i * stride));
+    return left != (int)per ? s + t : s;
 }
 
 // ====================================================================
-// Factored finalize.  Workgroups [0, nr): v_row EMA from the ct row partials
-// plus one float64 partial of sum(v_row); [nr, nr+nc): v_col EMA from the rt
-// column partials in row-tile order, csplit threads per column: thread p sums
-// the p-th run of ceil(rt / csplit) partials in order, then the runs are
-// added in order (one run, the plain sequential sum, when rt <= 32); the
-// rest: magnitudes.
+// Factored finalize.  Workgroups [0, nr): v_row EMA from the row partials of
+// the f_ct column tiles plus one float64 partial of sum(v_row); [nr, nr+nc):
+// v_col EMA from the column partials of the f_rt row tiles in order, csplit
+// threads per column: thread p sums the p-th run of ceil(f_rt / csplit) tiles
+// in order, then the runs are added in order; the rest: magnitudes.
 // v <- fma(sum/n, 1-beta2, v*beta2)  (gefen.py:2994-2996)
 // ====================================================================
 __device__ __forceinline__ void finalize_factored(const TensorWork& w, int64_t wg) {
@@ -78,7 +93,7 @@ __device__ __forceinline__ void finalize_factored(const TensorWork& w, int64_t w
         const int64_t i = wg * kFinRowsPerWg + tid;
         double v64 = 0.0;
         if (i < w.R) {
-            const double s = ordered_sum(w.row_part + i, w.ct, w.R);
+            const double s = tile_sum(row_partials(w) + i, 0, w.f_ct, w.pr_per, w.pr_n, w.R);
             const float ms = (float)s / (float)w.C;
             const float v = __builtin_fmaf(ms, w.alpha2, w.v0[i] * w.beta2);
             w.v0[i] = v;
@@ -100,10 +115,10 @@ __device__ __forceinline__ void finalize_factored(const TensorWork& w, int64_t w
         const int cpw = kThreads / sp;  // columns per workgroup
         const int part = tid / cpw;
         const int64_t j = (wg - w.nr) * cpw + tid % cpw;
-        const int64_t per = (w.rt + sp - 1) / sp;
-        const int64_t t0 = std::min<int64_t>((int64_t)part * per, w.rt);
-        const int64_t t1 = std::min<int64_t>(t0 + per, w.rt);
-        double tot = j < w.C ? ordered_sum(w.col_part + t0 * w.C + j, t1 - t0, w.C) : 0.0;
+        const int64_t per = (w.f_rt + sp - 1) / sp;
+        const int64_t t0 = std::min<int64_t>((int64_t)part * per, w.f_rt);
+        const int64_t t1 = std::min<int64_t>(t0 + per, w.f_rt);
+        double tot = j < w.C ? tile_sum(col_partials(w) + j, t0, t1, w.pc_per, w.pc_n, w.C) : 0.0;
         if (sp > 1) {
             s_run[tid] = tot;
             __syncthreads();
@@ -287,8 +302,6 @@ struct WorkInput {
     const int64_t* seed_dev;
     void* workspace;
     size_t ws_bytes;
-    int64_t launch_elems;  // elements of all tensors of the launch (sizes the stats tiles)
-    int64_t ws_elems;      // the launch size the factored workspace is laid out for (its smallest tiles)
 };
 
 // The divisor of the reference's decomposed step (bc2, or sqrt(bc2) on the
@@ -299,6 +312,96 @@ struct WorkInput {
 static float reference_divisor(double inv) {
     if (!(inv > 0.0) || !std::isfinite(inv)) return 0.0f;
     return (float)(1.0 / inv);
+}
+
+// Workgroup = tile q of the contiguous (lane or 1024-column) or view stats.
+static void set_tiles(TensorWork& w, const Tiling& q) {
+    w.ct = w.f_ct = w.pr_n = q.ct;
+    w.f_rt = w.pc_n = q.rt;
+    w.pc_per = w.pr_per = 1;
+    w.tile_rows = q.rows;
+    w.tile_cols = q.cols;
+    w.gran = q.gran;
+    w.stats_wgs = q.ct * q.rt;
+}
+
+// Granules of the launch's workgroups where a granule is one (0 columns or rows
+// of partials each: the block path's views leave none).
+struct Granules {
+    int64_t wgs, doubles;
+};
+
+static Granules granules(const TensorWork& w) {
+    if (w.fast_stats == 2) {
+        const int64_t ng = ceil_div(w.C, w.gran);
+        return Granules{ng * w.f_rt, w.mode == 0 ? ng * w.R : 0};
+    }
+    const int64_t ng = ceil_div(w.R, w.gran);
+    return Granules{w.f_ct * ng, ng * w.C};
+}
+
+// Workgroup = granule; the caller says where the partials are (part, or
+// col_part / row_part of a single tensor).
+static void take_granules(TensorWork& w) {
+    w.stats_wgs = granules(w).wgs;
+    if (w.fast_stats == 2) {
+        w.pr_per = w.tile_cols / w.gran;
+        w.ct = w.pr_n = ceil_div(w.C, w.gran);
+        w.tile_cols = w.gran;
+    } else {
+        w.pc_per = ceil_div(w.tile_rows, w.gran);
+        w.pc_n = ceil_div(w.R, w.gran);
+        w.tile_rows = w.gran;
+    }
+}
+
+// A granule is a workgroup where the tile holds more than this share of its
+// launch's elements: the 256 CUs take four workgroups each (the LDS of one
+// allows four), and fewer than two leave them waiting for loads.  Measured (stats
+// kernel, us; tiles of N/32 alone -> about 1/512, 1/1024, 1/2048 of the launch):
+// one decoder layer (218M bf16) 282 -> 154, 129, 136; 4096x4096 fp32 140 -> 28,
+// 30, 35; 43M fp16 elements in odd sizes 470 -> 57, 46, 47; 7.5M bf16 in 8 matrices
+// 258 -> 76, 75, 75; but 20 of 4096x4096 bf16, 640 tiles, 727 us a step in tiles
+// and 757 in 1024 parts.
+constexpr int64_t kFactLaunchWgs = 512;
+constexpr int64_t kTvLaunchWgs = 2048;  // kTvStatsMaxRows has the figures
+// Views whose bands hold more blocks than a workgroup's LDS send an atomic per
+// chunk, more of them to one block at a time the narrower the workgroups are
+// (4096 x 11008 in 256-element blocks, 176 tiles: 350 us a step in tiles, 385 and
+// 408 in 256 and 128 columns; 4096 x 4096, 64 tiles: 175 in tiles, 145 in 128).
+constexpr int64_t kTvManyBlockTiles = 128;
+
+static bool wants_granules(const TensorWork& w, int64_t launch_elems) {
+    if ((w.mode != 0 && w.fast_stats != 2) || granules(w).wgs <= w.stats_wgs) return false;
+    if (w.fast_stats == 2 && w.tile_rows * w.C / w.P > kTvLdsBlocks && w.stats_wgs >= kTvManyBlockTiles) return false;
+    const int64_t tile = std::min<int64_t>(w.tile_rows, w.R) * std::min<int64_t>(w.tile_cols, w.C);
+    return tile > launch_elems / (w.fast_stats == 2 ? kTvLaunchWgs : kFactLaunchWgs);
+}
+
+// Row steps of an apply task (apply_tasks), by the elements of its launch.
+static void set_apply_steps(TensorWork& w, int64_t launch_elems) {
+    if (w.mode != 0 || !(w.fast_apply & 1)) return;
+    w.a_steps = launch_elems < kSmallApplyElems ? 2 : kRowsPerTask;
+    const int64_t task_rows = (int64_t)w.a_steps * (64 >> w.a_lg);
+    w.apply_wgs = ceil_div(w.a_segs * ceil_div(w.R, task_rows), (int64_t)kWaves);
+}
+
+// Transposed views the view kernels take: strides (1, ld), storage rows 16-byte
+// aligned, chunks that cross no row, column or block border.
+static bool view_shape(int64_t R, int64_t C, int64_t P, const void* idx) {
+    return R > 1 && R % kChunk == 0 && C % kChunk == 0 && P % kChunk == 0 && aligned(idx, 8);
+}
+static bool view_strides(int64_t R, int64_t s0, int64_t s1, int dtype, const void* data) {
+    return s0 == 1 && s1 >= R && (s1 * (int64_t)elem_size(dtype)) % 16 == 0 && aligned(data, 16);
+}
+
+// The factored stats' variant and tiles.
+static void set_factored_stats(TensorWork& w, const FactTiles& t) {
+    const bool dense = w.gs1 == 1 && w.gs0 == w.C;
+    w.fast_stats = dense && w.C >= kChunk ? 1
+                 : view_shape(w.R, w.C, w.P, w.idx) && view_strides(w.R, w.gs0, w.gs1, w.dtype, w.grad) ? 2 : 0;
+    w.lg_lanes = w.fast_stats == 1 ? (int32_t)t.lg_lanes : -1;
+    set_tiles(w, w.fast_stats == 2 ? t.tv : w.lg_lanes >= 0 ? t.lane : t.wide);
 }
 
 static int build_work(const WorkInput& in, TensorWork& w) {
@@ -323,17 +426,13 @@ static int build_work(const WorkInput& in, TensorWork& w) {
     w.write_p = (in.step_scalars != nullptr) || !(in.sc.lr == 0.0f && in.sc.wdf == 1.0f);
     char* ws = static_cast<char*>(in.workspace);
     const int64_t nchunks = ceil_div(N, kChunk);
-    // transposed views: strides (1, ld), storage rows 16-byte aligned
-    const int64_t es = (int64_t)elem_size(in.dtype);
-    const bool tv_shape = in.R > 1 && in.R % kChunk == 0 && in.C % kChunk == 0 && in.period % kChunk == 0 &&
-                          aligned(in.idx, 8);
-    const bool tv_g = in.gs0 == 1 && in.gs1 >= in.R && (in.gs1 * es) % 16 == 0 && aligned(in.grad, 16);
-    const bool tv_p = in.ps0 == 1 && in.ps1 >= in.R && (in.ps1 * es) % 16 == 0 && aligned(in.p, 16);
+    const bool tv_shape = view_shape(in.R, in.C, in.period, in.idx);
+    const bool tv_g = view_strides(in.R, in.gs0, in.gs1, in.dtype, in.grad);
+    const bool tv_p = view_strides(in.R, in.ps0, in.ps1, in.dtype, in.p);
     if (in.mode == 0) {
-        const FactoredWs L = FactoredWs::make(in.R, in.C, nb, in.ws_elems);
+        const FactoredWs L = FactoredWs::make(in.R, in.C, nb);
         if (in.ws_bytes < L.total)
             return set_error(GEFENX_EINVAL, "factored update: workspace %zu bytes < required %zu", in.ws_bytes, L.total);
-        const FactTiles t = FactTiles::make(in.R, in.C, in.period, in.launch_elems);
         w.row_part = reinterpret_cast<double*>(ws + L.off_rowp);
         w.col_part = reinterpret_cast<double*>(ws + L.off_colp);
         w.magbits = reinterpret_cast<uint32_t*>(ws + L.off_magbits);
@@ -342,18 +441,11 @@ static int build_work(const WorkInput& in, TensorWork& w) {
         w.vsum = reinterpret_cast<double*>(ws + L.off_vsum);
         w.vcs = reinterpret_cast<float*>(ws + L.off_vcs);
         w.fin = reinterpret_cast<uint32_t*>(ws + L.off_fin);
-        w.ct = t.ct; w.rt = t.rt; w.tile_rows = t.tile_rows;
-        w.stats_wgs = t.ct * t.rt;
         w.nr = ceil_div(in.R, kFinRowsPerWg);
         w.nbw = std::max<int64_t>(1, std::min<int64_t>(1024, ceil_div(nb, kFinBlocksPerWg)));
         const bool contig_g = (in.gs1 == 1 && in.gs0 == in.C);
         const bool contig_p = (in.ps1 == 1 && in.ps0 == in.C);
-        w.fast_stats = contig_g && in.C >= kChunk;
-        w.lg_lanes = w.fast_stats ? (int32_t)t.lg_lanes : -1;
-        if (w.lg_lanes >= 0) {
-            w.ct = t.ct_l; w.rt = t.rt_l; w.tile_rows = t.l_rows; w.tile_cols = t.l_cols;
-            w.stats_wgs = t.ct_l * t.rt_l;
-        }
+        set_factored_stats(w, L.tiles);
         w.fast_apply = 0;
         if (contig_g && contig_p && in.C >= kChunk && in.period >= kChunk) {
             const bool hot = !in.sr && in.C >= kRowSegCols && in.C % kChunk == 0 && in.period % kChunk == 0 &&
@@ -361,17 +453,11 @@ static int build_work(const WorkInput& in, TensorWork& w) {
                              aligned(in.idx, 8);
             w.fast_apply = hot ? 1 : 3;
         }
-        if (!w.fast_stats && tv_shape && tv_g) {
-            w.fast_stats = 2;
-            w.ct = t.ct_tv; w.rt = t.rt_tv;
-            w.tile_rows = t.tv_rows; w.tile_cols = t.tv_cols;
-            w.stats_wgs = t.ct_tv * t.rt_tv;
-        }
-        // column sums over many row tiles (embeddings: ~250-300) split into
-        // up to 8 runs (of <= 32 partials up to 256 row tiles), so no thread
-        // waits on a long load chain
+        // column sums over many granules split into up to 8 runs (of <= 32
+        // values up to 256 of them), so no thread waits on a long load chain
+        const int64_t col_values = w.fast_stats == 2 ? w.f_rt : ceil_div(in.R, w.gran);
         w.csplit = 1;
-        while (w.csplit < 8 && ceil_div(w.rt, (int64_t)w.csplit) > 32) w.csplit *= 2;
+        while (w.csplit < 8 && ceil_div(col_values, (int64_t)w.csplit) > 32) w.csplit *= 2;
         w.nc = ceil_div(in.C, kThreads / w.csplit);
         w.fin_wgs = w.nr + w.nc + w.nbw;
         // the view apply reads v_row and sqrt(v_col) (v_col on the fp32
@@ -414,9 +500,7 @@ static int build_work(const WorkInput& in, TensorWork& w) {
             const bool g_contig = in.gs1 == 1 && in.gs0 == in.C;
             const bool p_contig = in.ps1 == 1 && in.ps0 == in.C;
             if (tv_shape && tv_g) {
-                const FactTiles t = FactTiles::make(in.R, in.C, in.period, in.launch_elems);
-                w.ct = t.ct_tv; w.rt = t.rt_tv; w.tile_rows = t.tv_rows; w.tile_cols = t.tv_cols;
-                w.stats_wgs = t.ct_tv * t.rt_tv;
+                set_tiles(w, FactTiles::make(in.R, in.C, in.period, false).tv);
                 w.fast_stats = 2;
                 w.det_rec = nullptr;  // the view tiles accumulate into the shards
             } else if (!g_contig) {
@@ -452,9 +536,7 @@ static int build_work(const WorkInput& in, TensorWork& w) {
         }
         w.a_lg = 0;
         while ((kChunk << w.a_lg) < w.a_cols) ++w.a_lg;
-        w.a_steps = in.launch_elems < kSmallApplyElems ? 2 : kRowsPerTask;
-        const int64_t task_rows = (int64_t)w.a_steps * (64 >> w.a_lg);
-        w.apply_wgs = ceil_div(w.a_segs * ceil_div(in.R, task_rows), (int64_t)kWaves);
+        set_apply_steps(w, N);
     }
     if (w.fast_apply == 2)
         w.apply_wgs = ceil_div(ceil_div(in.R, kTv) * ceil_div(in.C, kTv), (int64_t)kWaves * kTvTilesPerWave);
@@ -564,34 +646,79 @@ struct MtLayout {
     std::vector<Seg> segs;
     std::vector<int32_t> coarse;
     std::vector<Launch> launches;
+    size_t part_bytes = 0;  // granule partials
 };
 
-static void plan_multi(const std::vector<TensorWork>& works, MtLayout& L) {
-    L.works = works;
+// Granule partials of one call: at most so many bytes (a decoder layer of the
+// Llama-3-8B set takes 30 MB; launches of half a billion elements and more run
+// on tiles and take none).  Tensors past it keep their tiles as workgroups, with
+// the same sums.
+constexpr size_t kGranuleBytes = (size_t)64 << 20;
+
+// Stats launch of a tensor.  Block-path tensors other than transposed views
+// join the factored launches of their dtype (the kernels branch per tensor):
+// two launches fewer per step when both paths occur.
+static GroupKey stats_key(const TensorWork& w) {
+    if (w.mode == 1 && w.fast_stats != 2) return GroupKey{0, w.dtype, 1, 0};
+    return GroupKey{w.mode, w.dtype, w.fast_stats, 0};
+}
+
+static int64_t group_elems(const std::vector<TensorWork>& works, const std::vector<int>& group) {
+    int64_t n = 0;
+    for (int t : group) n += works[(size_t)t].N;
+    return n;
+}
+
+// Granules as workgroups for those tensors of a stats launch that want it,
+// partials from address at + used on, within cap bytes.
+static void cut_stats(std::vector<TensorWork>& works, const std::vector<int>& group, uintptr_t at, size_t cap,
+                      size_t& used) {
+    const int64_t elems = group_elems(works, group);
+    for (int t : group) {
+        TensorWork& w = works[(size_t)t];
+        if (!wants_granules(w, elems)) continue;
+        const size_t bytes = align256(sizeof(double) * (size_t)granules(w).doubles);
+        if (used + bytes > cap) continue;
+        if (bytes > 0) w.part = reinterpret_cast<double*>(at + used);
+        used += bytes;
+        take_granules(w);
+    }
+}
+
+// Cohort of consecutive tensors that starts at c0: its end.
+static int cohort_end(const std::vector<TensorWork>& works, int c0) {
+    const int64_t limit = cohort_limit();
+    const int n = (int)works.size();
+    int c1 = c0;
+    int64_t acc = 0;
+    while (c1 < n && (c1 == c0 || acc + works[(size_t)c1].N <= limit)) acc += works[(size_t)c1++].N;
+    return c1;
+}
+
+// part: part_cap bytes for granule partials (a device address, or for a plan the
+// offset in its buffer).
+static void plan_multi(const std::vector<TensorWork>& works_in, uintptr_t part, size_t part_cap, MtLayout& L) {
+    L.works = works_in;
     L.segs.clear();
     L.coarse.clear();
     L.launches.clear();
+    L.part_bytes = 0;
+    std::vector<TensorWork>& works = L.works;
     const int n = (int)works.size();
-    const int64_t limit = cohort_limit();
     int c0 = 0, cohort = 0;
     while (c0 < n) {
-        int c1 = c0;
-        int64_t acc = 0;
-        while (c1 < n && (c1 == c0 || acc + works[(size_t)c1].N <= limit)) acc += works[(size_t)c1++].N;
+        const int c1 = cohort_end(works, c0);
         // phases in launch order: 0 stats, 1 finalize, 3 mean(v_row), 2 apply
         for (int phase : {0, 1, 3, 2}) {
             std::map<GroupKey, std::vector<int>> groups;
             for (int t = c0; t < c1; ++t) {
                 const TensorWork& w = works[(size_t)t];
-                GroupKey k{w.mode, w.dtype, 0, 0};
-                if (phase == 0) k.fast = w.fast_stats;
-                if (phase == 2) { k.fast = w.fast_apply; k.sr = w.sr; }
-                if (phase == 1 || phase == 3) k = GroupKey{0, 0, 0, 0};
-                // block-path tensors other than transposed views join the
-                // factored launches of their dtype (the kernels branch per
-                // tensor): two launches fewer per step when both paths occur
-                if (w.mode == 1 && phase == 0 && k.fast != 2) k = GroupKey{0, w.dtype, 1, 0};
-                if (w.mode == 1 && phase == 2 && k.fast != 2) k.mode = 0;
+                GroupKey k{0, 0, 0, 0};
+                if (phase == 0) k = stats_key(w);
+                if (phase == 2) {
+                    k = GroupKey{w.mode, w.dtype, w.fast_apply, w.sr};
+                    if (w.fast_apply != 2) k.mode = 0;  // as in stats_key
+                }
                 if (phase == 3 && w.mode != 0) continue;
                 groups[k].push_back(t);
             }
@@ -600,7 +727,14 @@ static void plan_multi(const std::vector<TensorWork>& works, MtLayout& L) {
             // the finalize reads next, stay cached (measured on the Qwen3-4B
             // set: stats 2.04 -> 1.98 ms, finalize 65 -> 58 us)
             std::vector<std::pair<GroupKey, std::vector<int>>> ordered(groups.begin(), groups.end());
+            if (phase == 2) {
+                for (const auto& kv : ordered) {
+                    const int64_t elems = group_elems(works, kv.second);
+                    for (int t : kv.second) set_apply_steps(works[(size_t)t], elems);
+                }
+            }
             if (phase == 0) {
+                for (const auto& kv : ordered) cut_stats(works, kv.second, part, part_cap, L.part_bytes);
                 std::stable_sort(ordered.begin(), ordered.end(), [](const auto& a, const auto& b) {
                     return (a.first.fast == 2) > (b.first.fast == 2);
                 });
@@ -824,11 +958,17 @@ static size_t multi_scratch_bytes(int n_works, size_t n_segs) {
 // ------------------------------------------------------------ capturable plan
 
 // Descriptor image upload as a kernel node: src is the plan's pinned host
-// image (device-visible), dst the plan's device buffer; n16 16-byte words.
-__global__ __launch_bounds__(kThreads) void k_image_copy(const uint4* __restrict__ src, uint4* __restrict__ dst,
-                                                         int64_t n16) {
-    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n16; i += (int64_t)gridDim.x * kThreads)
-        dst[i] = src[i];
+// image (device-visible), dst the plan's device buffer; n 8-byte words.  The
+// first n_works descriptors' partials become addresses in that buffer.
+__global__ __launch_bounds__(kThreads) void k_image_copy(const uint64_t* __restrict__ src, uint64_t* __restrict__ dst,
+                                                         int64_t n, int64_t n_works) {
+    constexpr int64_t kWords = sizeof(TensorWork) / 8, kPart = offsetof(TensorWork, part) / 8;
+    static_assert(sizeof(TensorWork) % 8 == 0 && offsetof(TensorWork, part) % 8 == 0, "whole words");
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kThreads) {
+        uint64_t v = src[i];
+        if (v != 0 && i < n_works * kWords && i % kWords == kPart) v += reinterpret_cast<uint64_t>(dst);
+        dst[i] = v;
+    }
 }
 
 __device__ __forceinline__ double capt_lr(const gefenx_capt_desc& c) {
@@ -885,7 +1025,8 @@ struct gefenx_mt_plan {
     size_t capt_off = 0;
     int n_capt = 0;
     int64_t* counter = nullptr;
-    size_t bytes = 0;
+    size_t image_bytes = 0;    // image and capturable descriptors
+    size_t bytes = 0;          // of the device buffer
     int device = 0;
     void* host = nullptr;      // pinned image
     void* host_dev = nullptr;  // its device-visible address
@@ -912,6 +1053,7 @@ static int check_dtype(int dtype, const char* fn) {
 // host use -- kernel arguments, the clearing launch -- goes through the
 // resolved pointer.
 static __device__ __align__(256) unsigned char scratch[GEFENX_NOALLOC_SCRATCH_BYTES];
+static_assert(kNoallocScratch == GEFENX_NOALLOC_SCRATCH_BYTES, "FactoredWs::make keeps tensors within it");
 
 constexpr int kScratchDevices = 64;
 static void* g_scratch_addr[kScratchDevices];  // per device; nullptr until resolved
@@ -979,6 +1121,13 @@ static int factored_input(const char* fn, void* p, const void* grad, int dtype, 
     return GEFENX_OK;
 }
 
+// Granules as workgroups of a single tensor's launch where they fit at mem.
+static void cut_single(TensorWork& w, void* mem, size_t cap) {
+    if (!wants_granules(w, w.N) || align256(sizeof(double) * (size_t)granules(w).doubles) > cap) return;
+    (w.fast_stats == 2 ? w.row_part : w.col_part) = static_cast<double*>(mem);
+    take_granules(w);
+}
+
 int gefenx_factored_update(
     void* p, const void* grad, int dtype, int64_t rows, int64_t cols,
     int64_t ps0, int64_t ps1, int64_t gs0, int64_t gs1,
@@ -998,10 +1147,11 @@ int gefenx_factored_update(
     if (rc || empty) return rc;
     if (!workspace) return set_error(GEFENX_EINVAL, "gefenx_factored_update: null workspace");
     in.workspace = workspace; in.ws_bytes = workspace_bytes;
-    in.launch_elems = in.ws_elems = in.R * in.C;
     TensorWork w;
     rc = build_work(in, w);
     if (rc) return rc;
+    const size_t need = gefenx_workspace_bytes(GEFENX_WS_FACTORED, rows, cols, w.nb);
+    cut_single(w, static_cast<char*>(workspace) + need, workspace_bytes - need);
     return run_single(w, static_cast<hipStream_t>(stream));
 }
 
@@ -1022,7 +1172,7 @@ int gefenx_factored_update_noalloc(
                             inv_bias_correction_1, weight_decay_factor, stochastic_round, rng_seed, step_scalars,
                             seed_dev, in, empty);
     if (rc || empty) return rc;
-    const FactoredWs L = FactoredWs::make(rows, cols, rows * cols / period, kCoarseTiles);
+    const FactoredWs L = FactoredWs::make(rows, cols, rows * cols / period);
     if (L.total > (size_t)GEFENX_NOALLOC_SCRATCH_BYTES)
         return set_error(GEFENX_EINVAL, "%s: a [%lld, %lld] parameter with period %lld needs %zu bytes of scratch; "
                          "the static scratch holds %zu (use gefenx_factored_update with a workspace)", fn,
@@ -1033,10 +1183,10 @@ int gefenx_factored_update_noalloc(
     if (rc) return rc;
     in.workspace = ptr;
     in.ws_bytes = GEFENX_NOALLOC_SCRATCH_BYTES;
-    in.launch_elems = in.ws_elems = kCoarseTiles;
     TensorWork w;
     rc = build_work(in, w);
     if (rc) return rc;
+    cut_single(w, static_cast<char*>(ptr) + L.total, (size_t)GEFENX_NOALLOC_SCRATCH_BYTES - L.total);
     // the accumulators that must start at zero: block maxima and the
     // finalize counter (the previous call on this GPU left them zero unless
     // it failed part-way)
@@ -1081,7 +1231,6 @@ int gefenx_block_update(
     in.sr = stochastic_round ? 1 : 0; in.seed = (uint64_t)rng_seed;
     in.step_scalars = step_scalars; in.seed_dev = seed_dev;
     in.workspace = workspace; in.ws_bytes = workspace_bytes;
-    in.launch_elems = in.ws_elems = in.R * in.C;
     TensorWork w;
     rc = build_work(in, w);
     if (rc) return rc;
@@ -1108,7 +1257,6 @@ int gefenx_momentum_apply(
     in.lerp_w = (float)(1.0 - beta1); in.beta2 = 0.0f; in.alpha2 = 0.0f; in.eps = 0.0f;
     in.sc = StepScalars{(float)lr, 1.0f, 1.0f, 1.0f};
     in.workspace = workspace; in.ws_bytes = workspace_bytes;
-    in.launch_elems = in.ws_elems = in.R * in.C;
     TensorWork w;
     rc = build_work(in, w);
     if (rc) return rc;
@@ -1118,8 +1266,7 @@ int gefenx_momentum_apply(
 }
 
 static int desc_to_work(const gefenx_tensor_desc& d, int i, const void* const* qtables, int sr,
-                        int64_t seed, const float* step_scalars, const int64_t* seed_dev, int64_t launch_elems,
-                        TensorWork& w) {
+                        int64_t seed, const float* step_scalars, const int64_t* seed_dev, TensorWork& w) {
     int rc = check_dtype(d.dtype, "gefenx_multi_tensor_step");
     if (rc) return rc;
     const int64_t N = d.rows * d.cols;
@@ -1147,7 +1294,6 @@ static int desc_to_work(const gefenx_tensor_desc& d, int i, const void* const* q
     in.sr = sr ? 1 : 0; in.seed = (uint64_t)seed;
     in.step_scalars = step_scalars; in.seed_dev = seed_dev;
     in.workspace = d.workspace;
-    in.launch_elems = launch_elems; in.ws_elems = N;
     in.ws_bytes = d.factored ? gefenx_workspace_bytes(GEFENX_WS_FACTORED, d.rows, d.cols, N / d.period)
                              : gefenx_workspace_bytes(GEFENX_WS_BLOCK, d.rows, d.cols, N / d.period);
     return build_work(in, w);
@@ -1166,24 +1312,19 @@ static void merge_small_applies(std::vector<TensorWork>& works) {
     }
 }
 
-static int build_layout(const gefenx_tensor_desc* descs, int n, const void* const* qtables, int sr,
-                        int64_t seed, const float* const* step_scalars, const int64_t* seed_dev, MtLayout& L) {
+static int build_works(const gefenx_tensor_desc* descs, int n, const void* const* qtables, int sr, int64_t seed,
+                       const float* const* step_scalars, const int64_t* seed_dev, std::vector<TensorWork>& works) {
     if (n < 0 || (n > 0 && (!descs || !qtables)))
         return set_error(GEFENX_EINVAL, "gefenx_multi_tensor_step: bad descriptor array");
-    std::vector<TensorWork> works;
     works.reserve((size_t)n);
-    int64_t total = 0;
-    for (int i = 0; i < n; ++i) total += descs[i].rows * descs[i].cols;
     for (int i = 0; i < n; ++i) {
         if (descs[i].rows * descs[i].cols == 0) continue;  // empty tensors are a no-op
         TensorWork w;
-        int rc = desc_to_work(descs[i], i, qtables, sr, seed, step_scalars ? step_scalars[i] : nullptr,
-                              seed_dev, total, w);
+        int rc = desc_to_work(descs[i], i, qtables, sr, seed, step_scalars ? step_scalars[i] : nullptr, seed_dev, w);
         if (rc) return rc;
         works.push_back(w);
     }
     merge_small_applies(works);
-    plan_multi(works, L);
     return GEFENX_OK;
 }
 
@@ -1193,14 +1334,56 @@ size_t gefenx_multi_tensor_scratch_bytes(int n) {
     return multi_scratch_bytes(n, (size_t)n * 4);
 }
 
+size_t gefenx_multi_tensor_scratch_bytes_for(const gefenx_tensor_desc* descs, int n) {
+    const size_t base = gefenx_multi_tensor_scratch_bytes(n);
+    if (n <= 0 || !descs) return base;
+    // the stats launches of these tensors, from what decides their cut (views of
+    // the block path leave no partials)
+    std::vector<TensorWork> works;
+    std::map<GroupKey, std::vector<int>> groups;
+    size_t used = 0;
+    int64_t largest = 0;
+    for (int i = 0; i < n; ++i) largest = std::max<int64_t>(largest, descs[i].rows * descs[i].cols);
+    if (largest <= kFactGranuleElems) return base;  // a granule each
+    works.reserve((size_t)n);
+    for (int i = 0; i < n; ++i) {
+        const gefenx_tensor_desc& d = descs[i];
+        if (d.rows <= 0 || d.cols <= 0 || d.period <= 0 || (d.rows * d.cols) % d.period != 0) continue;
+        TensorWork w;
+        std::memset(&w, 0, sizeof(w));
+        w.R = d.rows; w.C = d.cols; w.P = d.period; w.N = d.rows * d.cols;
+        w.gs0 = d.gs0; w.gs1 = d.gs1; w.grad = d.grad; w.idx = d.m_codebook;
+        w.dtype = d.dtype; w.mode = d.factored ? 0 : 1;
+        if (d.factored) {
+            set_factored_stats(w, FactoredWs::make(d.rows, d.cols, w.N / d.period).tiles);
+        } else if (d.rows > 1 && view_strides(d.rows, d.gs0, d.gs1, d.dtype, d.grad)) {
+            w.fast_stats = 2;
+            set_tiles(w, FactTiles::make(d.rows, d.cols, d.period, false).tv);
+        }
+        works.push_back(w);
+    }
+    for (int c0 = 0; c0 < (int)works.size();) {
+        const int c1 = cohort_end(works, c0);
+        groups.clear();
+        for (int t = c0; t < c1; ++t) groups[stats_key(works[(size_t)t])].push_back(t);
+        for (const auto& kv : groups) cut_stats(works, kv.second, 256, kGranuleBytes, used);
+        c0 = c1;
+    }
+    return base + used;
+}
+
 int gefenx_multi_tensor_step(const gefenx_tensor_desc* descs, int n, const void* const* qtables_dev,
                              int stochastic_round, int64_t rng_seed, void* desc_scratch_dev,
                              size_t desc_scratch_bytes, void* stream) {
-    MtLayout L;
-    int rc = build_layout(descs, n, qtables_dev, stochastic_round, rng_seed, nullptr, nullptr, L);
+    std::vector<TensorWork> works;
+    int rc = build_works(descs, n, qtables_dev, stochastic_round, rng_seed, nullptr, nullptr, works);
     if (rc) return rc;
-    if (L.works.empty()) return GEFENX_OK;
+    if (works.empty()) return GEFENX_OK;
     if (!desc_scratch_dev) return set_error(GEFENX_EINVAL, "gefenx_multi_tensor_step: null scratch");
+    const size_t base = gefenx_multi_tensor_scratch_bytes(n);
+    MtLayout L;
+    plan_multi(works, reinterpret_cast<uintptr_t>(desc_scratch_dev) + base,
+               desc_scratch_bytes > base ? std::min(desc_scratch_bytes - base, kGranuleBytes) : 0, L);
     return run_multi(L, desc_scratch_dev, desc_scratch_bytes, static_cast<hipStream_t>(stream));
 }
 
@@ -1222,23 +1405,29 @@ int gefenx_mt_plan_create(const gefenx_tensor_desc* descs, int n, const float* c
     }
     const int64_t* seed_dev = counter_dev ? counter_dev + 2 : nullptr;
     auto plan = std::make_unique<gefenx_mt_plan>();
-    int rc = build_layout(descs, n, qtables_dev, stochastic_round, rng_seed, step_scalars, seed_dev, plan->L);
+    std::vector<TensorWork> works;
+    int rc = build_works(descs, n, qtables_dev, stochastic_round, rng_seed, step_scalars, seed_dev, works);
     if (rc) return rc;
+    // [image | capturable descriptors | granule partials]
+    const size_t capt_bytes = align256(sizeof(gefenx_capt_desc) * (size_t)n_capt);
+    const size_t part_off = gefenx_multi_tensor_scratch_bytes(n) + capt_bytes;
+    plan_multi(works, part_off, kGranuleBytes, plan->L);
     plan->im = image_layout(plan->L, 0);
     plan->capt_off = plan->im.end;
     plan->n_capt = n_capt;
     plan->counter = counter_dev;
     (void)hipGetDevice(&plan->device);
-    plan->bytes = std::max<size_t>(plan->capt_off + align256(sizeof(gefenx_capt_desc) * (size_t)n_capt), 256);
+    plan->image_bytes = std::max<size_t>(plan->capt_off + capt_bytes, 256);
+    plan->bytes = plan->L.part_bytes > 0 ? part_off + plan->L.part_bytes : plan->image_bytes;
     // Pinned allocation is host work; let it through while this thread's
     // stream is being captured.
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     (void)hipThreadExchangeStreamCaptureMode(&mode);
-    const hipError_t e = hipHostMalloc(&plan->host, plan->bytes, hipHostMallocDefault);
+    const hipError_t e = hipHostMalloc(&plan->host, plan->image_bytes, hipHostMallocDefault);
     (void)hipThreadExchangeStreamCaptureMode(&mode);
     if (e != hipSuccess) {
         plan->host = nullptr;
-        return set_error(GEFENX_ENOMEM, "gefenx_mt_plan_create: pinned image of %zu bytes failed", plan->bytes);
+        return set_error(GEFENX_ENOMEM, "gefenx_mt_plan_create: pinned image of %zu bytes failed", plan->image_bytes);
     }
     if (hipHostGetDevicePointer(&plan->host_dev, plan->host, 0) != hipSuccess) {
         (void)hipHostFree(plan->host);
@@ -1246,7 +1435,7 @@ int gefenx_mt_plan_create(const gefenx_tensor_desc* descs, int n, const float* c
         return set_error(GEFENX_ELAUNCH, "gefenx_mt_plan_create: pinned image has no device address");
     }
     char* h = static_cast<char*>(plan->host);
-    std::memset(h, 0, plan->bytes);
+    std::memset(h, 0, plan->image_bytes);
     write_image(plan->L, plan->im, h);
     if (n_capt > 0) std::memcpy(h + plan->capt_off, capt, sizeof(gefenx_capt_desc) * (size_t)n_capt);
     *plan_out = plan.release();
@@ -1269,10 +1458,10 @@ int gefenx_mt_plan_launch(gefenx_mt_plan* plan, void* dev_buf, size_t dev_bytes,
     const bool capturing = cs != hipStreamCaptureStatusNone;
     const dim3 block(kThreads);
     if (capturing || !plan->uploaded || plan->uploaded_to != dev_buf || plan->uploaded_on != s) {
-        const int64_t n16 = (int64_t)(plan->bytes / 16);
-        const unsigned grid = (unsigned)std::min<int64_t>((n16 + kThreads - 1) / kThreads, 1024);
-        hipLaunchKernelGGL(k_image_copy, dim3(grid), block, 0, s, static_cast<const uint4*>(plan->host_dev),
-                           static_cast<uint4*>(dev_buf), n16);
+        const int64_t n8 = (int64_t)(plan->image_bytes / 8);
+        const unsigned grid = (unsigned)std::min<int64_t>((n8 + kThreads - 1) / kThreads, 1024);
+        hipLaunchKernelGGL(k_image_copy, dim3(grid), block, 0, s, static_cast<const uint64_t*>(plan->host_dev),
+                           static_cast<uint64_t*>(dev_buf), n8, (int64_t)plan->L.works.size());
         int rc = launch_check("plan image copy");
         if (rc) return rc;
         if (!capturing) {

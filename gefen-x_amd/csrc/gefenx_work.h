@@ -16,6 +16,7 @@ constexpr int64_t kApplyChunksPerThread = 8;   // apply: 4 iterations of 2 chunk
 constexpr int64_t kFinBlocksPerWg = 1024;
 constexpr int64_t kDefaultCohortElems = 0;  // one cohort per step (see cohort_limit)
 constexpr int kTv = 64;                        // transposed views: square tiles of this side
+constexpr int kTvLdsBlocks = 512;              // ... stats: LDS block accumulators per workgroup
 constexpr int kTvTilesPerWave = 2;             // apply: consecutive tiles per wave
 constexpr int64_t kRowSegCols = 64 * kChunk;   // apply_tasks: most columns of a task
 constexpr int kRowsPerTask = 8;                // apply_tasks: row steps of a task
@@ -55,7 +56,14 @@ struct TensorWork {
     int64_t R, C, N, P, nb;
     double invC, invP;
     int64_t ps0, ps1, gs0, gs1;
-    int64_t ct, rt, tile_rows, tile_cols, shards;  // tile_cols: lane tiles and transposed views
+    // factored stats: column tiles of the launch, rows and columns of a
+    // workgroup, rows (views: columns) of a granule
+    int64_t ct, tile_rows, tile_cols, gran, shards;
+    // finalize: row and column tiles; column (row) partials per tile and in all
+    int64_t f_rt, f_ct, pc_per, pc_n, pr_per, pr_n;
+    // where a granule is a workgroup: the granules' column partials (views: row
+    // partials), in a plan's host image their byte offset in its buffer; else null
+    double* part;
     int64_t stats_wgs, nr, nc, nbw, fin_wgs, apply_wgs;
     int64_t det_elems;   // block stats: elements per workgroup
     int64_t fB, fP;          // flat apply: block advance for a stride of 256*8 elements
@@ -120,6 +128,14 @@ __device__ __forceinline__ float ref_step(const RefStep& r, float v_row, float v
 // mean(v_row) as finalize stored it (already clamped at FLT_MIN).
 __device__ __forceinline__ float stored_mean(const TensorWork& w) {
     return __uint_as_float(*gbl(w.fin + 1));
+}
+
+// Where the stats leave their column and row partials.
+__device__ __forceinline__ double* col_partials(const TensorWork& w) {
+    return w.part != nullptr && w.fast_stats != 2 ? w.part : w.col_part;
+}
+__device__ __forceinline__ double* row_partials(const TensorWork& w) {
+    return w.part != nullptr && w.fast_stats == 2 ? w.part : w.row_part;
 }
 
 struct Seg {

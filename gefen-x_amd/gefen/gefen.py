@@ -80,6 +80,8 @@ _DESC_DTYPE = np.dtype(_native.TensorDesc)
 _DESC_STRUCT = struct.Struct("<" + "".join({"c_void_p": "Q", "c_long": "q", "c_int": "i", "c_float": "f"}[t.__name__]
                                            for _, t in _native.TensorDesc._fields_))
 _DESC_BYTES = ctypes.sizeof(_native.TensorDesc)
+# bytes of multi-tensor scratch that an optimizer keeps between steps
+_MT_SCRATCH_KEPT = 1 << 20
 _STEP_DTYPES = frozenset((torch.float32, torch.float16, torch.bfloat16))
 
 
@@ -976,14 +978,17 @@ class Gefen(torch.optim.Optimizer):
         for dt in dtypes:
             qt[_fused._dtype_code(dt)] = _fused.quant_table(cb, dt).data_ptr()
         qt_arr = (ctypes.c_void_p * 3)(*qt)
-        need = int(lib.gefenx_multi_tensor_scratch_bytes(n))
+        descs_ptr = ctypes.addressof(ctypes.c_char.from_buffer(descs))
+        need = int(lib.gefenx_multi_tensor_scratch_bytes_for(descs_ptr, n))
         scratch = self._mt_scratch.get(device)
-        if scratch is None or scratch.numel() < need:
+        if need > _MT_SCRATCH_KEPT:  # partial sums: memory of this call alone
+            scratch = torch.empty(need, dtype=torch.uint8, device=device)
+        elif scratch is None or scratch.numel() < need:
             scratch = torch.empty(need, dtype=torch.uint8, device=device)
             self._mt_scratch[device] = scratch
         with _on_device(device):
             _native.check(lib.gefenx_multi_tensor_step(
-                ctypes.addressof(ctypes.c_char.from_buffer(descs)), n, qt_arr, 1 if self._stochastic_round else 0,
+                descs_ptr, n, qt_arr, 1 if self._stochastic_round else 0,
                 self._gefen_global_step, scratch.data_ptr(), scratch.numel(),
                 torch.cuda.current_stream(device).cuda_stream), "multi-tensor step")
 

@@ -122,6 +122,7 @@ SIGNATURES = {
     "gefenx_exact_dp_device": (_I, [_P, _P, _I, _I, _I, _P, _P]),
     "gefenx_multi_tensor_step": (_I, [_P, _I, _P, _I, _I64, _P, _SZ, _P]),
     "gefenx_multi_tensor_scratch_bytes": (_SZ, [_I]),
+    "gefenx_multi_tensor_scratch_bytes_for": (_SZ, [_P, _I]),
     "gefenx_mt_plan_create": (_I, [_P, _I, _P, _P, _I, _I64, _P, _I, _P, _P]),
     "gefenx_mt_plan_device_bytes": (_SZ, [_P]),
     "gefenx_mt_plan_launch": (_I, [_P, _P, _SZ, _P]),

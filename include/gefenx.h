@@ -100,7 +100,10 @@ size_t gefenx_workspace_bytes(int kind, int64_t rows, int64_t cols, int64_t num_
  *   v_row fp32 [rows]; v_col fp32 [cols]; all mutated in place.
  *   step_scalars: NULL, or a device fp32[4] = [lr, 1/bc2, 1/bc1, wd_factor]
  *   overriding the host scalars (capturable mode);
- *   seed_dev: NULL or a device int64 overriding rng_seed.
+ *   seed_dev: NULL or a device int64 overriding rng_seed;
+ *   workspace: bytes beyond the required ones hold finer partial sums (a
+ *   quarter of a byte per element is always enough), so that a tensor of a few
+ *   million elements fills the GPU.  The results do not depend on them.
  * ---------------------------------------------------------------------- */
 int gefenx_factored_update(
     void* p, const void* grad, int dtype, int64_t rows, int64_t cols,
@@ -307,6 +310,11 @@ int gefenx_multi_tensor_step(const gefenx_tensor_desc* descs, int n,
 /* Bytes of device scratch gefenx_multi_tensor_step needs for n tensors
  * (descriptors and the workgroup -> tensor segment tables). */
 size_t gefenx_multi_tensor_scratch_bytes(int n);
+
+/* The same plus what a call with these descriptors can use for finer partial
+ * sums (at most 64 MiB, 0 for large calls): with it, launches that would leave
+ * CUs idle are cut finer.  The results do not depend on it. */
+size_t gefenx_multi_tensor_scratch_bytes_for(const gefenx_tensor_desc* descs, int n);
 
 /* ------------------------------------------------------------------------
  * Capturable step (graph capture / replay).  Replaces the reference's
