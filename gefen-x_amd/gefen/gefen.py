@@ -1195,8 +1195,7 @@ class Gefen(torch.optim.Optimizer):
                 grad = p.grad
                 if grad is None or grad.numel() == 0:
                     continue
-                factored = (self._factored_v_2d and p.ndim == 2
-                            and (type(p) is nn.Parameter or not hasattr(p, "placements")))
+                factored = self._factored_v_2d and p.ndim == 2 and not hasattr(p, "placements")
                 if capturing and "step" not in self.state[p]:
                     raise RuntimeError("Gefen capturable: parameter {} has no state yet; its first step runs "
                                        "eagerly".format(name))
