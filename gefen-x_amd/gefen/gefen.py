@@ -28,7 +28,6 @@ from __future__ import annotations
 
 import contextlib
 import ctypes
-import functools
 import logging
 import math
 import os
@@ -85,9 +84,17 @@ _MT_SCRATCH_KEPT = 1 << 20
 _STEP_DTYPES = frozenset((torch.float32, torch.float16, torch.bfloat16))
 
 
-@functools.lru_cache(maxsize=4096)
+_WORKSPACE_BYTES = {}  # (kind, rows, cols, blocks) -> bytes; a plain dict, which tracing looks into without a warning
+
+
 def _workspace_bytes(kind: int, rows: int, cols: int, nb: int) -> int:
-    return int(_native.load().gefenx_workspace_bytes(kind, rows, cols, nb))
+    key = (kind, rows, cols, nb)
+    found = _WORKSPACE_BYTES.get(key)
+    if found is None:
+        if len(_WORKSPACE_BYTES) >= 4096:
+            _WORKSPACE_BYTES.clear()
+        found = _WORKSPACE_BYTES[key] = int(_native.load().gefenx_workspace_bytes(kind, rows, cols, nb))
+    return found
 
 
 def _on_device(device):

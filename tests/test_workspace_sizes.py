@@ -2,8 +2,10 @@
 from __future__ import annotations
 
 import ctypes
+import warnings
 
 import pytest
+import torch
 
 from gefen.kernels import _native
 
@@ -57,3 +59,20 @@ def test_scratch_follows_the_launches(lib):
     assert _extra(lib, large + [(4096, 4096, bf16)]) == 0
     assert 0 < _extra(lib, [(14336, 4096, bf16)] * 6 + [(4096, 4096, bf16)] * 4) <= 64 << 20
     assert _extra(lib, [(64, 64, f32)] * 20) == 0
+
+
+def test_workspace_memo_traces_without_a_warning(lib):
+    """torch.compile of a step reaches the memo; a functools cache there made it
+    warn that Dynamo ignores the cache."""
+    from gefen import gefen
+    key = (_native.WS_FACTORED, 64, 64, 64)
+    gefen._workspace_bytes(*key)
+
+    def f(x):
+        return x + gefen._workspace_bytes(*key)
+
+    torch._dynamo.reset()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        y = torch.compile(f, backend="eager")(torch.zeros(2))
+    assert y[0].item() == lib.gefenx_workspace_bytes(*key)
