@@ -412,8 +412,8 @@ class GefenMuon(Gefen):
                     raise ValueError(_swapped_param_groups_error(p))
 
     def _ns_batch_limit(self, rows, cols, itemsize):
-        m, n = min(rows, cols), max(rows, cols)
-        per_item = 2 * (3 * m * n + 2 * m * m) + itemsize * rows * cols
+        # the products' buffers are padded to multiples of 64, which thin matrices fill many times
+        per_item = int(_native.load().gefenx_ns_workspace_bytes(1, rows, cols)) + itemsize * rows * cols
         return max(1, NS_WORKSPACE_BUDGET // max(per_item, 1))
 
     @torch.no_grad()

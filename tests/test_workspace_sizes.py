@@ -76,3 +76,15 @@ def test_workspace_memo_traces_without_a_warning(lib):
         warnings.simplefilter("error")
         y = torch.compile(f, backend="eager")(torch.zeros(2))
     assert y[0].item() == lib.gefenx_workspace_bytes(*key)
+
+
+@pytest.mark.parametrize("rows,cols", [(4096, 4096), (4096, 8), (8, 14336), (1, 4096), (65, 1000)])
+def test_newton_schulz_batches_keep_their_budget(lib, rows, cols):
+    """The matrices of one batch fit the budget with their padded buffers."""
+    from gefen import GefenMuon
+    from gefen.gefen_muon import NS_WORKSPACE_BUDGET
+    opt = GefenMuon([("w", torch.nn.Parameter(torch.zeros(rows, cols)))], lr=1e-3)
+    n = opt._ns_batch_limit(rows, cols, 2)
+    assert n == 1 or lib.gefenx_ns_workspace_bytes(n, rows, cols) <= NS_WORKSPACE_BUDGET
+    one = lib.gefenx_ns_workspace_bytes(1, rows, cols) + 2 * rows * cols  # and the matrix in the stack
+    assert (n + 1) * one > NS_WORKSPACE_BUDGET
