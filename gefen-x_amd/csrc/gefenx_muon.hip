@@ -1059,10 +1059,13 @@ __global__ void __launch_bounds__(kT) k_gemm_dl(GemmArgs g) {
 // leaves the later stages' loads (kL instructions per wave and stage) in
 // flight; the bare barrier keeps the compiler from draining them.  Measured
 // against k_gemm_dl, us: 9 tiles of 128 x 128 (320 x 320, K 320) 13.2 -> 5.8;
-// 49 (1152 x 832, K 832) 19.5 -> 9.8; 133 21.2 -> 12.9; but 136 with K 6144 (a
-// lower triangle of 2048 x 2048) 71 -> 84, twice the operand traffic then
-// being what counts, and 272 42 -> 69.  (128 x 128 tiles in the same ring: no
-// gain, 13.2, 18.8 and 64 us.)
+// 49 (1152 x 832, K 832) 19.5 -> 9.8; 121 (1408 x 1408) with K 512, 2048 and 8192
+// 10.5, 24.4 and 77.6 -> 8.0, 16.4 and 52.7.  Taken while its tiles are one round
+// of workgroups, kRingTiles: 128 of 128 x 128 (512 of these) K 1024 15.0 -> 10.7,
+// but 132 (528) 15.1 -> 16.7, and 136 of a lower triangle (528) with K 6144
+// 71 -> 84.  (128 x 128 tiles in the same ring: no gain, 13.2, 18.8 and 64 us.)
+constexpr int64_t kRingTiles = 512;
+
 template <int WM, int BK>
 __global__ void __launch_bounds__(kT) k_gemm_ring(GemmArgs g) {
     constexpr int S = 4;
@@ -1439,14 +1442,15 @@ static int gemm_nt(const GemmArgs& g, int64_t batch, hipStream_t s) {
     if (g.tri && (g.M != g.N || g.Dt != g.D || g.lddt != g.ldd || g.sDt != g.sD))
         return set_error(GEFENX_EINVAL, "newton-schulz gemm: symmetric mode needs a square D mirrored into itself");
     // direct-to-LDS when K is a multiple of 64 and the operands are 16-byte
-    // aligned (every Newton-Schulz product of 64-multiple shapes), the
-    // register-staged kernel otherwise.  Direct-to-LDS products whose 256 x
+    // aligned (every Newton-Schulz product: its buffers are padded), the
+    // register-staged kernel otherwise (gefenx_gemm_nt_bf16 of other shapes, and
+    // a workspace that is not 16-byte aligned).  Direct-to-LDS products whose 256 x
     // 256 tiles (lower triangle only when symmetric) fill the 256 CUs at least
     // once take a 256 x 256 kernel (16x16x32 MFMAs when every tile is full,
     // the 32x32x16 kernel with its clamped loads and guarded epilogue
     // otherwise); smaller grids take 128 x 128 tiles (four times the
-    // workgroups), and grids that leave about half of the CUs without one 64 x
-    // 64 tiles.
+    // workgroups), and those whose 64 x 64 tiles are one round of workgroups
+    // these.
     const auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
     const bool dl = a.vec && g.K % 64 == 0 && al16(g.A) && al16(g.B);
     constexpr int bm = 128, bn = 128;
@@ -1469,10 +1473,11 @@ static int gemm_nt(const GemmArgs& g, int64_t batch, hipStream_t s) {
     a.nt_n = cdiv(g.N, bn);
     const int64_t tiles = gemm_tiles(a.nt_m, a.nt_n, g.tri) * batch;
     const dim3 grid((unsigned)tiles);
-    if (dl && tiles <= (g.K <= 1024 ? 192 : 128)) {  // k_gemm_ring's comment has both sides
+    const int64_t ring_tiles = gemm_tiles(cdiv(g.M, 64), cdiv(g.N, 64), g.tri) * batch;
+    if (dl && ring_tiles <= kRingTiles) {
         a.nt_m = cdiv(g.M, 64);
         a.nt_n = cdiv(g.N, 64);
-        hipLaunchKernelGGL((k_gemm_ring<1, 64>), dim3((unsigned)(gemm_tiles(a.nt_m, a.nt_n, g.tri) * batch)), dim3(kT), 0, s, a);
+        hipLaunchKernelGGL((k_gemm_ring<1, 64>), dim3((unsigned)ring_tiles), dim3(kT), 0, s, a);
     } else if (dl)
         hipLaunchKernelGGL((k_gemm_dl<2, 64, 2>), grid, dim3(kT), 0, s, a);
     else if (a.vec)
