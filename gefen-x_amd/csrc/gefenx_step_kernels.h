@@ -1375,9 +1375,43 @@ __device__ __forceinline__ void apply_phase(const TensorWork& w, int64_t wg, int
 // and one sqrt(v_row * scale) per chunk.
 // ====================================================================
 struct FastTables {
-    uint2 fq[kFqEntries];
+    union {
+        uint2 fq[kFqEntries];
+        struct {  // a table with several thresholds in one bucket
+            uint32_t bkt[kBuckets + 4];
+            float thr[kCodebookMax + 4];
+        } d;
+    };
     float cbr[kCodebookMax];
 };
+
+// Buckets (the last one again past the end: x = 1 lands there) and thresholds
+// (+inf past the end) for quant_dense.
+__device__ __forceinline__ void stage_dense(FastTables& s, const QTable* __restrict__ t) {
+    const GX_GLOBAL u32x4* src = gbl(reinterpret_cast<const u32x4*>(t->bucket));
+    u32x4* dst = reinterpret_cast<u32x4*>(s.d.bkt);
+#pragma unroll
+    for (int j = 0; j < kBuckets / 4 / kThreads; ++j) dst[threadIdx.x + j * kThreads] = src[threadIdx.x + j * kThreads];
+    s.d.thr[threadIdx.x] = *gbl(t->thr + threadIdx.x);
+    s.cbr[threadIdx.x] = *gbl(t->cbr + threadIdx.x);
+    if (threadIdx.x < 4) {
+        s.d.bkt[kBuckets + threadIdx.x] = *gbl(t->bucket + kBuckets - 1);
+        s.d.thr[kCodebookMax + threadIdx.x] = __builtin_inff();
+    }
+}
+
+// Nearest index for x in [-1, 1] (never NaN).  Thresholds in later buckets
+// are > x, so the first two from the bucket's base on are compared whatever
+// their bucket; a bucket that holds more goes on with the rest.
+__device__ __forceinline__ uint32_t quant_dense(float x, const FastTables& s) {
+    int b = (int)__builtin_fmaf(x, (float)(kBuckets / 2), (float)(kBuckets / 2));
+    b = b < 0 ? 0 : (b > kBuckets ? kBuckets : b);
+    const uint32_t e = s.d.bkt[b];
+    const uint32_t base = e & 0xffffu, cnt = e >> 16;
+    uint32_t idx = base + (s.d.thr[base] < x ? 1u : 0u) + (s.d.thr[base + 1] < x ? 1u : 0u);
+    for (uint32_t j = 2; j < cnt; ++j) idx += s.d.thr[base + j] < x ? 1u : 0u;
+    return idx;
+}
 
 // All loads of a thread's share are issued before the first LDS write.
 __device__ __forceinline__ void stage_fast(FastTables& s, const QTable* __restrict__ t) {
@@ -1410,7 +1444,10 @@ struct SrTables {
     uint32_t lut[kBuckets];
 };
 
-__device__ __forceinline__ void stage_tabs(FastTables& s, const QTable* __restrict__ t) { stage_fast(s, t); }
+__device__ __forceinline__ void stage_tabs(FastTables& s, const QTable* __restrict__ t) {
+    if (t->max_cnt > 1) stage_dense(s, t);
+    else stage_fast(s, t);
+}
 __device__ __forceinline__ void stage_tabs(SrTables& s, const QTable* __restrict__ t) {
     const int kk = t->k;
     for (int j = threadIdx.x; j < kCodebookMax + 2; j += kThreads) {
@@ -1554,7 +1591,9 @@ __device__ __forceinline__ void flat_load(const FastArgs<DT>& a, const Pos& ps, 
 // (stochastic rounding).  general_q: the table may hold several thresholds per
 // bucket (the fq entries do not describe it), so every element takes the exact
 // search.
-template <int DT, int MODE, int LF, class Tabs>
+// LDSQ: ft was staged for a general_q table (else such elements search it in
+// global memory).
+template <int DT, int MODE, int LF, bool LDSQ = true, class Tabs>
 __device__ __forceinline__ void chunk_math(const FastArgs<DT>& a, const Tabs& ft, const float g[kChunk],
                                            const float p[kChunk], const RawIdx8& iv, const float vc[kChunk],
                                            float m_old, float m_new, float y, float rv, bool general_q,
@@ -1562,7 +1601,7 @@ __device__ __forceinline__ void chunk_math(const FastArgs<DT>& a, const Tabs& ft
     constexpr bool SR = std::is_same_v<Tabs, SrTables>;
     const float tb = 0x1.00001p-100f * fmaxf(m_new, 1.0f);
     float xs[kChunk];
-    bool bad = (y == 0.0f) || general_q;
+    bool bad = (y == 0.0f) || (!LDSQ && general_q);
 #pragma unroll
     for (int k = 0; k < kChunk; ++k) {
         const float u = momentum_value<LF>(ft.cbr[raw_idx(iv, k)], m_old, g[k], a.mc);
@@ -1581,12 +1620,17 @@ __device__ __forceinline__ void chunk_math(const FastArgs<DT>& a, const Tabs& ft
             else ix[k] = quant_global(x, a.qt);
         }
     } else if constexpr (!SR) {
+        if (LDSQ && general_q) {
 #pragma unroll
-        for (int k = 0; k < kChunk; ++k) {
-            int b = (int)__builtin_fmaf(xs[k], (float)(kBuckets / 2), (float)(kBuckets / 2));
-            b = b < 0 ? 0 : (b > kFqEntries - 1 ? kFqEntries - 1 : b);  // |x| <= 1 already (v_med3)
-            const uint2 e = ft.fq[b];
-            ix[k] = e.y + (__uint_as_float(e.x) < xs[k] ? 1u : 0u);
+            for (int k = 0; k < kChunk; ++k) ix[k] = quant_dense(xs[k], ft);
+        } else {
+#pragma unroll
+            for (int k = 0; k < kChunk; ++k) {
+                int b = (int)__builtin_fmaf(xs[k], (float)(kBuckets / 2), (float)(kBuckets / 2));
+                b = b < 0 ? 0 : (b > kFqEntries - 1 ? kFqEntries - 1 : b);  // |x| <= 1 already (v_med3)
+                const uint2 e = ft.fq[b];
+                ix[k] = e.y + (__uint_as_float(e.x) < xs[k] ? 1u : 0u);
+            }
         }
     }
     if constexpr (SR) {
@@ -2059,7 +2103,7 @@ __device__ __forceinline__ void apply_tv(const TensorWork& w, int64_t wg, const 
             }
             uint32_t ix[kChunk];
             float pn[kChunk];
-            chunk_math<DT, MODE, LF>(a, ft, gj, pj, iv[j], vc, mo[j], mn[j], y[j], MODE == 0 ? vr[j] : bs[j],
+            chunk_math<DT, MODE, LF, false>(a, ft, gj, pj, iv[j], vc, mo[j], mn[j], y[j], MODE == 0 ? vr[j] : bs[j],
                                      general_q, 0, ix, pn);
             if (ok) store_idx8(a.idx + (r + j) * C + c, ix);
 #pragma unroll
