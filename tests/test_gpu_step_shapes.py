@@ -178,6 +178,51 @@ def test_step_matches_oracle(dev, case, companion):
     _check(dev, case, [(companion, companion[1], case[2], "c")] if companion else [])
 
 
+# whole tiles: several granules, the last cut by the last row (views: column);
+# tasks of 8 row steps with a cut last task (the aligned kernel and the any-width
+# one; several rows to a step)
+LARGE = [
+    ((257, 1024), 1024, BF16, "c", {}),
+    ((1501, 2048), 2048, F16, "c", {}),
+    ((301, 2056), 2056 * 301, F32, "c", {}),
+    ((300, 1025), 1025, BF16, "o", {}),
+    ((333, 768), 24, BF16, "c", {"sr": True}),
+    ((9000, 16), 48, BF16, "c", {}),
+    ((4099, 33), 4099, BF16, "c", {}),
+    ((2100, 250), 250, F16, "o", {}),
+    ((256, 256), 256, BF16, "t", {}),
+    ((264, 1096), 1096, BF16, "t", {}),
+    ((1000, 1800), 1800, F16, "t", {}),
+]
+
+
+def _granule_bytes(specs):
+    """What the launches of these tensors take for granules as workgroups."""
+    from gefen.kernels import _native
+    lib = _native.load()
+    code = {F32: _native.DT_F32, F16: _native.DT_F16, BF16: _native.DT_BF16}
+    d = (_native.TensorDesc * len(specs))()
+    for x, (shape, period, dtype, layout) in zip(d, specs):
+        for f in ("p", "grad", "m_codebook", "m_magnitude", "v0", "v1", "workspace"):
+            setattr(x, f, 4096 + (2 if layout == "o" else 0))
+        x.rows, x.cols, x.period, x.dtype, x.factored = shape[0], shape[1], period, code[dtype], 1
+        x.ps0 = x.gs0 = 1 if layout.endswith("t") else shape[1]
+        x.ps1 = x.gs1 = shape[0] if layout.endswith("t") else 1
+    return lib.gefenx_multi_tensor_scratch_bytes_for(ctypes.addressof(d), len(specs)) - \
+        lib.gefenx_multi_tensor_scratch_bytes(len(specs))
+
+
+@pytest.mark.parametrize("case", LARGE, ids=_id)
+def test_large_launch(dev, case):
+    """Beside 67M elements (views: 1.1e9) of its own kernel: the launch takes
+    whole tiles, where alone it takes granules."""
+    spec = case[:4]
+    big = ((16384, 65536), 65536, case[2], "big-t") if case[3] == "t" else ((16384, 4096), 4096, case[2], "big")
+    assert _granule_bytes([spec]) > 0
+    assert _granule_bytes([spec, big]) == _granule_bytes([big])
+    _check(dev, case, [big])
+
+
 def _dense_codebook():
     """Many codewords within 1/2048 of each other, equal ones among them, near
     zero, at a quarter and at the end."""
@@ -189,3 +234,22 @@ def _dense_codebook():
 @pytest.mark.parametrize("case", CASES, ids=_id)
 def test_dense_codebook(dev, case):
     _check(dev, case, [], cb=_dense_codebook(), steps=3)
+
+
+@pytest.mark.parametrize("kind", ["nan", "inf", "huge"])
+@pytest.mark.parametrize("case", CASES, ids=_id)
+def test_nonfinite_grads(dev, case, kind):
+    """Magnitudes (torch's amax: NaN above inf), indices and v where grads of the
+    second step hold NaN, infinities, or values whose squares overflow, in the
+    first and the last element, beside chunk borders and in the last column; the
+    third step has the state that they left."""
+    def plant(g):
+        big = 6e4 if g.dtype == F16 else 1e20
+        a, b = {"nan": (float("nan"), float("nan")), "inf": (float("inf"), -float("inf")), "huge": (big, -big)}[kind]
+        x, c = g.clone().reshape(-1), g.shape[-1]
+        n = x.numel()
+        x[0], x[n - 1], x[n // 2 // c * c + c - 1] = a, b, b
+        x[min(n // 3 // 8 * 8 + 7, n - 1)] = a
+        x[min(n // 5 // 8 * 8, n - 1)] = b
+        return x.reshape(g.shape)
+    _check(dev, case, [], steps=3, plants={1: plant})
