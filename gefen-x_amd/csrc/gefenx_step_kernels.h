@@ -1465,30 +1465,30 @@ __device__ __forceinline__ void stage_tabs(SrTables& s, const QTable* __restrict
     }
 }
 
-// quant_stochastic, bit for bit, for four elements at a time (z: their hash
-// inputs): one LUT read, the entries of the bucket's first insertion point and
+// quant_stochastic, bit for bit, for two elements at a time (z0 + k dz: their
+// hash inputs; four took 141 VGPRs in the apply): one LUT read, the entries of the bucket's first insertion point and
 // of the next in one go (a bucket usually holds at most one codeword), the
 // probability of rounding up through the span's reciprocal with one Markstein
 // correction (exact where the offset and the quotient are at least 2^-100; a
 // smaller one divides), and the hash's top 24 bits, which need neither its last
 // xor-shift nor the low half of its last product.
-__device__ __forceinline__ void quant_sr4(const float* xs, const SrTables& s, int kk, uint64_t z0, uint64_t dz,
+__device__ __forceinline__ void quant_sr2(const float* xs, const SrTables& s, int kk, uint64_t z0, uint64_t dz,
                                           uint32_t* ix) {
-    uint32_t pk[4];
+    uint32_t pk[2];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < 2; ++k) {
         int b = (int)floorf((xs[k] + 1.0f) * (float)(kBuckets / 2));
         b = b < 0 ? 0 : (b > kBuckets - 1 ? kBuckets - 1 : b);
         pk[k] = s.lut[b];
     }
-    f32x4 e0[4], e1[4];
+    f32x4 e0[2], e1[2];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < 2; ++k) {
         e0[k] = s.e[pk[k] & 0xffffu];
         e1[k] = s.e[(pk[k] & 0xffffu) + 1u];
     }
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < 2; ++k) {
         const float x = xs[k];
         uint32_t j = pk[k] & 0xffffu;
         const uint32_t hi = pk[k] >> 16;
@@ -1635,9 +1635,11 @@ __device__ __forceinline__ void chunk_math(const FastArgs<DT>& a, const Tabs& ft
     }
     if constexpr (SR) {
         const uint64_t z0 = a.seed + kSrStep * ((uint64_t)e0 + 1ull);
-        quant_sr4(xs, ft, a.kk, z0, kSrStep, ix);
-        __builtin_amdgcn_sched_barrier(0);  // four at a time: registers
-        quant_sr4(xs + 4, ft, a.kk, z0 + 4ull * kSrStep, kSrStep, ix + 4);
+#pragma unroll
+        for (int k = 0; k < kChunk; k += 2) {
+            quant_sr2(xs + k, ft, a.kk, z0 + (uint64_t)k * kSrStep, kSrStep, ix + k);
+            __builtin_amdgcn_sched_barrier(0);  // two at a time: registers
+        }
     }
     if constexpr (MODE == 0 && DT == F32) {
         if (a.ref.on) {  // reference order; vc holds v_col
@@ -2264,14 +2266,20 @@ __global__ void __launch_bounds__(kThreads) k_mt_apply_tv(const TensorWork* __re
     apply_tv_wg<DT, MODE>(ws[sg.t], L - sg.wg_begin, ft);
 }
 
+// Waves per SIMD of the apply.  Stochastic rounding is bound by its arithmetic and
+// LDS reads: 4 waves in 128 VGPRs against 3 in 141 took the step of 4096 x 4096
+// bf16 from 97 to 85 us (factored 103 to 91, 9001 x 4111 fp16 191 to 174).
+template <bool SR, int FAST>
+constexpr int kApplyWaves = FAST == 1 || (SR && FAST == 3) ? 4 : SR ? 2 : 3;
+
 // Apply of a launch group; with MODE 0 the group's block-path tensors of the
 // same dtype and variant (not transposed views) ride in the same launch.
 template <int DT, int MODE, bool SR, int FAST>
 // Each XCD runs a contiguous range of the launch's workgroups, i.e. streams
 // its own part of each tensor (measured on the Llama-3-8B set: apply
 // 11.51-11.61 -> 11.42-11.44 ms, with a smaller spread between processes).
-__global__ void __launch_bounds__(kThreads, FAST == 1 ? 4 : SR ? 2 : 3) k_mt_apply(const TensorWork* __restrict__ ws,
-                                                       SegTable tb) {
+__global__ void __launch_bounds__(kThreads, (kApplyWaves<SR, FAST>)) k_mt_apply(const TensorWork* __restrict__ ws,
+                                                                                         SegTable tb) {
     __shared__ ApplyLds<SR, FAST> lds;
     const int64_t L = xcd_contiguous(blockIdx.x, gridDim.x);
     const Seg sg = find_seg(tb, L);
