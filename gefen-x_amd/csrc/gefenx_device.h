@@ -26,6 +26,9 @@ template <class T> __device__ __forceinline__ GX_GLOBAL T* gbl(T* p) { return (G
 template <class T> __device__ __forceinline__ const GX_GLOBAL T* gbl(const T* p) {
     return (const GX_GLOBAL T*)p;
 }
+// The same for a vector type of less than its own alignment, an attribute that a
+// template argument would lose.
+#define GX_GLOBAL_AS(V, p) ((V GX_GLOBAL*)(p))
 
 // Wave-uniform read of device memory that no kernel writes while this one
 // runs, through the scalar cache (an s_load: it waits on lgkmcnt, not on the
@@ -205,13 +208,13 @@ typedef f32x4 f32x4_a4 __attribute__((aligned(4)));
 template <int DT>
 __device__ __forceinline__ void load_raw8_any(const typename Elem<DT>::T* __restrict__ base, Raw8<DT>& r) {
     if constexpr (DT == F32) {
-        const GX_GLOBAL f32x4_a4* q = gbl(reinterpret_cast<const f32x4_a4*>(base));
+        const GX_GLOBAL f32x4_a4* q = GX_GLOBAL_AS(const f32x4_a4, base);
         const f32x4 a = __builtin_nontemporal_load(q);
         const f32x4 b = __builtin_nontemporal_load(q + 1);
         r.f[0] = a.x; r.f[1] = a.y; r.f[2] = a.z; r.f[3] = a.w;
         r.f[4] = b.x; r.f[5] = b.y; r.f[6] = b.z; r.f[7] = b.w;
     } else {
-        const u32x4 v = __builtin_nontemporal_load(gbl(reinterpret_cast<const u32x4_a2*>(base)));
+        const u32x4 v = __builtin_nontemporal_load(GX_GLOBAL_AS(const u32x4_a2, base));
         r.w[0] = v.x; r.w[1] = v.y; r.w[2] = v.z; r.w[3] = v.w;
     }
 }
@@ -219,7 +222,7 @@ __device__ __forceinline__ void load_raw8_any(const typename Elem<DT>::T* __rest
 template <int DT>
 __device__ __forceinline__ void store8_any(typename Elem<DT>::T* __restrict__ base, const float v[8]) {
     if constexpr (DT == F32) {
-        GX_GLOBAL f32x4_a4* q = gbl(reinterpret_cast<f32x4_a4*>(base));
+        GX_GLOBAL f32x4_a4* q = GX_GLOBAL_AS(f32x4_a4, base);
         const f32x4 a = {v[0], v[1], v[2], v[3]}, b = {v[4], v[5], v[6], v[7]};
         __builtin_nontemporal_store(a, q);
         __builtin_nontemporal_store(b, q + 1);
@@ -229,7 +232,7 @@ __device__ __forceinline__ void store8_any(typename Elem<DT>::T* __restrict__ ba
         for (int i = 0; i < 4; ++i)
             w[i] = (uint32_t)from_f32<DT>(v[2 * i]) | ((uint32_t)from_f32<DT>(v[2 * i + 1]) << 16);
         const u32x4 a = {w[0], w[1], w[2], w[3]};
-        __builtin_nontemporal_store(a, gbl(reinterpret_cast<u32x4_a2*>(base)));
+        __builtin_nontemporal_store(a, GX_GLOBAL_AS(u32x4_a2, base));
     }
 }
 
@@ -252,7 +255,7 @@ __device__ __forceinline__ RawIdx8 load_raw_idx8_cached(const uint8_t* __restric
 // The same at any alignment.
 typedef u32x2 u32x2_a1 __attribute__((aligned(1)));
 __device__ __forceinline__ RawIdx8 load_raw_idx8_any(const uint8_t* __restrict__ base) {
-    const u32x2 v = __builtin_nontemporal_load(gbl(reinterpret_cast<const u32x2_a1*>(base)));
+    const u32x2 v = __builtin_nontemporal_load(GX_GLOBAL_AS(const u32x2_a1, base));
     return RawIdx8{v.x, v.y};
 }
 
@@ -260,7 +263,7 @@ __device__ __forceinline__ void store_idx8_any(uint8_t* __restrict__ base, const
     u32x2 a;
     a.x = ix[0] | (ix[1] << 8) | (ix[2] << 16) | (ix[3] << 24);
     a.y = ix[4] | (ix[5] << 8) | (ix[6] << 16) | (ix[7] << 24);
-    __builtin_nontemporal_store(a, gbl(reinterpret_cast<u32x2_a1*>(base)));
+    __builtin_nontemporal_store(a, GX_GLOBAL_AS(u32x2_a1, base));
 }
 
 __device__ __forceinline__ RawIdx8 load_raw_idx8_elems(const uint8_t* __restrict__ base) {

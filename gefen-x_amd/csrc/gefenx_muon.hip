@@ -697,7 +697,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const f32x16 (&
             if (full) {
                 const u32x4 dv = {(uint32_t)hv[0] | ((uint32_t)hv[1] << 16), (uint32_t)hv[2] | ((uint32_t)hv[3] << 16),
                                   (uint32_t)hv[4] | ((uint32_t)hv[5] << 16), (uint32_t)hv[6] | ((uint32_t)hv[7] << 16)};
-                *gbl(reinterpret_cast<u32x4_a2*>(dp)) = dv;  // rows of any alignment
+                *GX_GLOBAL_AS(u32x4_a2, dp) = dv;  // rows of any alignment
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
@@ -719,7 +719,7 @@ __device__ __forceinline__ void gemm_epilogue(const GemmArgs& g, const f32x16 (&
                 if (gr + 8 <= g.M) {
                     const u32x4 tv = {(uint32_t)hv[0] | ((uint32_t)hv[1] << 16), (uint32_t)hv[2] | ((uint32_t)hv[3] << 16),
                                       (uint32_t)hv[4] | ((uint32_t)hv[5] << 16), (uint32_t)hv[6] | ((uint32_t)hv[7] << 16)};
-                    *gbl(reinterpret_cast<u32x4_a2*>(tp)) = tv;
+                    *GX_GLOBAL_AS(u32x4_a2, tp) = tv;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
@@ -1935,7 +1935,7 @@ __global__ void __launch_bounds__(kT) k_cautious_count(const uint16_t* U, const 
             u32x4 uv;
             Raw8<DT> gr;
             if (nval == kPiece) {
-                uv = __builtin_nontemporal_load(gbl(reinterpret_cast<const u32x4_a2*>(u + e0)));
+                uv = __builtin_nontemporal_load(GX_GLOBAL_AS(const u32x4_a2, u + e0));
                 load_raw8_any<DT>(g + e0, gr);
             }
             int64_t r = div_floor(e0, C, invC);

@@ -385,8 +385,8 @@ __device__ __forceinline__ void stats_factored(const TensorWork& wr, int64_t wg,
     constexpr int64_t kStep = 2 * kWaves;
     // A granule ends inside the tile before row r - wave.  Every wave comes here
     // with that row: one that left the loop before has r >= r_end, so r_end lies
-    // within the 3 rows after an r - wave below it.  A granule is a multiple of 32 rows, 8 of each wave, so the fp32
-    // sums are flushed.
+    // within the 3 rows after an r - wave below it.  A granule is a multiple of
+    // 32 rows, 8 of each wave, so the fp32 sums are flushed.
     auto granule_ends = [&](int64_t r) { return r - wave == fold_at && fold_at < r_end; };
     auto end_granule = [&]() {
         fold(fold_at - gran == r_begin, std::true_type{});
@@ -1228,7 +1228,7 @@ __device__ __forceinline__ void load_vcol(const float* __restrict__ vc, float v[
 }
 
 __device__ __forceinline__ void load_vcol_any(const float* __restrict__ vc, float v[8]) {
-    const GX_GLOBAL f32x4_a4* q = gbl(reinterpret_cast<const f32x4_a4*>(vc));
+    const GX_GLOBAL f32x4_a4* q = GX_GLOBAL_AS(const f32x4_a4, vc);
     const f32x4 v0 = q[0], v1 = q[1];
     v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
     v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
